@@ -554,14 +554,15 @@ typedef struct jv_graph jv_graph;
 /* Validates the items and uploads the instance table (synchronous). */
 int jv_batch_create(const jv_batch_item* items, int32_t count, jv_batch** out);
 int jv_batch_destroy(jv_batch* batch);
-/* Launch shape of a phase: waves per workgroup (1, 2, 4, 8) and, for the
- * gradient and O_loc phases, samples per wave (1..64); re-uploads the table.
+/* Launch shape of a phase: waves per workgroup (1, 2, 4, 8; O_loc workgroups
+ * always have four) and, for the gradient phase, samples per wave (1..64), for
+ * the O_loc phase tiles of samples per workgroup; re-uploads the table.
  * Chosen by the package's autotuner (vmc_jax_amd/batch.py). */
 int jv_batch_set_shape(jv_batch* batch, int32_t phase, int32_t waves, int32_t samples_per_wave);
 /* One phase for every instance. */
 int jv_batch_phase(jv_batch* batch, int32_t phase, void* stream);
 /* Counters cleared, then sampling, gradients (+ log psi) and O_loc for every
- * instance: 5 launches, no allocation, host synchronisation or memset. */
+ * instance: 6 launches, no allocation, host synchronisation or memset. */
 int jv_batch_step(jv_batch* batch, void* stream);
 /* jv_batch_step captured into a HIP graph on `stream` (not the default
  * stream) and instantiated; jv_graph_launch replays it (parameters, walkers

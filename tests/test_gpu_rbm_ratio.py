@@ -1,0 +1,152 @@
+"""Amplitude-ratio kernels of the RBMs (csrc/rbmq.hpp) against the FP64 oracle
+at the sizes where their tiling can go wrong: hidden units around a wavefront
+and above the eight-sample tile's limit, strings that fill less than, exactly
+and more than a pass, sample counts around a tile, operators whose strings
+leave sites unchanged, repeat each other or change more than two sites, and
+parameters outside the products' range (which take the log-cosh form).
+
+Tolerance 1e-11 relative, as for every E_loc comparison: each term is a product
+of H + 2 factors, each within a few rounding errors of exact."""
+import numpy as np
+import pytest
+import torch
+
+from oracle import nets as onets
+from oracle import operator as oop
+
+from helpers import tfim_pair, to_np, xxz_pair
+
+pytestmark = pytest.mark.gpu
+
+jv = pytest.importorskip("vmc_jax_amd")
+
+TOL = 1e-11
+
+
+def _mixed_pair(L):
+    """Strings of every kind the kernels tell apart: repeated and padded
+    flips, flips that cancel, raising / lowering pairs (no flip on half the
+    configurations), complex elements, a single diagonal string."""
+    from vmc_jax_amd import operator as dop
+    out = []
+    for o in (dop, oop):
+        H = o.BranchFreeOperator()
+        for i in range(L):
+            j = (i + 1) % L
+            H.add(o.scal_opstr(0.3, (o.Sx(i),)))
+            H.add(o.scal_opstr(0.2 + 0.1j, (o.Sy(i),)))
+            H.add(o.scal_opstr(0.7, (o.Sp(i), o.Sm(j))))
+            H.add(o.scal_opstr(0.5, (o.Sm(i), o.Sp(j))))
+            H.add(o.scal_opstr(0.4, (o.Sx(i), o.Sz(j))))
+        H.add(o.scal_opstr(0.9, (o.Sx(0), o.Sx(0))))
+        H.add(o.scal_opstr(1.1, (o.Sz(1),)))
+        out.append(H)
+    return out
+
+
+def _long_pair(L):
+    """Three- and four-site strings (the general loop)."""
+    from vmc_jax_amd import operator as dop
+    out = []
+    for o in (dop, oop):
+        H = o.BranchFreeOperator()
+        for i in range(L):
+            a, b, c = (i + 1) % L, (i + 2) % L, (i + 3) % L
+            H.add(o.scal_opstr(0.3, (o.Sx(i), o.Sx(a), o.Sx(b))))
+            H.add(o.scal_opstr(0.2, (o.Sx(i), o.Sy(a), o.Sx(b), o.Sy(c))))
+            H.add(o.scal_opstr(-0.5, (o.Sz(i), o.Sz(a))))
+        out.append(H)
+    return out
+
+
+OPS = {"tfim": lambda L: tfim_pair((L,), -1.0, -0.7), "xxz": lambda L: xxz_pair(L, 0.6), "mixed": _mixed_pair,
+       "long": _long_pair}
+
+
+def _states(cpx, L, H, bias, vbias, P):
+    if cpx:
+        net, onet = jv.nets.CpxRBM(H, bias=bias, visibleBias=vbias), onets.CpxRBM((L,), H, bias=bias, visibleBias=vbias)
+    else:
+        net, onet = jv.nets.RBM(H, bias=bias), onets.RBM((L,), H, bias=bias)
+    psi = jv.NQS(net)
+    psi(torch.zeros((1, 1, L), dtype=torch.int32))
+    psi.set_parameters(P)
+    return psi, onets.NQS(onet, P)
+
+
+def _num(cpx, L, H, bias, vbias):
+    return (2 if cpx else 1) * (L * H + (H if bias else 0) + (L if vbias else 0))
+
+
+def _rel(a, b):
+    return np.linalg.norm(a - b) / np.linalg.norm(b)
+
+
+@pytest.mark.parametrize("cpx,L,H,bias,vbias,op,n", [
+    (True, 10, 20, True, True, "tfim", 9), (True, 5, 1, False, False, "tfim", 1), (True, 8, 63, True, False, "xxz", 7),
+    (True, 7, 64, False, True, "mixed", 8), (True, 33, 65, True, False, "tfim", 5), (False, 12, 130, True, False, "xxz", 20),
+    (False, 6, 3, False, False, "mixed", 33), (True, 65, 40, True, False, "tfim", 6), (True, 70, 9, True, True, "xxz", 5),
+    (True, 6, 257, True, False, "mixed", 5), (True, 9, 12, True, True, "long", 10), (False, 9, 70, True, False, "long", 3),
+    (True, 4, 6, True, False, "mixed", 8200)])
+def test_eloc(cpx, L, H, bias, vbias, op, n):
+    rng = np.random.default_rng(L * 1000 + H)
+    P = 0.3 / np.sqrt(L) * rng.normal(size=_num(cpx, L, H, bias, vbias))
+    psi, opsi = _states(cpx, L, H, bias, vbias, P)
+    Hd, Ho = OPS[op](L)
+    s = rng.integers(0, 2, size=(n, L)).astype(np.int32)
+    sd = torch.as_tensor(s[None], device="cuda")
+    e = to_np(Hd.get_O_loc(sd, psi, psi(sd)))[0]
+    ref = Ho.get_O_loc(s, opsi, opsi(s))
+    assert _rel(e, ref) < TOL
+
+
+@pytest.mark.parametrize("big", [10.0, 60.0])
+def test_eloc_out_of_range(big):
+    """A site whose summed |Re W| (80, 480) or a unit whose |Re theta| leaves the
+    ratio form's range: the log-cosh form gives the oracle's values."""
+    L, H = 6, 8
+    rng = np.random.default_rng(3)
+    P = 0.1 * rng.normal(size=_num(True, L, H, False, False))
+    P[:H] = big * np.sign(P[:H])  # Re W of site 0
+    psi, opsi = _states(True, L, H, False, False, P)
+    Hd, Ho = _mixed_pair(L)
+    s = rng.integers(0, 2, size=(11, L)).astype(np.int32)
+    sd = torch.as_tensor(s[None], device="cuda")
+    e = to_np(Hd.get_O_loc(sd, psi, psi(sd)))[0]
+    ref = Ho.get_O_loc(s, opsi, opsi(s))
+    assert np.all(np.isfinite(ref))
+    assert np.max(np.abs(e - ref) / np.abs(ref)) < TOL
+
+
+def test_eloc_nan_parameters():
+    L, H = 6, 8
+    P = 0.1 * np.random.default_rng(4).normal(size=_num(True, L, H, True, False))
+    P[3] = np.nan
+    psi, _ = _states(True, L, H, True, False, P)
+    Hd, _ = tfim_pair((L,), -1.0, -0.7)
+    sd = torch.zeros((1, 5, L), dtype=torch.int32, device="cuda")
+    e = to_np(Hd.get_O_loc(sd, psi, torch.zeros((1, 5), dtype=torch.complex128, device="cuda")))
+    assert np.all(np.isnan(e))
+
+
+def test_eloc_streams():
+    """Calls on two streams of one thread, each with its own parameters, keep
+    their tables apart."""
+    L, H, n = 10, 20, 4000
+    rng = np.random.default_rng(5)
+    Hd, _ = tfim_pair((L,), -1.0, -0.7)
+    Hd.compile()
+    sd = torch.as_tensor(rng.integers(0, 2, size=(1, n, L)).astype(np.int32), device="cuda")
+    psis = [_states(True, L, H, True, False, 0.1 * rng.normal(size=_num(True, L, H, True, False)))[0] for _ in range(2)]
+    lps = [p(sd) for p in psis]
+    ref = [Hd.get_O_loc(sd, p, lp).clone() for p, lp in zip(psis, lps)]
+    streams = [torch.cuda.Stream() for _ in range(2)]
+    torch.cuda.synchronize()
+    out = [[], []]
+    for _ in range(4):
+        for k, st in enumerate(streams):
+            with torch.cuda.stream(st):
+                out[k].append(Hd.get_O_loc(sd, psis[k], lps[k]))
+    torch.cuda.synchronize()
+    for k in range(2):
+        assert all(torch.equal(o, ref[k]) for o in out[k])

@@ -1,8 +1,8 @@
 // Batched field sweep: many independent RBM states (different lattice sizes,
 // hidden-unit counts and operators) advanced by one launch per phase.  A
 // device-resident instance table maps every workgroup of a launch to one
-// instance; the kernels then run the same per-chain / per-sample routines as
-// the single-network kernels (rbm.hpp), so each instance's samples, O_loc and
+// instance; the kernels then run the same routines as the single-network
+// kernels (rbm.hpp, rbmq.hpp), so each instance's samples, O_loc and
 // O_k are those of jv_mc_sample / jv_eloc / jv_net_gradients on its own.
 //
 // The Philox call index of every instance lives in the table and is advanced
@@ -15,7 +15,7 @@
 #include <string>
 #include <vector>
 
-#include "rbm.hpp"
+#include "rbmq.hpp"
 
 namespace jv {
 
@@ -35,7 +35,9 @@ struct BatchInst {
   double* grad;
   int32_t layout;
   int64_t n;       // samples_per_chain * num_chains
-  int32_t wg[3];   // first workgroup of this instance in the sample / gradient / O_loc launches
+  RbmTab tab;      // ratio tables (rbmq.hpp), rebuilt before each phase that reads them
+  int32_t tile, nstr;  // O_loc: samples per tile (0: log-cosh form), strings per sample
+  int32_t wg[4];   // first workgroup of this instance in the sample / gradient / O_loc / table launches
 };
 
 }  // namespace jv
@@ -46,7 +48,8 @@ struct jv_batch {
   int32_t count = 0;
   int32_t waves[3] = {4, 4, 4};      // waves per workgroup per phase
   int32_t per_wave[3] = {1, 1, 1};   // samples per wave (gradient and O_loc phases)
-  int32_t total_wg[3] = {0, 0, 0};
+  int32_t total_wg[4] = {0, 0, 0, 0};
+  double* tabs = nullptr;            // the instances' ratio tables
   size_t lds[3] = {0, 0, 0};
 };
 
@@ -98,19 +101,34 @@ __global__ void __launch_bounds__(512) batch_grad(const BatchInst* __restrict__ 
   }
 }
 
-__global__ void __launch_bounds__(512) batch_eloc(const BatchInst* __restrict__ T, int count, int per_wave,
-                                                  size_t lds_per_wave) {
+// O_loc: a workgroup takes `per_wave` tiles of one instance.
+__global__ void __launch_bounds__(64 * RBMQ_WAVES) batch_eloc(const BatchInst* __restrict__ T, int count,
+                                                              int per_wave) {
   extern __shared__ double lds[];
   const int i = batch_find(T, count, 2, blockIdx.x);
   const BatchInst& I = T[i];
-  const int lane = threadIdx.x % WAVE, w = threadIdx.x / WAVE, nw = blockDim.x / WAVE;
-  cd* th = (cd*)(lds + (size_t)w * lds_per_wave);
-  const int64_t s0 = (int64_t)(blockIdx.x - I.wg[2]) * nw * per_wave;
-  for (int k = 0; k < per_wave; ++k) {
-    const int64_t s = s0 + (int64_t)k * nw + w;
-    if (s >= I.n) break;
-    eloc_rbm_sample(I.g, I.P, I.op, I.configs + s * I.g.L, I.logpsi + 2 * s, I.eloc + 2 * s, th, lane);
+  const int64_t per = (int64_t)max(I.tile, RBMQ_WAVES) * per_wave;
+  const int64_t s0 = (int64_t)(blockIdx.x - I.wg[2]) * per, cnt = min(per, I.n - s0);
+  const bool small = I.op.max_len <= 2 && !I.op.fermi;
+#define JV_BATCH_ELO(CPX, SMALL)                                                                             \
+  rbmq_eloc_range<CPX, SMALL>(I.g, I.P, I.op, I.tab, I.configs, s0, cnt, I.tile, I.nstr, I.logpsi, I.eloc, lds)
+  if (I.g.cpx) {
+    if (small) JV_BATCH_ELO(true, true);
+    else JV_BATCH_ELO(true, false);
+  } else {
+    if (small) JV_BATCH_ELO(false, true);
+    else JV_BATCH_ELO(false, false);
   }
+#undef JV_BATCH_ELO
+}
+
+// Ratio tables of every instance from its current parameters.
+__global__ void __launch_bounds__(256) batch_tables(const BatchInst* __restrict__ T, int count) {
+  __shared__ double red[4];
+  __shared__ int wcnt[4];
+  const int i = batch_find(T, count, 3, blockIdx.x);
+  const BatchInst& I = T[i];
+  rbm_tab_build(I.g, I.P, I.tab, &I.op, blockIdx.x - I.wg[3], red, wcnt);
 }
 
 __global__ void batch_begin(BatchInst* __restrict__ T, int count) {
@@ -137,27 +155,31 @@ static int batch_layout(jv_batch* b) {
   size_t mc_lds = 8, el_lds = 8;
   for (auto& I : b->host) {
     mc_lds = std::max(mc_lds, 8 * mc_rbm_lds_doubles(I.g));
-    el_lds = std::max(el_lds, (size_t)2 * sizeof(cd) * I.g.H);
+    const size_t q = I.g.H <= RBMQ_MAX_H ? 8 * rbmq_block_lds_doubles(I.g, I.nstr, I.n) : 0;
+    I.tile = q > 0 && q <= 160 * 1024 ? rbmq_tile(I.g, I.n) : 0;
+    el_lds = std::max(el_lds, I.tile ? q : RBMQ_WAVES * 2 * sizeof(cd) * (size_t)I.g.H);
   }
-  int tot[3] = {0, 0, 0};
+  int tot[4] = {0, 0, 0, 0};
   for (auto& I : b->host) {
     I.wg[0] = tot[0];
     tot[0] += (I.a.num_chains + b->waves[0] - 1) / b->waves[0];
     for (int ph = 1; ph < 3; ++ph) {
       I.wg[ph] = tot[ph];
-      const int64_t per = (int64_t)b->waves[ph] * b->per_wave[ph];
+      const int64_t per = (int64_t)(ph == 2 ? std::max(I.tile, RBMQ_WAVES) : b->waves[ph]) * b->per_wave[ph];
       tot[ph] += (int)((I.n + per - 1) / per);
     }
+    I.wg[3] = tot[3];
+    tot[3] += rbm_tab_blocks(I.g, I.op.num_ops);
   }
-  for (int ph = 0; ph < 3; ++ph) b->total_wg[ph] = tot[ph];
+  for (int ph = 0; ph < 4; ++ph) b->total_wg[ph] = tot[ph];
   b->lds[0] = mc_lds;
   b->lds[1] = 0;
   b->lds[2] = el_lds;
-  if (b->waves[0] * mc_lds > 160 * 1024 || b->waves[2] * el_lds > 160 * 1024)
+  if (b->waves[0] * mc_lds > 160 * 1024 || el_lds > 160 * 1024)
     return fail(JV_E_NOMEM, "jv_batch: the launch shape needs more than 160 KiB of LDS per workgroup");
   JV_HIP(hipMemcpy(b->dev, b->host.data(), sizeof(BatchInst) * b->host.size(), hipMemcpyHostToDevice));
   int rc = set_lds_limit((const void*)batch_sample, b->waves[0] * mc_lds);
-  if (!rc) rc = set_lds_limit((const void*)batch_eloc, b->waves[2] * el_lds);
+  if (!rc) rc = set_lds_limit((const void*)batch_eloc, el_lds);
   return rc;
 }
 
@@ -190,8 +212,10 @@ static int batch_launch(jv_batch* b, int ph, hipStream_t st) {
     }
     case JV_BATCH_ELOC: {
       ScopedTimer tm(cap ? nullptr : "batch_eloc", st);
-      hipLaunchKernelGGL(batch_eloc, dim3((unsigned)b->total_wg[2]), dim3(64 * nw), nw * b->lds[2], st, b->dev,
-                         b->count, b->per_wave[2], b->lds[2] / 8);
+      hipLaunchKernelGGL(batch_tables, dim3((unsigned)b->total_wg[3]), dim3(256), 0, st, b->dev, b->count);
+      JV_LAUNCH_CHECK("batch_tables");
+      hipLaunchKernelGGL(batch_eloc, dim3((unsigned)b->total_wg[2]), dim3(64 * RBMQ_WAVES), b->lds[2], st, b->dev,
+                         b->count, b->per_wave[2]);
       JV_LAUNCH_CHECK("batch_eloc");
       return JV_OK;
     }
@@ -238,14 +262,28 @@ int jv_batch_create(const jv_batch_item* items, int32_t count, jv_batch** out) {
     I.grad = it.grad;
     I.layout = it.grad_layout;
     I.n = (int64_t)a.samples_per_chain * a.num_chains;
+    I.nstr = rbmq_strings(I.op);
+  }
+  size_t tab_doubles = 0;
+  for (auto& I : b->host) tab_doubles += rbm_tab_doubles(I.g, false, true, I.op.num_ops);
+  if (hipMalloc((void**)&b->tabs, sizeof(double) * tab_doubles) != hipSuccess) {
+    delete b;
+    return fail(JV_E_NOMEM, "jv_batch_create: ratio table allocation failed");
+  }
+  double* at = b->tabs;
+  for (auto& I : b->host) {
+    I.tab = rbm_tab_at(I.g, at, false, true, I.op.num_ops);
+    at += rbm_tab_doubles(I.g, false, true, I.op.num_ops);
   }
   if (hipMalloc((void**)&b->dev, sizeof(BatchInst) * count) != hipSuccess) {
+    (void)hipFree(b->tabs);
     delete b;
     return fail(JV_E_NOMEM, "jv_batch_create: instance table allocation failed");
   }
   int rc = batch_layout(b);
   if (rc) {
     (void)hipFree(b->dev);
+    (void)hipFree(b->tabs);
     delete b;
     return rc;
   }
@@ -256,6 +294,7 @@ int jv_batch_create(const jv_batch_item* items, int32_t count, jv_batch** out) {
 int jv_batch_destroy(jv_batch* b) {
   if (!b) return JV_OK;
   if (b->dev) (void)hipFree(b->dev);
+  if (b->tabs) (void)hipFree(b->tabs);
   delete b;
   return JV_OK;
 }

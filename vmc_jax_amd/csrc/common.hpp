@@ -27,6 +27,10 @@ int hip_fail(hipError_t e, const char* what);
 
 // Per-device scratch arena (grown on demand, released by jv_shutdown).
 void* workspace(size_t bytes, int slot);
+// The same per stream (WS_STREAMS slots from slot0 on).
+constexpr int WS_STREAMS = 8;
+void* stream_workspace(size_t bytes, int slot0, hipStream_t st);
+bool stream_capturing(hipStream_t st);
 
 // Optional event timing of named kernels (jv_timer_enable / jv_timer_read).
 void* timer_begin(const char* name, hipStream_t st);

@@ -31,6 +31,9 @@ struct DeviceState {
   std::vector<size_t> size;
   rocblas_handle blas = nullptr;
   hipStream_t aux = nullptr;             // second stream for work that overlaps the caller's
+  hipStream_t ws_stream[WS_STREAMS] = {};  // owners of stream_workspace's buffers
+  uint64_t ws_used[WS_STREAMS] = {};       // time of last use (0: free)
+  uint64_t ws_clock = 0;
   hipEvent_t ev[2] = {nullptr, nullptr};
 };
 // Workspaces and solver handles are per host thread and device, so threads
@@ -53,6 +56,7 @@ void release(DeviceState& s, int d) {
     if (p) (void)hipFree(p);
   s.ptr.clear();
   s.size.clear();
+  for (auto& u : s.ws_used) u = 0;
   if (s.blas) rocblas_destroy_handle(s.blas);
   s.blas = nullptr;
   for (auto& e : s.ev)
@@ -160,6 +164,36 @@ void* workspace(size_t bytes, int slot) {
     s.size[slot] = b;
   }
   return s.ptr[slot];
+}
+
+// Scratch buffer of a stream: calls on different streams of one thread get
+// buffers of their own (slots slot0 .. slot0 + WS_STREAMS - 1), so they may
+// overlap.  Beyond WS_STREAMS streams the longest unused one's buffer passes
+// to the new stream after a device synchronisation.
+void* stream_workspace(size_t bytes, int slot0, hipStream_t st) {
+  DeviceState& s = state();
+  int k = -1, old = 0;
+  for (int i = 0; i < WS_STREAMS; ++i) {
+    if (s.ws_used[i] && s.ws_stream[i] == st) k = i;
+    if (s.ws_used[i] < s.ws_used[old]) old = i;
+  }
+  if (k < 0) {
+    k = old;
+    if (s.ws_used[k]) (void)hipDeviceSynchronize();
+    s.ws_stream[k] = st;
+  }
+  s.ws_used[k] = ++s.ws_clock;
+  return workspace(bytes, slot0 + k);
+}
+
+// The stream is being captured into a graph (or cannot be asked).
+bool stream_capturing(hipStream_t st) {
+  hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
+  if (hipStreamIsCapturing(st, &cs) != hipSuccess) {
+    (void)hipGetLastError();
+    return true;
+  }
+  return cs != hipStreamCaptureStatusNone;
 }
 
 // The calling thread's auxiliary stream on the current device (default

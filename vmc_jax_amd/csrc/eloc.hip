@@ -7,13 +7,15 @@
 
 #include "cnnwin.hpp"
 #include "ops.hpp"
-#include "rbm.hpp"
+#include "rbmq.hpp"
 
 namespace jv {
 
 bool make_rbm_geom(const jv_net* net, RbmGeom& g);
 bool make_cnn_geom(const jv_net* net, CnnGeom& g);
 int set_lds_limit(const void* fn, size_t bytes);
+int build_rbm_tables(const RbmGeom& g, const double* params, const OpDev* op, bool me, bool he, hipStream_t st,
+                     int slot0, RbmTab* out);
 
 // ------------------------------------------------------------------ s' enumeration
 // One thread per sample: merged matrix elements, compaction order (base.py:91-114).
@@ -71,6 +73,17 @@ __global__ void __launch_bounds__(256) eloc_rbm(RbmGeom g, const double* __restr
   cd* th = (cd*)lds + (size_t)w * 2 * g.H;
   for (int64_t s = (int64_t)blockIdx.x * nw + w; s < n; s += (int64_t)gridDim.x * nw)
     eloc_rbm_sample(g, P, op, cfg + s * g.L, lps + 2 * s, out + 2 * s, th, lane);
+}
+
+// The ratio form (rbmq.hpp): a workgroup per tile of samples.
+template <bool CPX, bool SMALL>
+__global__ void __launch_bounds__(64 * RBMQ_WAVES, 4) eloc_rbmq(RbmGeom g, const double* __restrict__ P, OpDev op,
+                                                                RbmTab tab, const int32_t* __restrict__ cfg,
+                                                                const double* __restrict__ lps, int64_t n, int S, int nstr,
+                                                                double* __restrict__ out) {
+  extern __shared__ double lds[];
+  const int64_t s0 = (int64_t)blockIdx.x * S;
+  rbmq_eloc_range<CPX, SMALL>(g, P, op, tab, cfg, s0, min((int64_t)S, n - s0), S, nstr, lps, out, lds);
 }
 
 // ------------------------------------------------------------------ CNN O_loc
@@ -617,11 +630,30 @@ int jv_eloc(const jv_net* net, const double* params, const jv_optable* op, const
   RbmGeom rg;
   CnnGeom cg;
   if (make_rbm_geom(net, rg)) {
+    ScopedTimer tm("eloc", st);
+    // ratio form, except where its tables cannot be built (a graph capture:
+    // the captured call keeps no pointer into scratch memory) or do not fit
+    const int nstr = rbmq_strings(d);
+    const size_t lq = 8 * rbmq_block_lds_doubles(rg, nstr, n);
+    if (rg.H <= RBMQ_MAX_H && lq <= 160 * 1024 && !stream_capturing(st)) {
+      RbmTab tab;
+      rc = build_rbm_tables(rg, params, &d, false, true, st, WS_RBMQ_ELOC, &tab);
+      if (rc) return rc;
+      const bool small = d.max_len <= 2 && !d.fermi;
+      const auto fn = rg.cpx ? (small ? eloc_rbmq<true, true> : eloc_rbmq<true, false>)
+                             : (small ? eloc_rbmq<false, true> : eloc_rbmq<false, false>);
+      rc = set_lds_limit((const void*)fn, lq);
+      if (rc) return rc;
+      const int S = rbmq_tile(rg, n);
+      hipLaunchKernelGGL(fn, dim3((unsigned)((n + S - 1) / S)), dim3(64 * RBMQ_WAVES), lq, st, rg, params, d, tab,
+                         configs, logpsi_s, n, S, nstr, out);
+      JV_LAUNCH_CHECK("eloc_rbmq");
+      return JV_OK;
+    }
     size_t lds = 4 * 2 * sizeof(cd) * (size_t)rg.H;
     rc = set_lds_limit((const void*)eloc_rbm, lds);
     if (rc) return rc;
     int64_t blocks = std::min<int64_t>((n + 3) / 4, 8192);
-    ScopedTimer tm("eloc", st);
     hipLaunchKernelGGL(eloc_rbm, dim3((unsigned)blocks), dim3(256), lds, st, rg, params, d, configs, logpsi_s,
                        n, out);
     JV_LAUNCH_CHECK("eloc_rbm");

@@ -4,7 +4,7 @@
 #include <vector>
 
 #include "cnnwin.hpp"
-#include "rbm.hpp"
+#include "rbmq.hpp"
 
 namespace jv {
 
@@ -73,6 +73,27 @@ __global__ void __launch_bounds__(256) rbm_fwd_grad(RbmGeom g, const double* __r
   for (int64_t s = (int64_t)blockIdx.x * (blockDim.x / WAVE) + threadIdx.x / WAVE; s < n; s += wstride)
     rbm_fwd_grad_sample(g, P, cfg + s * g.L, layout, grad ? grad + s * rowlen : nullptr,
                         logpsi ? logpsi + 2 * s : nullptr, lane);
+}
+
+// ------------------------------------------------------------------ RBM ratio tables
+__global__ void __launch_bounds__(256) rbm_tables(RbmGeom g, const double* __restrict__ P, OpDev op, RbmTab t) {
+  __shared__ double red[4];
+  __shared__ int wcnt[4];
+  rbm_tab_build(g, P, t, &op, blockIdx.x, red, wcnt);
+}
+
+// Tables of one parameter vector in the stream's scratch buffer (op: null for
+// the chains' tables, else the operator whose strings are listed).
+int build_rbm_tables(const RbmGeom& g, const double* params, const OpDev* op, bool me, bool he, hipStream_t st,
+                     int slot0, RbmTab* out) {
+  const int nops = op ? op->num_ops : 0;
+  double* base = (double*)stream_workspace(sizeof(double) * rbm_tab_doubles(g, me, he, nops), slot0, st);
+  if (!base) return fail(JV_E_NOMEM, "RBM ratio tables: workspace allocation failed");
+  *out = rbm_tab_at(g, base, me, he, nops);
+  hipLaunchKernelGGL(rbm_tables, dim3((unsigned)rbm_tab_blocks(g, nops)), dim3(256), 0, st, g, params,
+                     op ? *op : OpDev(), *out);
+  JV_LAUNCH_CHECK("rbm_tables");
+  return JV_OK;
 }
 
 // ------------------------------------------------------------------ CNN kernel
