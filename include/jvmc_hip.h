@@ -562,7 +562,7 @@ int jv_batch_set_shape(jv_batch* batch, int32_t phase, int32_t waves, int32_t sa
 /* One phase for every instance. */
 int jv_batch_phase(jv_batch* batch, int32_t phase, void* stream);
 /* Counters cleared, then sampling, gradients (+ log psi) and O_loc for every
- * instance: 6 launches, no allocation, host synchronisation or memset. */
+ * instance: 7 launches, no allocation, host synchronisation or memset. */
 int jv_batch_step(jv_batch* batch, void* stream);
 /* jv_batch_step captured into a HIP graph on `stream` (not the default
  * stream) and instantiated; jv_graph_launch replays it (parameters, walkers

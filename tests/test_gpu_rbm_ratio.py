@@ -150,3 +150,30 @@ def test_eloc_streams():
     torch.cuda.synchronize()
     for k in range(2):
         assert all(torch.equal(o, ref[k]) for o in out[k])
+
+
+@pytest.mark.parametrize("cpx,L,H,bias,vbias,mu,big", [
+    (True, 10, 20, True, True, 2.0, 0.0), (True, 7, 1, False, False, 1.0, 0.0), (False, 12, 65, True, False, 2.0, 0.0),
+    (True, 65, 130, True, False, 2.0, 0.0), (False, 9, 256, False, False, 0.5, 0.0), (True, 6, 257, True, False, 2.0, 0.0),
+    (True, 6, 8, False, False, 2.0, 10.0), (True, 8, 64, True, False, 0.0, 0.0)])
+def test_chains(cpx, L, H, bias, vbias, mu, big):
+    """Configurations, counters and walkers of the chains equal the oracle's
+    (sites beyond one word of spins, several units per lane, the sizes and the
+    weights that take the log-cosh form, every mu); long sweeps cross the
+    interval after which theta is recomputed."""
+    from oracle import sampler as osamp
+    rng = np.random.default_rng(L * 100 + H)
+    P = 0.3 / np.sqrt(L) * rng.normal(size=_num(cpx, L, H, bias, vbias))
+    if big:
+        P[:H] = big
+    psi, opsi = _states(cpx, L, H, bias, vbias, P)
+    kw = dict(numChains=6, numSamples=24, thermalizationSweeps=5, sweepSteps=45, mu=mu)
+    ms = jv.sampler.MCSampler(psi, (L,), 17, updateProposer=jv.sampler.propose_spin_flip, **kw)
+    mo = osamp.MCSampler(opsi, (L,), 17, **kw)
+    for _ in range(2):
+        s, lp, p = ms.sample()
+        so, lpo, po = mo.sample()
+        assert np.array_equal(to_np(s)[0], so)
+        assert _rel(to_np(lp)[0], lpo) < TOL
+    assert np.array_equal(to_np(ms.states), mo.states)
+    assert abs(float(ms.acceptance_ratio()[0]) - float(np.ravel(mo.acceptance_ratio())[0])) < 1e-15

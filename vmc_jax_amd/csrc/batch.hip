@@ -76,10 +76,11 @@ __global__ void __launch_bounds__(512) batch_sample(const BatchInst* __restrict_
   extern __shared__ double lds[];
   const int i = batch_find(T, count, 0, blockIdx.x);
   const BatchInst& I = T[i];
-  const int lane = threadIdx.x % WAVE, w = threadIdx.x / WAVE, nw = blockDim.x / WAVE;
+  const int lane = threadIdx.x % WAVE, nw = blockDim.x / WAVE;
+  const int w = __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE);
   const int chain = (blockIdx.x - I.wg[0]) * nw + w;
   if (chain >= I.a.num_chains) return;
-  const int64_t nacc = mc_rbm_chain(I.g, I.P, I.a, I.walkers, I.configs, chain, lane, lds + (size_t)w * lds_per_wave);
+  const int64_t nacc = rbmq_mc(I.g, I.P, I.a, I.tab, I.walkers, I.configs, chain, lane, lds + (size_t)w * lds_per_wave);
   if (lane == 0) {
     const int total = I.a.therm_steps + I.a.samples_per_chain * I.a.sweep_steps;
     atomicAdd((unsigned long long*)&I.counters[0], (unsigned long long)total);
@@ -196,6 +197,8 @@ static int batch_launch(jv_batch* b, int ph, hipStream_t st) {
   switch (ph) {
     case JV_BATCH_SAMPLE: {
       ScopedTimer tm(cap ? nullptr : "batch_sample", st);
+      hipLaunchKernelGGL(batch_tables, dim3((unsigned)b->total_wg[3]), dim3(256), 0, st, b->dev, b->count);
+      JV_LAUNCH_CHECK("batch_tables");
       hipLaunchKernelGGL(batch_sample, dim3((unsigned)b->total_wg[0]), dim3(64 * nw), nw * b->lds[0], st, b->dev,
                          b->count, b->lds[0] / 8);
       JV_LAUNCH_CHECK("batch_sample");
@@ -265,15 +268,15 @@ int jv_batch_create(const jv_batch_item* items, int32_t count, jv_batch** out) {
     I.nstr = rbmq_strings(I.op);
   }
   size_t tab_doubles = 0;
-  for (auto& I : b->host) tab_doubles += rbm_tab_doubles(I.g, false, true, I.op.num_ops);
+  for (auto& I : b->host) tab_doubles += rbm_tab_doubles(I.g, true, true, I.op.num_ops);
   if (hipMalloc((void**)&b->tabs, sizeof(double) * tab_doubles) != hipSuccess) {
     delete b;
     return fail(JV_E_NOMEM, "jv_batch_create: ratio table allocation failed");
   }
   double* at = b->tabs;
   for (auto& I : b->host) {
-    I.tab = rbm_tab_at(I.g, at, false, true, I.op.num_ops);
-    at += rbm_tab_doubles(I.g, false, true, I.op.num_ops);
+    I.tab = rbm_tab_at(I.g, at, true, true, I.op.num_ops);
+    at += rbm_tab_doubles(I.g, true, true, I.op.num_ops);
   }
   if (hipMalloc((void**)&b->dev, sizeof(BatchInst) * count) != hipSuccess) {
     (void)hipFree(b->tabs);

@@ -645,4 +645,178 @@ __host__ __device__ inline int rbmq_strings(const OpDev& op) {
   return n > 1 ? n : 1;
 }
 
+// ------------------------------------------------------------------ Metropolis chains
+constexpr int RBMQ_MC_MAX_H = 256, RBMQ_MC_MAX_L = 2048;
+constexpr int RBMQ_MC_REFRESH = 128;  // proposals after which an emission recomputes theta
+__host__ __device__ inline bool rbmq_mc_fits(const RbmGeom& g) {
+  return g.H <= RBMQ_MC_MAX_H && g.L <= RBMQ_MC_MAX_L;
+}
+
+// Metropolis chain `chain` of MCSampler._get_samples_mcmc / _sweep
+// (sampler.py:264-367) by one wavefront, lane = hidden unit (NH units per
+// lane, H <= 64 NH); returns the accepted proposals (every lane).  A proposal
+// is |psi(s') / psi(s)|^2 = |pre|^2 prod_h |alpha + beta g|^2 against the
+// uniform number.  One wave's issue and latency set its time (1024 chains are
+// one wave per SIMD): the sites of 64 proposals are drawn at once, so g and pre
+// are loaded four proposals ahead (502 us with one ahead), the spins sit in a register per lane
+// (bit w of lane l: site 64 w + l), and the accepted state e' = e g, alpha' =
+// 1 / (1 + e') is formed beside the wave product, before the decision.
+// e = e^{-2 theta} is updated by products (relative error only) and recomputed
+// from the weights at emissions at least RBMQ_MC_REFRESH proposals apart.
+// 1024 chains x 1312 proposals, 32 sites x 64 units: 2080 us with a complex
+// log-cosh per unit and proposal, 440 us here (0.34 us per proposal).
+template <bool CPX, int NH>
+__device__ inline int64_t rbmq_mc_chain(const RbmGeom& g, const double* __restrict__ P, const jv_mc_args& a,
+                                        const RbmTab& tab, int32_t* __restrict__ walkers,
+                                        int32_t* __restrict__ configs, int chain, int lane) {
+  typedef typename num_of<CPX>::type T;
+  const int L = g.L, H = g.H, words = (L + WAVE - 1) / WAVE;
+  const double* Wr = P + g.ow;
+  const double* Wi = Wr + (int64_t)L * H;
+  const T* me = (const T*)tab.me;
+  uint32_t sp = 0;
+  for (int w = 0; w < words; ++w) {
+    const int i = w * WAVE + lane;
+    if (i < L && walkers[(int64_t)chain * L + i] > 0) sp |= 1u << w;
+  }
+  T e[NH], al[NH], be[NH];
+  auto refresh = [&]() {
+    cd th[NH];
+#pragma unroll
+    for (int c = 0; c < NH; ++c) {
+      const int hc = min(c * WAVE + lane, H - 1);
+      th[c] = {0.0, 0.0};
+      if (g.ob >= 0) {
+        th[c].re = P[g.ob + hc];
+        if (CPX) th[c].im = P[g.ob + H + hc];
+      }
+    }
+    for (int w = 0; w < words; ++w) {
+      const uint64_t up = __ballot((sp >> w) & 1);
+      const int ni = min(WAVE, L - w * WAVE);
+#pragma unroll 8
+      for (int i = 0; i < ni; ++i) {
+        const double sg = (up >> i) & 1 ? 1.0 : -1.0;
+#pragma unroll
+        for (int c = 0; c < NH; ++c) {
+          const int64_t wi = (int64_t)(w * WAVE + i) * H + min(c * WAVE + lane, H - 1);
+          th[c].re = fma(sg, Wr[wi], th[c].re);
+          if (CPX) th[c].im = fma(sg, Wi[wi], th[c].im);
+        }
+      }
+    }
+#pragma unroll
+    for (int c = 0; c < NH; ++c) {
+      const bool in = c * WAVE + lane < H;
+      if constexpr (CPX) e[c] = in ? cexp({-2.0 * th[c].re, -2.0 * th[c].im}) : cd{0.0, 0.0};
+      else e[c] = in ? exp(-2.0 * th[c].re) : 0.0;
+      al[c] = recip(plus1(e[c]));
+      be[c] = mulc(e[c], al[c]);
+    }
+  };
+  refresh();
+  const int total = a.therm_steps + a.samples_per_chain * a.sweep_steps;
+  int dsite = 0;
+  double du = 0.0;
+  auto batch = [&](int base) {
+    if (base + lane < total)
+      mc_draw(a.seed, (uint32_t)(base + lane), (uint32_t)chain, a.call_index, a.stream, L, dsite, du);
+  };
+  // g and |pre|^2 of the next AHEAD proposals, for either spin
+  constexpr int AHEAD = NH == 1 ? 4 : 2;
+  T q0[AHEAD][NH], q1[AHEAD][NH];
+  double p0[AHEAD], p1[AHEAD];
+  int sites[AHEAD];
+  double us[AHEAD];
+  auto fetch = [&](int d, int step) {
+    if (step < total && (step & 63) == 0) batch(step);
+    const int site = __builtin_amdgcn_readlane(dsite, step & 63);
+    sites[d] = site;
+    us[d] = __hiloint2double(__builtin_amdgcn_readlane(__double2hiint(du), step & 63),
+                             __builtin_amdgcn_readlane(__double2loint(du), step & 63));
+#pragma unroll
+    for (int c = 0; c < NH; ++c) {
+      const int64_t at = (int64_t)site * 2 * H + min(c * WAVE + lane, H - 1);
+      q0[d][c] = me[at];
+      q1[d][c] = me[at + H];
+    }
+    p0[d] = tab.site[8 * (int64_t)site];
+    p1[d] = tab.site[8 * (int64_t)site + 1];
+  };
+#pragma unroll
+  for (int d = 0; d < AHEAD; ++d) fetch(d, d);
+  int64_t nacc = 0;
+  int since = 0, left = a.therm_steps + a.sweep_steps;
+  int64_t row = chain;
+  for (int step0 = 0; step0 < total; step0 += AHEAD) {
+#pragma unroll
+    for (int d = 0; d < AHEAD; ++d) {
+      const int step = step0 + d;
+      if (step >= total) break;
+      const double u = us[d];
+      const int wd = sites[d] >> 6, ln = sites[d] & 63;
+      const bool up = (__builtin_amdgcn_readlane((int)sp, ln) >> wd) & 1;
+      T gq[NH];
+#pragma unroll
+      for (int c = 0; c < NH; ++c) gq[c] = sel(up, q1[d][c], q0[d][c]);
+      const double pre = up ? p1[d] : p0[d];
+      fetch(d, step + AHEAD);
+      double p = 1.0;
+      T en[NH], an[NH], bn[NH];
+#pragma unroll
+      for (int c = 0; c < NH; ++c) {
+        p *= norm2(fmac(be[c], gq[c], al[c]));
+        en[c] = mulc(e[c], gq[c]);
+        an[c] = recip(plus1(en[c]));
+        bn[c] = mulc(en[c], an[c]);
+      }
+      const double ratio = pre * wave_prod(p);
+      // random.bernoulli(key, P), sampler.py:336-340
+      const bool acc = a.mu == 2.0 ? u < ratio : u < exp(a.mu * (0.5 * log(ratio)));
+      if (acc) {
+#pragma unroll
+        for (int c = 0; c < NH; ++c) {
+          e[c] = en[c];
+          al[c] = an[c];
+          be[c] = bn[c];
+        }
+        if (lane == ln) sp ^= 1u << wd;
+        ++nacc;
+      }
+      ++since;
+      if (--left == 0) {
+        left = a.sweep_steps;
+        int32_t* out = configs + row * L;
+        row += a.num_chains;
+        for (int w = 0; w < words; ++w)
+          if (w * WAVE + lane < L) out[w * WAVE + lane] = (sp >> w) & 1;
+        if (since >= RBMQ_MC_REFRESH) {
+          refresh();
+          since = 0;
+        }
+      }
+    }
+  }
+  for (int w = 0; w < words; ++w)
+    if (w * WAVE + lane < L) walkers[(int64_t)chain * L + w * WAVE + lane] = (sp >> w) & 1;
+  return nacc;
+}
+
+// The chain in the form the parameters' range and the sizes allow
+// (lds: mc_rbm_lds_doubles(g), used by the log-cosh form).
+__device__ inline int64_t rbmq_mc(const RbmGeom& g, const double* __restrict__ P, const jv_mc_args& a,
+                                  const RbmTab& tab, int32_t* __restrict__ walkers, int32_t* __restrict__ configs,
+                                  int chain, int lane, double* lds) {
+  if (rbmq_mc_fits(g) && rbmq_ok(g, tab, 2, lane)) {  // squared moduli: twice the exponent of one flip
+#define JV_RBMQ_MC(NHv)                                                                         \
+  return g.cpx ? rbmq_mc_chain<true, NHv>(g, P, a, tab, walkers, configs, chain, lane)          \
+               : rbmq_mc_chain<false, NHv>(g, P, a, tab, walkers, configs, chain, lane)
+    if (g.H <= 64) JV_RBMQ_MC(1);
+    if (g.H <= 128) JV_RBMQ_MC(2);
+    JV_RBMQ_MC(4);
+#undef JV_RBMQ_MC
+  }
+  return mc_rbm_chain(g, P, a, walkers, configs, chain, lane, lds);
+}
+
 }  // namespace jv

@@ -3,13 +3,15 @@
 #include <algorithm>
 
 #include "cnnwin.hpp"
-#include "rbm.hpp"
+#include "rbmq.hpp"
 
 namespace jv {
 
 bool make_rbm_geom(const jv_net* net, RbmGeom& g);
 bool make_cnn_geom(const jv_net* net, CnnGeom& g);
 int set_lds_limit(const void* fn, size_t bytes);
+int build_rbm_tables(const RbmGeom& g, const double* params, const OpDev* op, bool me, bool he, hipStream_t st,
+                     int slot0, RbmTab* out);
 
 __global__ void zero_i64(int64_t* p, int n) {
   int i = blockIdx.x * blockDim.x + threadIdx.x;
@@ -26,6 +28,23 @@ __global__ void __launch_bounds__(256) mc_rbm(RbmGeom g, const double* __restric
   const int chain = blockIdx.x * nw + w;
   if (chain >= a.num_chains) return;
   const int64_t nacc = mc_rbm_chain(g, P, a, walkers, configs, chain, lane, lds + (size_t)w * mc_rbm_lds_doubles(g));
+  if (lane == 0) {
+    const int total = a.therm_steps + a.samples_per_chain * a.sweep_steps;
+    atomicAdd((unsigned long long*)&counters[0], (unsigned long long)total);
+    atomicAdd((unsigned long long*)&counters[1], (unsigned long long)nacc);
+  }
+}
+
+// The same with ratio tables (rbmq_mc in rbmq.hpp).
+__global__ void __launch_bounds__(256, 1) mc_rbmq(RbmGeom g, const double* __restrict__ P, jv_mc_args a, RbmTab tab,
+                                                  int32_t* __restrict__ walkers, int32_t* __restrict__ configs,
+                                                  int64_t* __restrict__ counters) {
+  extern __shared__ double lds[];
+  const int lane = threadIdx.x % WAVE, nw = blockDim.x / WAVE;
+  const int w = __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE);
+  const int chain = blockIdx.x * nw + w;
+  if (chain >= a.num_chains) return;
+  const int64_t nacc = rbmq_mc(g, P, a, tab, walkers, configs, chain, lane, lds + (size_t)w * mc_rbm_lds_doubles(g));
   if (lane == 0) {
     const int total = a.therm_steps + a.samples_per_chain * a.sweep_steps;
     atomicAdd((unsigned long long*)&counters[0], (unsigned long long)total);
@@ -621,14 +640,26 @@ int jv_mc_sample(const jv_net* net, const double* params, const jv_mc_args* args
   CnnGeom cg;
   bool fused_lp = false;  // log psi of the emitted samples written by the sampling kernel
   if (make_rbm_geom(net, rg)) {
-    const int nw = 4;
-    size_t lds = nw * 8 * mc_rbm_lds_doubles(rg);
-    int rc = set_lds_limit((const void*)mc_rbm, lds);
-    if (rc) return rc;
     ScopedTimer tm("mc_sweep", st);
+    // ratio form, except in a graph capture (the captured call keeps no
+    // pointer into scratch memory); up to 256 chains get a CU each
+    const bool q = rbmq_mc_fits(rg) && !stream_capturing(st);
+    const int nw = q && a.num_chains <= 256 ? 1 : 4;
+    size_t lds = nw * 8 * mc_rbm_lds_doubles(rg);
+    int rc = set_lds_limit(q ? (const void*)mc_rbmq : (const void*)mc_rbm, lds);
+    if (rc) return rc;
+    if (q) {
+      RbmTab tab;
+      rc = build_rbm_tables(rg, params, nullptr, true, false, st, WS_RBMQ_MC, &tab);
+      if (rc) return rc;
+      hipLaunchKernelGGL(mc_rbmq, dim3((unsigned)((a.num_chains + nw - 1) / nw)), dim3(64 * nw), lds, st, rg, params,
+                         a, tab, walkers, configs, counters);
+      JV_LAUNCH_CHECK("mc_rbmq");
+    } else {
     hipLaunchKernelGGL(mc_rbm, dim3((unsigned)((a.num_chains + nw - 1) / nw)), dim3(64 * nw), lds, st, rg,
                        params, a, walkers, configs, counters);
     JV_LAUNCH_CHECK("mc_rbm");
+    }
   } else if (make_cnn_geom(net, cg) && win_ok(cg) && cnn_cmax(cg) > 0 && mc_win_cs(cg) > 0 &&
              mc_win_bytes(cg, cnn_cmax(cg), mc_win_cs(cg), net->precision == JV_PREC_MIXED ? 4 : 8) <= 160 * 1024) {
     const bool mixed = net->precision == JV_PREC_MIXED;
