@@ -13,6 +13,7 @@ import torch
 
 from oracle import nets as onets
 from oracle import operator as oop
+from oracle import sampler as osamp
 
 from helpers import tfim_pair, to_np, xxz_pair
 
@@ -161,7 +162,6 @@ def test_chains(cpx, L, H, bias, vbias, mu, big):
     (sites beyond one word of spins, several units per lane, the sizes and the
     weights that take the log-cosh form, every mu); long sweeps cross the
     interval after which theta is recomputed."""
-    from oracle import sampler as osamp
     rng = np.random.default_rng(L * 100 + H)
     P = 0.3 / np.sqrt(L) * rng.normal(size=_num(cpx, L, H, bias, vbias))
     if big:

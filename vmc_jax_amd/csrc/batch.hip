@@ -111,8 +111,15 @@ __global__ void __launch_bounds__(64 * RBMQ_WAVES) batch_eloc(const BatchInst* _
   const int64_t per = (int64_t)max(I.tile, RBMQ_WAVES) * per_wave;
   const int64_t s0 = (int64_t)(blockIdx.x - I.wg[2]) * per, cnt = min(per, I.n - s0);
   const bool small = I.op.max_len <= 2 && !I.op.fermi;
-#define JV_BATCH_ELO(CPX, SMALL)                                                                             \
-  rbmq_eloc_range<CPX, SMALL>(I.g, I.P, I.op, I.tab, I.configs, s0, cnt, I.tile, I.nstr, I.logpsi, I.eloc, lds)
+#define JV_BATCH_ELO_S(CPX, SMALL, S)                                                                            \
+  rbmq_eloc_range<CPX, SMALL, S>(I.g, I.P, I.op, I.tab, I.configs, s0, cnt, I.nstr, I.logpsi, I.eloc, lds)
+#define JV_BATCH_ELO(CPX, SMALL)                 \
+  do {                                           \
+    if (I.tile == 8) JV_BATCH_ELO_S(CPX, SMALL, 8); \
+    else if (I.tile == 4) JV_BATCH_ELO_S(CPX, SMALL, 4); \
+    else if (I.tile == 2) JV_BATCH_ELO_S(CPX, SMALL, 2); \
+    else JV_BATCH_ELO_S(CPX, SMALL, 0);          \
+  } while (0)
   if (I.g.cpx) {
     if (small) JV_BATCH_ELO(true, true);
     else JV_BATCH_ELO(true, false);
@@ -120,6 +127,7 @@ __global__ void __launch_bounds__(64 * RBMQ_WAVES) batch_eloc(const BatchInst* _
     if (small) JV_BATCH_ELO(false, true);
     else JV_BATCH_ELO(false, false);
   }
+#undef JV_BATCH_ELO_S
 #undef JV_BATCH_ELO
 }
 

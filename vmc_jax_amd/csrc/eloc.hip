@@ -76,14 +76,14 @@ __global__ void __launch_bounds__(256) eloc_rbm(RbmGeom g, const double* __restr
 }
 
 // The ratio form (rbmq.hpp): a workgroup per tile of samples.
-template <bool CPX, bool SMALL>
+template <bool CPX, bool SMALL, int S>
 __global__ void __launch_bounds__(64 * RBMQ_WAVES, 4) eloc_rbmq(RbmGeom g, const double* __restrict__ P, OpDev op,
                                                                 RbmTab tab, const int32_t* __restrict__ cfg,
-                                                                const double* __restrict__ lps, int64_t n, int S, int nstr,
+                                                                const double* __restrict__ lps, int64_t n, int nstr,
                                                                 double* __restrict__ out) {
   extern __shared__ double lds[];
   const int64_t s0 = (int64_t)blockIdx.x * S;
-  rbmq_eloc_range<CPX, SMALL>(g, P, op, tab, cfg, s0, min((int64_t)S, n - s0), S, nstr, lps, out, lds);
+  rbmq_eloc_range<CPX, SMALL, S>(g, P, op, tab, cfg, s0, min((int64_t)S, n - s0), nstr, lps, out, lds);
 }
 
 // ------------------------------------------------------------------ CNN O_loc
@@ -640,13 +640,16 @@ int jv_eloc(const jv_net* net, const double* params, const jv_optable* op, const
       rc = build_rbm_tables(rg, params, &d, false, true, st, WS_RBMQ_ELOC, &tab);
       if (rc) return rc;
       const bool small = d.max_len <= 2 && !d.fermi;
-      const auto fn = rg.cpx ? (small ? eloc_rbmq<true, true> : eloc_rbmq<true, false>)
-                             : (small ? eloc_rbmq<false, true> : eloc_rbmq<false, false>);
+      const int S = rbmq_tile(rg, n);
+#define JV_RBMQ_FN(Sv)                                                                     \
+  (rg.cpx ? (small ? eloc_rbmq<true, true, Sv> : eloc_rbmq<true, false, Sv>)               \
+          : (small ? eloc_rbmq<false, true, Sv> : eloc_rbmq<false, false, Sv>))
+      const auto fn = S == 8 ? JV_RBMQ_FN(8) : S == 4 ? JV_RBMQ_FN(4) : JV_RBMQ_FN(2);
+#undef JV_RBMQ_FN
       rc = set_lds_limit((const void*)fn, lq);
       if (rc) return rc;
-      const int S = rbmq_tile(rg, n);
       hipLaunchKernelGGL(fn, dim3((unsigned)((n + S - 1) / S)), dim3(64 * RBMQ_WAVES), lq, st, rg, params, d, tab,
-                         configs, logpsi_s, n, S, nstr, out);
+                         configs, logpsi_s, n, nstr, out);
       JV_LAUNCH_CHECK("eloc_rbmq");
       return JV_OK;
     }

@@ -614,26 +614,24 @@ __device__ inline void rbmq_eloc_tile(const RbmGeom& g, const double* __restrict
   }
 }
 
-// Samples [s0, s0 + cnt) by one workgroup of RBMQ_WAVES waves: the ratio form
-// where the parameters' range allows it, rbm.hpp's log-cosh form otherwise
-// (S = 0: always).
-template <bool CPX, bool SMALL>
+// Samples [s0, s0 + cnt) by one workgroup of RBMQ_WAVES waves, S at a time:
+// the ratio form where the parameters' range allows it, rbm.hpp's log-cosh
+// form otherwise (S = 0: always).
+template <bool CPX, bool SMALL, int S>
 __device__ inline void rbmq_eloc_range(const RbmGeom& g, const double* __restrict__ P, const OpDev& op,
                                        const RbmTab& tab, const int32_t* __restrict__ cfg, int64_t s0, int64_t cnt,
-                                       int S, int nstr, const double* __restrict__ lps, double* __restrict__ out,
+                                       int nstr, const double* __restrict__ lps, double* __restrict__ out,
                                        double* lds) {
   const int lane = threadIdx.x % WAVE, w = __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE);
-  if (S > 0 && rbmq_ok(g, tab, max(2, op.max_len), lane)) {
-    for (int64_t k = 0; k < cnt; k += S) {
-      const int ns = (int)min((int64_t)S, cnt - k);
-      const int64_t s = s0 + k;
-#define JV_RBMQ_TILE(Sv)                                                                                        \
-  if (S == Sv)                                                                                                  \
-    rbmq_eloc_tile<CPX, SMALL, Sv>(g, P, op, tab, cfg + s * g.L, ns, nstr, lps + 2 * s, out + 2 * s, lds, lane, w);
-      JV_RBMQ_TILE(8) JV_RBMQ_TILE(4) JV_RBMQ_TILE(2)
-#undef JV_RBMQ_TILE
+  if constexpr (S > 0) {
+    if (rbmq_ok(g, tab, max(2, op.max_len), lane)) {
+      for (int64_t k = 0; k < cnt; k += S) {
+        const int64_t s = s0 + k;
+        rbmq_eloc_tile<CPX, SMALL, S>(g, P, op, tab, cfg + s * g.L, (int)min((int64_t)S, cnt - k), nstr, lps + 2 * s,
+                                      out + 2 * s, lds, lane, w);
+      }
+      return;
     }
-    return;
   }
   for (int64_t k = w; k < cnt; k += RBMQ_WAVES)
     eloc_rbm_sample(g, P, op, cfg + (s0 + k) * g.L, lps + 2 * (s0 + k), out + 2 * (s0 + k),

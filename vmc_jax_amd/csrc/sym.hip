@@ -17,7 +17,19 @@
 
 namespace jv {
 
+int check_op(const jv_optable* op, const double* pref);
+// Resident forms for RBMs under avgFun_Coefficients_Exp (symrbm.hip).
+int sym_rbm_forward_launch(const jv_net* net, const double* params, const jv_orbit* orbit, const int32_t* configs,
+                           int64_t n, double* logpsi, hipStream_t st, int slot0, bool* done);
+int sym_rbm_eloc_launch(const jv_net* net, const double* params, const jv_orbit* orbit, const jv_optable* op,
+                        const double* prefactor, const int32_t* configs, const double* lps, int64_t n, double* out,
+                        hipStream_t st, int slot0, bool* done);
+int sym_rbm_mc_launch(const jv_net* net, const double* params, const jv_orbit* orbit, const jv_mc_args& a,
+                      int32_t* walkers, int32_t* configs, int64_t* counters, hipStream_t st, int slot0, bool* done);
+
 namespace {
+// first slots of the resident forms' tables in stream_workspace
+constexpr int WS_SYM_FWD_TAB = 150, WS_SYM_ELOC_TAB = 160, WS_SYM_MC_TAB = 170;
 // workspace slots of this file.  jv_sym_eloc may run on a side stream while
 // jv_sym_gradients runs on the main stream, so the forward pass inside
 // jv_sym_eloc has rows / log-psi slots of its own (WS_EROWS, WS_ELP).
@@ -299,6 +311,9 @@ int sym_forward(const jv_net* net, const double* params, const jv_orbit* orbit, 
   if (!params || !configs || !logpsi || n < 0) return fail(JV_E_ARG, "jv_sym_forward: bad arguments");
   if (n == 0) return JV_OK;
   hipStream_t st = (hipStream_t)stream;
+  bool done = false;
+  rc = sym_rbm_forward_launch(net, params, orbit, configs, n, logpsi, st, WS_SYM_FWD_TAB, &done);
+  if (rc || done) return rc;
   const int L = net->num_sites, G = orbit->num_elements;
   const int64_t cs = std::min<int64_t>(n, rows_per_chunk(net, orbit, 0));
   int32_t* rows = (int32_t*)workspace(sizeof(int32_t) * (size_t)cs * G * L, ws_rows);
@@ -380,6 +395,11 @@ int jv_sym_eloc(const jv_net* net, const double* params, const jv_orbit* orbit, 
   if (n == 0) return JV_OK;
   if (op->num_ops < 1) return fail(JV_E_ARG, "jv_sym_eloc: empty operator");
   hipStream_t st = (hipStream_t)stream;
+  if ((rc = check_op(op, prefactor))) return rc;
+  ScopedTimer tm("sym_eloc", st);
+  bool done = false;
+  rc = sym_rbm_eloc_launch(net, params, orbit, op, prefactor, configs, logpsi_s, n, out, st, WS_SYM_ELOC_TAB, &done);
+  if (rc || done) return rc;
   const int L = net->num_sites, nops = op->num_ops;
   // s' of cs samples are cs * nops configurations, each expanded |orbit| times by jv_sym_forward
   const int64_t cs = std::max<int64_t>(1, std::min<int64_t>(n, rows_per_chunk(net, orbit, 0) * 4 / nops));
@@ -388,7 +408,6 @@ int jv_sym_eloc(const jv_net* net, const double* params, const jv_orbit* orbit, 
   int32_t* cnt = (int32_t*)workspace(sizeof(int32_t) * (size_t)cs, WS_CNT);
   double* lpsp = (double*)workspace(sizeof(double) * 2 * (size_t)cs * nops, WS_LPSP);
   if (!sp || !me || !cnt || !lpsp) return fail(JV_E_NOMEM, "jv_sym_eloc: workspace allocation failed");
-  ScopedTimer tm("sym_eloc", st);
   for (int64_t s0 = 0; s0 < n; s0 += cs) {
     const int64_t ns = std::min(cs, n - s0);
     if ((rc = jv_get_s_primes(op, prefactor, configs + s0 * L, ns, L, sp, me, cnt, stream))) return rc;
@@ -412,18 +431,23 @@ int jv_sym_mc_sample(const jv_net* net, const double* params, const jv_orbit* or
   if (a.mu < 0.0 || a.mu > 2.0) return fail(JV_E_ARG, "mu must be in the range [0, 2]");
   hipStream_t st = (hipStream_t)stream;
   const int C = a.num_chains, L = net->num_sites;
+  const int64_t ns = (int64_t)a.samples_per_chain * C;
+  const int64_t total = (int64_t)a.therm_steps + (int64_t)a.samples_per_chain * a.sweep_steps;
+  if (total > INT32_MAX) return fail(JV_E_ARG, "jv_sym_mc_sample: too many steps");
+  ScopedTimer tm("sym_mc", st);
+  bool done = false;
+  rc = sym_rbm_mc_launch(net, params, orbit, a, walkers, configs, counters, st, WS_SYM_MC_TAB, &done);
+  if (rc) return rc;
+  if (done) return logpsi && ns > 0 ? jv_sym_forward(net, params, orbit, configs, ns, logpsi, stream) : JV_OK;
   double* lacc = (double*)workspace(sizeof(double) * (size_t)C, WS_MC_LP);
   int32_t* prop = (int32_t*)workspace(sizeof(int32_t) * (size_t)C * L, WS_MC_PROP);
   double* u = (double*)workspace(sizeof(double) * (size_t)C, WS_MC_U);
   int64_t* nacc = (int64_t*)workspace(sizeof(int64_t) * (size_t)C, WS_MC_NACC);
   double* lpp = (double*)workspace(sizeof(double) * 2 * (size_t)C, WS_MC_LPP);
   if (!lacc || !prop || !u || !nacc || !lpp) return fail(JV_E_NOMEM, "jv_sym_mc_sample: workspace allocation failed");
-  ScopedTimer tm("sym_mc", st);
   if ((rc = jv_sym_forward(net, params, orbit, walkers, C, lpp, stream))) return rc;
   hipLaunchKernelGGL(sym_mc_init, dim3((unsigned)((C + 255) / 256)), dim3(256), 0, st, lpp, C, a.mu, lacc, nacc);
   JV_LAUNCH_CHECK("sym_mc_init");
-  const int64_t total = (int64_t)a.therm_steps + (int64_t)a.samples_per_chain * a.sweep_steps;
-  if (total > INT32_MAX) return fail(JV_E_ARG, "jv_sym_mc_sample: too many steps");
   const unsigned pblocks = (unsigned)(((int64_t)C * L + 255) / 256);
   for (int step = 0; step < (int)total; ++step) {
     hipLaunchKernelGGL(sym_mc_propose, dim3(pblocks), dim3(256), 0, st, walkers, C, L, a, step, prop, u);
@@ -435,7 +459,6 @@ int jv_sym_mc_sample(const jv_net* net, const double* params, const jv_orbit* or
   }
   hipLaunchKernelGGL(sym_mc_count, dim3(1), dim3(64), 0, st, nacc, C, total * C, counters);
   JV_LAUNCH_CHECK("sym_mc_count");
-  const int64_t ns = (int64_t)a.samples_per_chain * C;
   if (logpsi && ns > 0) return jv_sym_forward(net, params, orbit, configs, ns, logpsi, stream);
   return JV_OK;
 }

@@ -1,0 +1,746 @@
+// Symmetrised RBMs (avgFun_Coefficients_Exp over an RBM, sym_wrapper.py:7-9,
+// 66-77) with the orbit resident in one workgroup: log psi, local energies and
+// Metropolis chains without materialising the |G| transformed configurations,
+// their s' or a launch per proposal.
+//
+// psi(s) = sum_g b_g psi_net(g s).  Flipping site i flips one site of every row
+// g s, so psi(s') / psi(s) = sum_g w_g r_g with w_g = b_g psi_net(g s) / psi(s)
+// and r_g the RBM ratio of rbmq.hpp: eight FP64 operations per row, hidden
+// unit and flip.  Parameters outside the ratio form's range are evaluated row
+// by row with rbm.hpp's log-cosh (slow_* below).
+#include <algorithm>
+#include <cmath>
+#include <string>
+
+#include "rbmq.hpp"
+
+namespace jv {
+
+int set_lds_limit(const void* fn, size_t bytes);
+int build_rbm_tables(const RbmGeom& g, const double* params, const OpDev* op, bool me, bool he, hipStream_t st,
+                     int slot0, RbmTab* out);
+bool make_rbm_geom(const jv_net* net, RbmGeom& g);
+OpDev make_opdev(const jv_optable* op, const double* pref, int L);
+
+namespace {
+
+struct SymGeom {
+  int G, cpx;          // orbit elements; complex coefficients or factors
+  const int32_t* map;  // [G][L]: j for s_j, -1 - j for 1 - s_j
+  const double* fac;   // [G] complex
+};
+
+constexpr int SYM_MAX_G = 2048;  // per-row sums of one configuration stay in LDS
+constexpr int SYM_T = 256;       // threads of the forward and local-energy workgroups
+
+// Row r of the orbit at site i of configuration s.
+__device__ inline int row_spin(const SymGeom& o, int L, const int32_t* s, int r, int i) {
+  const int m = o.map[(int64_t)r * L + i];
+  return m >= 0 ? (s[m] > 0) : !(s[-1 - m] > 0);
+}
+
+// theta of hidden units h .. h + 3 (clamped to H - 1) for one row's spins.
+template <bool CPX>
+__device__ inline void theta4(const RbmGeom& g, const double* __restrict__ P, const unsigned char* row, int h,
+                              cd* th) {
+  const double* Wr = P + g.ow;
+  const double* Wi = Wr + (int64_t)g.L * g.H;
+  int hc[4];
+#pragma unroll
+  for (int k = 0; k < 4; ++k) {
+    hc[k] = min(h + k, g.H - 1);
+    th[k] = {g.ob >= 0 ? P[g.ob + hc[k]] : 0.0, CPX && g.ob >= 0 ? P[g.ob + g.H + hc[k]] : 0.0};
+  }
+#pragma unroll 4
+  for (int i = 0; i < g.L; ++i) {
+    const double sg = row[i] ? 1.0 : -1.0;
+    const int64_t w = (int64_t)i * g.H;
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+      th[k].re = fma(sg, Wr[w + hc[k]], th[k].re);
+      if (CPX) th[k].im = fma(sg, Wi[w + hc[k]], th[k].im);
+    }
+  }
+}
+template <bool CPX>
+__device__ inline void ab_of(cd th, typename num_of<CPX>::type& al, typename num_of<CPX>::type& be, cd& lin,
+                             typename num_of<CPX>::type& d) {
+  if constexpr (CPX) {
+    rbm_ab(th, al, be, lin, d);
+  } else {
+    double l;
+    rbm_ab(th.re, al, be, l, d);
+    lin = {l, 0.0};
+  }
+}
+// Visible part of log psi of one row, the sites split over `sl` of SL lanes.
+__device__ inline cd visible(const RbmGeom& g, const double* __restrict__ P, const unsigned char* row, int sl, int SL) {
+  cd v = {0.0, 0.0};
+  if (g.oa >= 0)
+    for (int i = sl; i < g.L; i += SL) {
+      const double sg = row[i] ? 1.0 : -1.0;
+      v.re = fma(sg, P[g.oa + i], v.re);
+      v.im = fma(sg, P[g.oa + g.L + i], v.im);
+    }
+  return v;
+}
+
+__device__ inline cd block_sum_cd(cd v, double* red) { return {block_sum(v.re, red), block_sum(v.im, red)}; }
+__device__ inline double block_max(double v, double* red) {
+  for (int o = WAVE / 2; o > 0; o >>= 1) v = fmax(v, __shfl_xor(v, o));
+  __syncthreads();
+  if (threadIdx.x % WAVE == 0) red[threadIdx.x / WAVE] = v;
+  __syncthreads();
+  double m = red[0];
+  for (int i = 1; i < (int)blockDim.x / WAVE; ++i) m = fmax(m, red[i]);
+  __syncthreads();
+  return m;
+}
+// log of sum_g b_g e^{x_g} d_g from its shifted sum (jax's logsumexp: a
+// negative sum of real terms is NaN).
+__device__ inline cd log_of_sum(cd S, double shift, int cpx) {
+  if (cpx) return {log(hypot(S.re, S.im)) + shift, atan2(S.im, S.re)};
+  return {S.re < 0.0 ? NAN : log(fabs(S.re)) + shift, 0.0};
+}
+
+// log psi of the spins s (LDS) by the whole workgroup, one row per thread at a
+// time, log-cosh per hidden unit; c: [G] scratch.  Same value in every thread.
+__device__ inline cd slow_logpsi(const RbmGeom& g, const SymGeom& o, const double* __restrict__ P, const int32_t* s,
+                                 cd* c, double* red) {
+  double mx = -INFINITY;
+  for (int r = threadIdx.x; r < o.G; r += blockDim.x) {
+    cd a = {0.0, 0.0};
+    for (int h = 0; h < g.H; ++h) {
+      cd th = {g.ob >= 0 ? P[g.ob + h] : 0.0, g.cpx && g.ob >= 0 ? P[g.ob + g.H + h] : 0.0};
+      for (int i = 0; i < g.L; ++i) {
+        const double sg = row_spin(o, g.L, s, r, i) ? 1.0 : -1.0;
+        const int64_t w = g.ow + (int64_t)i * g.H + h;
+        th.re = fma(sg, P[w], th.re);
+        if (g.cpx) th.im = fma(sg, P[w + (int64_t)g.L * g.H], th.im);
+      }
+      a = a + (g.cpx ? log_cosh(th) : cd{log_cosh(th.re), 0.0});
+    }
+    if (g.oa >= 0)
+      for (int i = 0; i < g.L; ++i) {
+        const double sg = row_spin(o, g.L, s, r, i) ? 1.0 : -1.0;
+        a.re = fma(sg, P[g.oa + i], a.re);
+        a.im = fma(sg, P[g.oa + g.L + i], a.im);
+      }
+    c[r] = a;
+    if (o.fac[2 * r] != 0.0 || o.fac[2 * r + 1] != 0.0) mx = fmax(mx, a.re);
+  }
+  mx = block_max(mx, red);
+  if (!isfinite(mx)) mx = 0.0;
+  cd S = {0.0, 0.0};
+  for (int r = threadIdx.x; r < o.G; r += blockDim.x) {
+    const cd b = {o.fac[2 * r], o.fac[2 * r + 1]};
+    if (b.re == 0.0 && b.im == 0.0) continue;
+    const double e = exp(c[r].re - mx);
+    S = S + (o.cpx ? cd{e * cos(c[r].im), e * sin(c[r].im)} * b : cd{e * b.re, 0.0});
+  }
+  return log_of_sum(block_sum_cd(S, red), mx, o.cpx);
+}
+
+// ------------------------------------------------------------------ log psi
+// A workgroup per configuration: four threads per row, four hidden units at a
+// time.  FP64 issue (exp and sincos of every theta) sets its time.
+template <bool CPX>
+__global__ void __launch_bounds__(SYM_T, 3) sym_rbm_forward(RbmGeom g, SymGeom o, const double* __restrict__ P,
+                                                            RbmTab tab, const int32_t* __restrict__ cfg, int64_t n,
+                                                            double* __restrict__ out) {
+  typedef typename num_of<CPX>::type T;
+  extern __shared__ double lds[];
+  constexpr int SL = 4, RC = SYM_T / SL;
+  const int L = g.L, H = g.H, G = o.G, tid = threadIdx.x;
+  double* red = lds;
+  cd* lin = (cd*)(red + 8);  // [G]
+  cd* dd = lin + G;          // [G]
+  int32_t* s = (int32_t*)(dd + G);
+  unsigned char* rb = (unsigned char*)(s + L);  // [RC][L]
+  const bool ok = rbmq_ok(g, tab, 2, tid % WAVE);
+  for (int64_t q = blockIdx.x; q < n; q += gridDim.x) {
+    __syncthreads();
+    for (int i = tid; i < L; i += SYM_T) s[i] = cfg[q * L + i];
+    __syncthreads();
+    if (!ok) {
+      const cd lp = slow_logpsi(g, o, P, s, lin, red);
+      if (tid == 0) {
+        out[2 * q] = lp.re;
+        out[2 * q + 1] = lp.im;
+      }
+      continue;
+    }
+    double mx = -INFINITY;
+    for (int r0 = 0; r0 < G; r0 += RC) {
+      const int nr = min(RC, G - r0);
+      for (int t = tid; t < nr * L; t += SYM_T) rb[t] = row_spin(o, L, s, r0 + t / L, t % L);
+      __syncthreads();
+      const int r = tid / SL, sl = tid % SL;
+      if (r < nr) {
+        const unsigned char* row = rb + r * L;
+        cd li = visible(g, P, row, sl, SL);
+        T dp;
+        set_one(dp);
+        for (int h = 4 * sl; h < H; h += 4 * SL) {
+          cd th[4];
+          theta4<CPX>(g, P, row, h, th);
+#pragma unroll
+          for (int k = 0; k < 4; ++k)
+            if (h + k < H) {
+              T al, be, d;
+              cd l;
+              ab_of<CPX>(th[k], al, be, l, d);
+              li = li + l;
+              dp = mulc(dp, d);
+            }
+        }
+        for (int m = 1; m < SL; m *= 2) {
+          li = li + shfl_xor(li, m);
+          dp = mulc(dp, shfl_xor(dp, m));
+        }
+        if (sl == 0) {
+          lin[r0 + r] = li;
+          dd[r0 + r] = to_cd(dp);
+        }
+        if (o.fac[2 * (r0 + r)] != 0.0 || o.fac[2 * (r0 + r) + 1] != 0.0) mx = fmax(mx, li.re);
+      }
+      __syncthreads();
+    }
+    mx = block_max(mx, red);
+    if (!isfinite(mx)) mx = 0.0;
+    cd S = {0.0, 0.0};
+    for (int r = tid; r < G; r += SYM_T) {
+      const cd b = {o.fac[2 * r], o.fac[2 * r + 1]};
+      if (b.re == 0.0 && b.im == 0.0) continue;
+      S = S + mulc(mulc(cexp({fma(-(double)H, LN2, lin[r].re - mx), lin[r].im}), dd[r]), b);
+    }
+    const cd lp = log_of_sum(block_sum_cd(S, red), mx, o.cpx);
+    if (tid == 0) {
+      out[2 * q] = lp.re;
+      out[2 * q + 1] = lp.im;
+    }
+  }
+}
+size_t sym_fwd_lds(const RbmGeom& g, int G) {
+  return 8 * 8 + 32 * (size_t)G + 4 * (size_t)g.L + (size_t)(SYM_T / 4) * g.L + 16;
+}
+
+// ------------------------------------------------------------------ local energies
+// A workgroup per configuration.  The orbit in chunks of RC rows: four (eight,
+// sixteen) threads per row form alpha, beta and w_g; then lane = row (RC < 64:
+// several groups of strings per wave), a wave takes four strings at a time, so
+// that one read of (alpha, beta) serves four products, and sums them over its
+// rows.  LDS reads (24 bytes per row, unit and string) and FP64 issue bound it.
+// LDS of alpha, beta chooses RC: rows of 2 H + 1 entries (an odd number of
+// 16-byte units, so rows do not share banks).  TAB: the g table in LDS.
+// 4096 samples, 16 sites x 32 units, 64 elements, Ising chain: 17644 us with
+// materialised rows (4.5e6 forward passes).
+template <bool CPX, int RC, bool TAB>
+__global__ void __launch_bounds__(SYM_T, 2) sym_rbm_eloc(RbmGeom g, SymGeom o, const double* __restrict__ P,
+                                                         OpDev op, RbmTab tab, const int32_t* __restrict__ cfg,
+                                                         const double* __restrict__ lps, int64_t n, int nstr,
+                                                         double* __restrict__ out) {
+  typedef typename num_of<CPX>::type T;
+  extern __shared__ double lds[];
+  constexpr int SL = SYM_T / RC, NG = WAVE / RC * (SYM_T / WAVE);  // threads per row; groups of strings at once
+  const int L = g.L, H = g.H, G = o.G, tid = threadIdx.x, lane = tid % WAVE;
+  const int w = __builtin_amdgcn_readfirstlane(tid / WAVE);
+  const int stride = 2 * H + 1, gq = (nstr + 3) / 4;
+  double* red = lds;
+  T* ab = (T*)(red + 8);                  // [RC][2 H + 1]
+  T* he = ab + (size_t)RC * stride;       // [H][L][2] if TAB
+  // the row-by-row form's [G] sums take the place of alpha, beta and the table
+  const size_t abb = sizeof(T) * ((size_t)RC * stride + (TAB ? (size_t)2 * H * L : 0)), slowb = sizeof(cd) * (size_t)G;
+  cd* wt = (cd*)((char*)ab + (abb > slowb ? abb : slowb));  // [RC]
+  cd* mel = wt + RC;                      // [nstr] matrix elements
+  cd* sum = mel + nstr;                   // [4 gq] sums over the orbit
+  int32_t* site = (int32_t*)(sum + 4 * gq);  // [4 gq][2] changed sites, -1: none
+  int32_t* s = site + 8 * gq;
+  unsigned short* inv = (unsigned short*)(s + L);  // [RC][L]: position of a site in the row
+  unsigned char* rb = (unsigned char*)(inv + RC * L);  // [RC][L]
+  const int nl = tab.lead[0];
+  const bool ok = rbmq_ok(g, tab, 2, lane);
+  if (TAB && ok)
+    for (int t = tid; t < 2 * H * L; t += SYM_T) he[t] = ((const T*)tab.he)[t];
+  for (int64_t q = blockIdx.x; q < n; q += gridDim.x) {
+    const cd lq = {lps[2 * q], lps[2 * q + 1]};
+    __syncthreads();
+    for (int i = tid; i < L; i += SYM_T) s[i] = cfg[q * L + i];
+    __syncthreads();
+    // matrix elements; the merged diagonal strings (branch_free.py:483-485)
+    cd ds = {0.0, 0.0};
+    if (op.num_diag > 1)
+      for (int d = tid; d < op.num_diag; d += SYM_T) {
+        bool fa, fb;
+        ds = ds + string2(op, op.diag[d], s, fa, fb);
+      }
+    for (int j = tid; j < 4 * gq; j += SYM_T) {
+      cd m = {0.0, 0.0};
+      int sa = -1, sb = -1;
+      if (j < nl) {
+        const int code = tab.lead[1 + j], st = code >> 4, fol = code & 15;
+        for (int f = 0; f <= fol; ++f) {
+          bool fa, fb;
+          const cd mf = string2(op, st + f, s, fa, fb);
+          if (!nonzero(mf)) continue;
+          m = m + mf;
+          const int i0 = min(max(op.idx[(st + f) * op.max_len], 0), L - 1);
+          sa = fa ? i0 : -1;
+          sb = fb ? min(max(op.idx[(st + f) * op.max_len + 1], 0), L - 1) : -1;
+          if (sa < 0) {
+            sa = sb;
+            sb = -1;
+          }
+        }
+      }
+      if (j < nstr) mel[j] = m;
+      site[2 * j] = sa;
+      site[2 * j + 1] = sb;
+      sum[j] = {0.0, 0.0};
+    }
+    ds = block_sum_cd(ds, red);
+    if (!ok) {
+      // every s' from scratch
+      cd acc = {0.0, 0.0};
+      cd* c = (cd*)ab;
+      for (int j = -1; j < nl; ++j) {
+        const cd m = j < 0 ? ds : mel[j];
+        if (j < 0 ? !nonzero(m) : (m.re == 0.0 && m.im == 0.0)) continue;
+        __syncthreads();
+        if (j >= 0 && tid < 2 && site[2 * j + tid] >= 0) s[site[2 * j + tid]] = 1 - s[site[2 * j + tid]];
+        __syncthreads();
+        acc = acc + m * cexp(slow_logpsi(g, o, P, s, c, red) - lq);
+        __syncthreads();
+        if (j >= 0 && tid < 2 && site[2 * j + tid] >= 0) s[site[2 * j + tid]] = 1 - s[site[2 * j + tid]];
+      }
+      if (tid == 0) {
+        out[2 * q] = acc.re;
+        out[2 * q + 1] = acc.im;
+      }
+      continue;
+    }
+    cd base = {0.0, 0.0};  // sum_g w_g (threads that own a row's first slice)
+    for (int r0 = 0; r0 < G; r0 += RC) {
+      const int nr = min(RC, G - r0);
+      __syncthreads();
+      for (int t = tid; t < nr * L; t += SYM_T) {
+        const int r = t / L, i = t % L, m = o.map[(int64_t)(r0 + r) * L + i];
+        rb[t] = m >= 0 ? (s[m] > 0) : !(s[-1 - m] > 0);
+        inv[r * L + (m >= 0 ? m : -1 - m)] = (unsigned short)i;
+      }
+      __syncthreads();
+      {
+        const int r = tid / SL, sl = tid % SL;
+        if (r < nr) {
+          const unsigned char* row = rb + r * L;
+          cd li = visible(g, P, row, sl, SL);
+          T dp;
+          set_one(dp);
+          for (int h = 4 * sl; h < H; h += 4 * SL) {
+            cd th[4];
+            theta4<CPX>(g, P, row, h, th);
+#pragma unroll
+            for (int k = 0; k < 4; ++k)
+              if (h + k < H) {
+                T al, be, d;
+                cd l;
+                ab_of<CPX>(th[k], al, be, l, d);
+                li = li + l;
+                dp = mulc(dp, d);
+                ab[(size_t)r * stride + 2 * (h + k)] = al;
+                ab[(size_t)r * stride + 2 * (h + k) + 1] = be;
+              }
+          }
+          for (int m = 1; m < SL; m *= 2) {
+            li = li + shfl_xor(li, m);
+            dp = mulc(dp, shfl_xor(dp, m));
+          }
+          if (sl == 0) {
+            const cd b = {o.fac[2 * (r0 + r)], o.fac[2 * (r0 + r) + 1]};
+            cd x = {0.0, 0.0};
+            if (b.re != 0.0 || b.im != 0.0)
+              x = mulc(mulc(cexp({fma(-(double)H, LN2, li.re - lq.re), li.im - lq.im}), to_cd(dp)), b);
+            wt[r] = x;
+            base = base + x;
+          }
+        }
+      }
+      __syncthreads();
+      // products: row = lane % RC, strings 4 jg .. 4 jg + 3
+      const int r = lane % RC;
+      const T* arow = ab + (size_t)min(r, nr - 1) * stride;
+      const T* tabq = TAB ? (const T*)he : (const T*)tab.he;
+      for (int jg = w * (WAVE / RC) + lane / RC; jg < (gq + NG - 1) / NG * NG; jg += NG) {
+        const int j4 = 4 * min(jg, gq - 1);
+        int at[4], at2[4];
+        cd pre[4];
+        bool two = false;
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+          pre[k] = {1.0, 0.0};
+          at[k] = at2[k] = -1;
+          for (int z = 0; z < 2; ++z) {
+            const int si = site[2 * (j4 + k) + z];
+            if (si < 0) continue;
+            const int rr = min(r, nr - 1), i = inv[rr * L + si], v = rb[rr * L + i];
+            const double* pq = tab.site + 8 * (int64_t)i + 2 + 2 * v;
+            pre[k] = mulc(pre[k], cd{pq[0], pq[1]});
+            (z ? at2[k] : at[k]) = 2 * i + v;
+            two = two || z;
+          }
+        }
+        T pr[4];
+#pragma unroll
+        for (int k = 0; k < 4; ++k) set_one(pr[k]);
+        if (__any(two)) {
+          for (int h = 0; h < H; ++h) {
+            const T a = arow[2 * h], b = arow[2 * h + 1];
+            const T* qh = tabq + (size_t)2 * h * L;
+#pragma unroll
+            for (int k = 0; k < 4; ++k) {
+              T x = qh[max(at[k], 0)], y = qh[max(at2[k], 0)], one;
+              set_one(one);
+              y = sel(at2[k] >= 0, y, one);
+              pr[k] = mulc(pr[k], fmac(b, mulc(x, y), a));
+            }
+          }
+        } else {
+#pragma unroll 2
+          for (int h = 0; h < H; ++h) {
+            const T a = arow[2 * h], b = arow[2 * h + 1];
+            const T* qh = tabq + (size_t)2 * h * L;
+#pragma unroll
+            for (int k = 0; k < 4; ++k) pr[k] = mulc(pr[k], fmac(b, qh[max(at[k], 0)], a));
+          }
+        }
+        const cd wr = r < nr ? wt[r] : cd{0.0, 0.0};
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+          cd z = wr;
+          if (at[k] >= 0) z = mulc(mulc(to_cd(pr[k]), pre[k]), wr);
+          for (int m = 1; m < RC; m *= 2) z = z + shfl_xor(z, m);
+          if (r == 0 && jg < gq) sum[4 * jg + k] = sum[4 * jg + k] + z;
+        }
+      }
+    }
+    __syncthreads();
+    base = block_sum_cd(base, red);
+    // a negative sum of real terms has no logarithm (jax's logsumexp): NaN
+    cd acc = {0.0, 0.0};
+    for (int j = tid; j < nl; j += SYM_T) {
+      const cd m = mel[j];
+      if (m.re == 0.0 && m.im == 0.0) continue;
+      acc = acc + (!o.cpx && sum[j].re < 0.0 ? cd{NAN, NAN} : mulc(m, sum[j]));
+    }
+    if (tid == 0 && nonzero(ds)) acc = acc + (!o.cpx && base.re < 0.0 ? cd{NAN, NAN} : mulc(ds, base));
+    acc = block_sum_cd(acc, red);
+    if (tid == 0) {
+      out[2 * q] = acc.re;
+      out[2 * q + 1] = acc.im;
+    }
+  }
+}
+size_t sym_eloc_lds(const RbmGeom& g, int G, int RC, bool tabl, int nstr) {
+  const size_t cw = 8 * (size_t)rbm_cw(g), gq = (nstr + 3) / 4;
+  size_t abb = cw * RC * (2 * g.H + 1);
+  abb += tabl ? cw * 2 * g.H * g.L : 0;
+  // the row-by-row form keeps [G] sums where alpha, beta and the table are
+  return 64 + std::max(abb, (size_t)16 * G) + 16 * (size_t)RC + 16 * (size_t)nstr + 64 * gq + 32 * gq +
+         4 * (size_t)g.L + 3 * (size_t)RC * g.L + 16;
+}
+
+// ------------------------------------------------------------------ Metropolis chains
+// A workgroup per chain (sampler.py:264-367), SL threads per row, HT hidden
+// units each: e, alpha, beta live in registers, the spins and the flipped
+// position of every row in LDS.  A proposal: one product per row, a sum over
+// the orbit (one barrier: the partial sums alternate between two slots), the
+// decision, and on acceptance e' = e g and one reciprocal per unit.  Proposals
+// use the Philox counters of the other chain kernels.  theta is recomputed at
+// emissions at least RBMQ_MC_REFRESH proposals apart.
+// 1024 chains x 140 proposals, 16 sites x 32 units, 64 elements: 22.0 ms with
+// one batched forward per proposal.
+template <bool CPX, int HT, int MAXT>
+__global__ void __launch_bounds__(MAXT) sym_rbm_mc(RbmGeom g, SymGeom o, const double* __restrict__ P, jv_mc_args a,
+                                                   RbmTab tab, int SL, int tab_lds, int32_t* __restrict__ walkers,
+                                                   int32_t* __restrict__ configs, int64_t* __restrict__ counters) {
+  typedef typename num_of<CPX>::type T;
+  extern __shared__ double lds[];
+  const int L = g.L, H = g.H, G = o.G, tid = threadIdx.x, nt = blockDim.x, lane = tid % WAVE, nw = nt / WAVE;
+  const int chain = blockIdx.x;
+  double* red = lds;                     // block reductions; [2][16] complex partial sums of the proposals
+  cd* part = (cd*)(red + 16);
+  cd* slow = part + 32;                  // [G]
+  T* me = (T*)(slow + G);                // [L][2][H] if tab_lds
+  int32_t* s = (int32_t*)(me + (tab_lds ? (size_t)2 * L * H : 0));
+  unsigned short* inv = (unsigned short*)(s + L);  // [G][L]: 2 * position + (row holds the flipped spin)
+  unsigned char* rb = (unsigned char*)(inv + (size_t)G * L);  // [G][L] spins of the rows (refresh only)
+  const bool ok = rbmq_ok(g, tab, 2, lane);
+  for (int i = tid; i < L; i += nt) s[i] = walkers[(int64_t)chain * L + i] > 0;
+  if (tab_lds)
+    for (int t = tid; t < 2 * L * H; t += nt) me[t] = ((const T*)tab.me)[t];
+  for (int t = tid; t < G * L; t += nt) {
+    const int r = t / L, i = t % L, m = o.map[t];
+    inv[r * L + (m >= 0 ? m : -1 - m)] = (unsigned short)(2 * i + (m < 0));
+  }
+  __syncthreads();
+  const int r = tid / SL, sl = tid % SL, h0 = sl * HT;
+  const bool mine = r < G;
+  const int rc = min(r, G - 1);
+  const cd b = {o.fac[2 * rc], o.fac[2 * rc + 1]};
+  T e[HT], al[HT], be[HT];
+  cd wt = {0.0, 0.0};   // b_g psi_net(g s) up to a common factor (every lane of the row)
+  double cur2 = 0.0;    // |sum_g wt|^2
+  cd cur = {0.0, 0.0};  // slow form: log psi
+  auto refresh = [&]() {
+    if (!ok) {
+      cur = slow_logpsi(g, o, P, s, slow, red);
+      return;
+    }
+    __syncthreads();
+    for (int t = tid; t < G * L; t += nt) rb[t] = row_spin(o, L, s, t / L, t % L);
+    __syncthreads();
+    const unsigned char* row = rb + rc * L;
+    cd li = visible(g, P, row, sl, SL);
+    T dp;
+    set_one(dp);
+#pragma unroll
+    for (int k0 = 0; k0 < HT; k0 += 4) {
+      cd th[4];
+      theta4<CPX>(g, P, row, h0 + k0, th);
+#pragma unroll
+      for (int k = k0; k < k0 + 4 && k < HT; ++k) {
+        const bool in = h0 + k < H;
+        if constexpr (CPX) e[k] = in ? cexp({-2.0 * th[k - k0].re, -2.0 * th[k - k0].im}) : cd{0.0, 0.0};
+        else e[k] = in ? exp(-2.0 * th[k - k0].re) : 0.0;
+        al[k] = recip(plus1(e[k]));
+        be[k] = mulc(e[k], al[k]);
+        // cosh theta = e^{theta} (1 + e) / 2 with |1 + e| <= 2 on the side where |e| <= 1
+        const bool neg = th[k - k0].re < 0.0;
+        if (in) {
+          li = li + (neg ? cd{-th[k - k0].re, -th[k - k0].im} : th[k - k0]);
+          dp = mulc(dp, sel(neg, be[k], al[k]));
+        }
+      }
+    }
+    for (int m = 1; m < SL; m *= 2) {
+      li = li + shfl_xor(li, m);
+      dp = mulc(dp, shfl_xor(dp, m));
+    }
+    const bool on = mine && (b.re != 0.0 || b.im != 0.0);
+    double mx = block_max(on ? li.re : -INFINITY, red);
+    if (!isfinite(mx)) mx = 0.0;
+    wt = on ? mulc(mulc(cexp({fma(-(double)H, LN2, li.re - mx), li.im}), to_cd(recip(dp))), b) : cd{0.0, 0.0};
+    const cd S = block_sum_cd(sl == 0 ? wt : cd{0.0, 0.0}, red);
+    cur2 = !o.cpx && S.re < 0.0 ? NAN : norm2(S);
+  };
+  refresh();
+  const int total = a.therm_steps + a.samples_per_chain * a.sweep_steps;
+  int dsite = 0;
+  double du = 0.0;
+  int64_t nacc = 0;
+  int since = 0, left = a.therm_steps + a.sweep_steps;
+  int64_t row_out = chain;
+  for (int step = 0; step < total; ++step) {
+    const int k64 = step & 63;
+    if (k64 == 0 && step + lane < total)
+      mc_draw(a.seed, (uint32_t)(step + lane), (uint32_t)chain, a.call_index, a.stream, L, dsite, du);
+    const int site = __builtin_amdgcn_readlane(dsite, k64);
+    const double u = __hiloint2double(__builtin_amdgcn_readlane(__double2hiint(du), k64),
+                                      __builtin_amdgcn_readlane(__double2loint(du), k64));
+    bool acc;
+    if (!ok) {
+      __syncthreads();
+      if (tid == 0) s[site] = 1 - s[site];
+      __syncthreads();
+      const cd lp = slow_logpsi(g, o, P, s, slow, red);
+      acc = u < exp(a.mu * lp.re - a.mu * cur.re);
+      __syncthreads();
+      if (tid == 0 && !acc) s[site] = 1 - s[site];
+      __syncthreads();
+      if (acc) cur = lp;
+    } else {
+      const int iv = inv[rc * L + site], pos = iv >> 1, v = s[site] ^ (iv & 1);
+      T gq[HT], pr;
+      set_one(pr);
+      const int64_t at = (int64_t)(2 * pos + v) * H;
+#pragma unroll
+      for (int k = 0; k < HT; ++k) {
+        const int hc = min(h0 + k, H - 1);
+        gq[k] = tab_lds ? me[at + hc] : ((const T*)tab.me)[at + hc];
+        pr = mulc(pr, fmac(be[k], gq[k], al[k]));
+      }
+      for (int m = 1; m < SL; m *= 2) pr = mulc(pr, shfl_xor(pr, m));
+      const double* pq = tab.site + 8 * (int64_t)pos + 2 + 2 * v;
+      const cd z = mulc(mulc(to_cd(pr), cd{pq[0], pq[1]}), wt);
+      const double zr = wave_sum(mine && sl == 0 ? z.re : 0.0), zi = o.cpx ? wave_sum(mine && sl == 0 ? z.im : 0.0) : 0.0;
+      cd* slot = part + 16 * (step & 1);
+      if (lane == 0) slot[tid / WAVE] = {zr, zi};
+      __syncthreads();
+      cd S = slot[0];
+      for (int i = 1; i < nw; ++i) S = S + slot[i];
+      const double new2 = !o.cpx && S.re < 0.0 ? NAN : norm2(S);
+      // random.bernoulli(key, P), sampler.py:336-340
+      acc = a.mu == 2.0 ? u * cur2 < new2 : u < exp(a.mu * (0.5 * log(new2) - 0.5 * log(cur2)));
+      if (acc) {
+#pragma unroll
+        for (int k = 0; k < HT; ++k)
+          if (h0 + k < H) {
+            e[k] = mulc(e[k], gq[k]);
+            al[k] = recip(plus1(e[k]));
+            be[k] = mulc(e[k], al[k]);
+          }
+        const double sc = new2 > 0.0 ? 1.0 / sqrt(new2) : 1.0;
+        wt = {z.re * sc, z.im * sc};
+        cur2 = new2 > 0.0 ? 1.0 : 0.0;
+        if (tid == 0) s[site] ^= 1;
+      }
+      // the flip is seen by the other waves after the next barrier; a proposal
+      // at the same site right after needs it now
+      __syncthreads();
+    }
+    nacc += acc;
+    ++since;
+    if (--left == 0) {
+      left = a.sweep_steps;
+      int32_t* out = configs + row_out * L;
+      row_out += a.num_chains;
+      for (int i = tid; i < L; i += nt) out[i] = s[i];
+      if (since >= RBMQ_MC_REFRESH) {
+        refresh();
+        since = 0;
+      }
+    }
+  }
+  for (int i = tid; i < L; i += nt) walkers[(int64_t)chain * L + i] = s[i];
+  if (tid == 0) {
+    atomicAdd((unsigned long long*)&counters[0], (unsigned long long)total);
+    atomicAdd((unsigned long long*)&counters[1], (unsigned long long)nacc);
+  }
+}
+size_t sym_mc_lds(const RbmGeom& g, int G, bool tabl) {
+  return 8 * 16 + 16 * 32 + 16 * (size_t)G + (tabl ? 8 * (size_t)rbm_cw(g) * 2 * g.L * g.H : 0) + 4 * (size_t)g.L +
+         3 * (size_t)G * g.L + 16;
+}
+
+__global__ void sym_zero_counters(int64_t* c) {
+  if (threadIdx.x < 2) c[threadIdx.x] = 0;
+}
+
+bool sym_rbm_geom(const jv_net* net, const jv_orbit* orbit, RbmGeom& g, SymGeom& o) {
+  if (orbit->avg != JV_AVG_EXP || !make_rbm_geom(net, g)) return false;
+  o.G = orbit->num_elements;
+  o.cpx = net->is_complex || orbit->complex_factor;
+  o.map = orbit->map;
+  o.fac = orbit->factor;
+  return o.G <= SYM_MAX_G && g.H <= RBMQ_MAX_H && g.L <= 16384;
+}
+
+}  // namespace
+
+// Each returns JV_OK with *done = true when the resident form applies (RBM,
+// avgFun_Coefficients_Exp, LDS and registers suffice), else *done = false.
+int sym_rbm_forward_launch(const jv_net* net, const double* params, const jv_orbit* orbit, const int32_t* configs,
+                           int64_t n, double* logpsi, hipStream_t st, int slot0, bool* done) {
+  *done = false;
+  RbmGeom g;
+  SymGeom o;
+  if (!sym_rbm_geom(net, orbit, g, o)) return JV_OK;
+  const size_t lds = sym_fwd_lds(g, o.G);
+  if (lds > 160 * 1024) return JV_OK;
+  RbmTab tab;
+  int rc = build_rbm_tables(g, params, nullptr, false, false, st, slot0, &tab);
+  const auto fn = g.cpx ? sym_rbm_forward<true> : sym_rbm_forward<false>;
+  if (!rc) rc = set_lds_limit((const void*)fn, lds);
+  if (rc) return rc;
+  hipLaunchKernelGGL(fn, dim3((unsigned)std::min<int64_t>(n, 1 << 20)), dim3(SYM_T), lds, st, g, o, params, tab, configs,
+                     n, logpsi);
+  JV_LAUNCH_CHECK("sym_rbm_forward");
+  *done = true;
+  return JV_OK;
+}
+
+int sym_rbm_eloc_launch(const jv_net* net, const double* params, const jv_orbit* orbit, const jv_optable* op,
+                        const double* prefactor, const int32_t* configs, const double* lps, int64_t n, double* out,
+                        hipStream_t st, int slot0, bool* done) {
+  *done = false;
+  RbmGeom g;
+  SymGeom o;
+  if (!sym_rbm_geom(net, orbit, g, o) || op->max_len > 2 || op->fermi || !prefactor) return JV_OK;
+  const OpDev d = make_opdev(op, prefactor, net->num_sites);
+  const int nstr = rbmq_strings(d);
+  // the most rows at once, with the table in LDS where two workgroups still
+  // share a CU (or where it fits at all beside the rows)
+  int RC = 0;
+  bool tabl = false;
+  size_t lds = 0;
+  for (int rows : {64, 32, 16}) {
+    if (RC) break;
+    for (bool t : {true, false}) {
+      const size_t b = sym_eloc_lds(g, o.G, rows, t, nstr);
+      if (b <= (size_t)(t ? 80 : 160) * 1024 || (t && rows == 64 && b <= 160 * 1024)) {
+        RC = rows;
+        tabl = t;
+        lds = b;
+        break;
+      }
+    }
+  }
+  if (!RC) return JV_OK;
+  RbmTab tab;
+  int rc = build_rbm_tables(g, params, &d, false, true, st, slot0, &tab);
+  if (rc) return rc;
+#define JV_SYM_ELO(RCv)                                                                           \
+  (g.cpx ? (tabl ? sym_rbm_eloc<true, RCv, true> : sym_rbm_eloc<true, RCv, false>)                \
+         : (tabl ? sym_rbm_eloc<false, RCv, true> : sym_rbm_eloc<false, RCv, false>))
+  const auto fn = RC == 64 ? JV_SYM_ELO(64) : RC == 32 ? JV_SYM_ELO(32) : JV_SYM_ELO(16);
+#undef JV_SYM_ELO
+  rc = set_lds_limit((const void*)fn, lds);
+  if (rc) return rc;
+  hipLaunchKernelGGL(fn, dim3((unsigned)std::min<int64_t>(n, 4096)), dim3(SYM_T), lds, st, g, o, params, d, tab, configs,
+                     lps, n, nstr, out);
+  JV_LAUNCH_CHECK("sym_rbm_eloc");
+  *done = true;
+  return JV_OK;
+}
+
+int sym_rbm_mc_launch(const jv_net* net, const double* params, const jv_orbit* orbit, const jv_mc_args& a,
+                      int32_t* walkers, int32_t* configs, int64_t* counters, hipStream_t st, int slot0, bool* done) {
+  *done = false;
+  RbmGeom g;
+  SymGeom o;
+  if (!sym_rbm_geom(net, orbit, g, o) || g.H > RBMQ_MC_MAX_H) return JV_OK;
+  // hidden units per thread: as many as leave the fewest threads (a power of
+  // two of them per row, inside one wave), with registers for 512 threads of
+  // eight units or 1024 of four
+  int HT = 0, SL = 0;
+  for (int ht : {8, 4}) {
+    int sl = 1;
+    while (sl * ht < g.H) sl *= 2;
+    if (!HT && sl <= WAVE && (int64_t)o.G * sl <= (ht == 8 ? 512 : 1024)) {
+      HT = ht;
+      SL = sl;
+    }
+  }
+  if (!HT) return JV_OK;
+  const bool tabl = sym_mc_lds(g, o.G, true) <= 64 * 1024;
+  const size_t lds = sym_mc_lds(g, o.G, tabl);
+  if (lds > 160 * 1024) return JV_OK;
+  RbmTab tab;
+  int rc = build_rbm_tables(g, params, nullptr, true, false, st, slot0, &tab);
+  if (rc) return rc;
+  const int T = (o.G * SL + WAVE - 1) / WAVE * WAVE;
+  const auto fn = HT == 8 ? (T <= 256 ? (g.cpx ? sym_rbm_mc<true, 8, 256> : sym_rbm_mc<false, 8, 256>)
+                                      : (g.cpx ? sym_rbm_mc<true, 8, 512> : sym_rbm_mc<false, 8, 512>))
+                          : (g.cpx ? sym_rbm_mc<true, 4, 1024> : sym_rbm_mc<false, 4, 1024>);
+  rc = set_lds_limit((const void*)fn, lds);
+  if (rc) return rc;
+  hipLaunchKernelGGL(sym_zero_counters, dim3(1), dim3(64), 0, st, counters);
+  JV_LAUNCH_CHECK("sym_zero_counters");
+  hipLaunchKernelGGL(fn, dim3((unsigned)a.num_chains), dim3(T), lds, st, g, o, params, a, tab, SL, (int)tabl, walkers,
+                     configs, counters);
+  JV_LAUNCH_CHECK("sym_rbm_mc");
+  *done = true;
+  return JV_OK;
+}
+
+}  // namespace jv
