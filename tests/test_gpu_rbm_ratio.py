@@ -177,3 +177,54 @@ def test_chains(cpx, L, H, bias, vbias, mu, big):
         assert _rel(to_np(lp)[0], lpo) < TOL
     assert np.array_equal(to_np(ms.states), mo.states)
     assert abs(float(ms.acceptance_ratio()[0]) - float(np.ravel(mo.acceptance_ratio())[0])) < 1e-15
+
+
+def _sym_states(cpx, L, H, names, P, **kw):
+    import warnings
+
+    from oracle import symmetries as osym
+    with warnings.catch_warnings():
+        warnings.simplefilter("ignore", UserWarning)
+        orb = jv.util.symmetries.get_orbit_1D(L, *names, **kw)
+        d, f = osym.orbit_1d(L, *names, **kw)
+    net, onet = (jv.nets.CpxRBM(H, bias=True), onets.CpxRBM((L,), H, bias=True)) if cpx else \
+        (jv.nets.RBM(H, bias=True), onets.RBM((L,), H, bias=True))
+    psi = jv.NQS(net, orbit=orb)
+    psi(torch.zeros((1, 1, L), dtype=torch.int32))
+    psi.set_parameters(P)
+    return psi, onets.NQS(osym.SymNet(onet, d, f, "exp"), P)
+
+
+ALL = ("translation", "reflection", "spinflip")
+
+
+@pytest.mark.parametrize("cpx,L,H,names,op,big", [
+    (True, 5, 1, ("reflection",), "tfim", 0.0), (True, 17, 9, ALL, "xxz", 0.0), (False, 9, 33, ALL, "mixed", 0.0),
+    (True, 12, 70, ("translation",), "tfim", 0.0), (True, 9, 150, ALL, "xxz", 0.0), (True, 6, 300, ("translation",), "mixed", 0.0),
+    (True, 33, 8, ALL, "tfim", 0.0), (True, 6, 8, ALL, "mixed", 10.0), (True, 6, 5, ALL, "long", 0.0)])
+def test_sym_resident(cpx, L, H, names, op, big):
+    """Symmetrised RBMs: log psi, local energies and chains against the oracle
+    over row counts below, at and above the kernels' chunks (2 to 132), units
+    beyond one pass, the smaller row tiles, a group and unit count too large
+    for one workgroup's chain, out-of-range weights, and strings the resident
+    form leaves to the materialised one."""
+    rng = np.random.default_rng(L * 1000 + H)
+    P = 0.3 / np.sqrt(L) * rng.normal(size=_num(cpx, L, H, True, False))
+    if big:
+        P[2 * H:3 * H] = big
+    psi, opsi = _sym_states(cpx, L, H, names, P)
+    s = rng.integers(0, 2, size=(7, L)).astype(np.int32)
+    sd = torch.as_tensor(s[None], device="cuda")
+    lp, lpo = psi(sd), opsi(s)
+    assert np.max(np.abs(to_np(lp)[0] - lpo)) < TOL * np.max(np.abs(lpo))
+    Hd, Ho = OPS[op](L)
+    e = to_np(Hd.get_O_loc(sd, psi, lp))[0]
+    assert _rel(e, Ho.get_O_loc(s, opsi, lpo)) < TOL
+    kw = dict(numChains=3, numSamples=9, thermalizationSweeps=3, sweepSteps=50)
+    ms = jv.sampler.MCSampler(psi, (L,), 5, updateProposer=jv.sampler.propose_spin_flip, **kw)
+    mo = osamp.MCSampler(opsi, (L,), 5, **kw)
+    for _ in range(2):
+        so = mo.sample()[0]
+        assert np.array_equal(to_np(ms.sample()[0])[0], so)
+    assert np.array_equal(to_np(ms.states), mo.states)
+    assert float(ms.acceptance_ratio()[0]) == float(np.ravel(mo.acceptance_ratio())[0])

@@ -39,26 +39,41 @@ __device__ inline int row_spin(const SymGeom& o, int L, const int32_t* s, int r,
   return m >= 0 ? (s[m] > 0) : !(s[-1 - m] > 0);
 }
 
+struct quad {
+  double v[4];
+};
+// Four neighbouring doubles (two 16-byte loads; h + 3 < H), or the clamped ones.
+__device__ inline quad load4(const double* __restrict__ p, int h, int H) {
+  quad q;
+  if (h + 4 <= H) {
+    q = *(const quad*)(p + h);
+  } else {
+#pragma unroll
+    for (int k = 0; k < 4; ++k) q.v[k] = p[min(h + k, H - 1)];
+  }
+  return q;
+}
 // theta of hidden units h .. h + 3 (clamped to H - 1) for one row's spins.
 template <bool CPX>
 __device__ inline void theta4(const RbmGeom& g, const double* __restrict__ P, const unsigned char* row, int h,
                               cd* th) {
   const double* Wr = P + g.ow;
   const double* Wi = Wr + (int64_t)g.L * g.H;
-  int hc[4];
 #pragma unroll
   for (int k = 0; k < 4; ++k) {
-    hc[k] = min(h + k, g.H - 1);
-    th[k] = {g.ob >= 0 ? P[g.ob + hc[k]] : 0.0, CPX && g.ob >= 0 ? P[g.ob + g.H + hc[k]] : 0.0};
+    const int hc = min(h + k, g.H - 1);
+    th[k] = {g.ob >= 0 ? P[g.ob + hc] : 0.0, CPX && g.ob >= 0 ? P[g.ob + g.H + hc] : 0.0};
   }
 #pragma unroll 4
   for (int i = 0; i < g.L; ++i) {
     const double sg = row[i] ? 1.0 : -1.0;
-    const int64_t w = (int64_t)i * g.H;
+    const quad wr = load4(Wr + (int64_t)i * g.H, h, g.H);
+    quad wm = wr;
+    if (CPX) wm = load4(Wi + (int64_t)i * g.H, h, g.H);
 #pragma unroll
     for (int k = 0; k < 4; ++k) {
-      th[k].re = fma(sg, Wr[w + hc[k]], th[k].re);
-      if (CPX) th[k].im = fma(sg, Wi[w + hc[k]], th[k].im);
+      th[k].re = fma(sg, wr.v[k], th[k].re);
+      if (CPX) th[k].im = fma(sg, wm.v[k], th[k].im);
     }
   }
 }
@@ -105,7 +120,7 @@ __device__ inline cd log_of_sum(cd S, double shift, int cpx) {
 
 // log psi of the spins s (LDS) by the whole workgroup, one row per thread at a
 // time, log-cosh per hidden unit; c: [G] scratch.  Same value in every thread.
-__device__ inline cd slow_logpsi(const RbmGeom& g, const SymGeom& o, const double* __restrict__ P, const int32_t* s,
+__device__ __forceinline__ cd slow_logpsi(const RbmGeom& g, const SymGeom& o, const double* __restrict__ P, const int32_t* s,
                                  cd* c, double* red) {
   double mx = -INFINITY;
   for (int r = threadIdx.x; r < o.G; r += blockDim.x) {
@@ -143,9 +158,10 @@ __device__ inline cd slow_logpsi(const RbmGeom& g, const SymGeom& o, const doubl
 
 // ------------------------------------------------------------------ log psi
 // A workgroup per configuration: four threads per row, four hidden units at a
-// time.  FP64 issue (exp and sincos of every theta) sets its time.
+// time.  FP64 issue (exp and sincos of every theta) sets its time: 4096
+// samples, 16 sites x 32 units, 64 elements 600 -> 100 us.
 template <bool CPX>
-__global__ void __launch_bounds__(SYM_T, 3) sym_rbm_forward(RbmGeom g, SymGeom o, const double* __restrict__ P,
+__global__ void __launch_bounds__(SYM_T, 2) sym_rbm_forward(RbmGeom g, SymGeom o, const double* __restrict__ P,
                                                             RbmTab tab, const int32_t* __restrict__ cfg, int64_t n,
                                                             double* __restrict__ out) {
   typedef typename num_of<CPX>::type T;
@@ -157,19 +173,11 @@ __global__ void __launch_bounds__(SYM_T, 3) sym_rbm_forward(RbmGeom g, SymGeom o
   cd* dd = lin + G;          // [G]
   int32_t* s = (int32_t*)(dd + G);
   unsigned char* rb = (unsigned char*)(s + L);  // [RC][L]
-  const bool ok = rbmq_ok(g, tab, 2, tid % WAVE);
+  if (!rbmq_ok(g, tab, 2, tid % WAVE)) return;  // sym_slow_forward's
   for (int64_t q = blockIdx.x; q < n; q += gridDim.x) {
     __syncthreads();
     for (int i = tid; i < L; i += SYM_T) s[i] = cfg[q * L + i];
     __syncthreads();
-    if (!ok) {
-      const cd lp = slow_logpsi(g, o, P, s, lin, red);
-      if (tid == 0) {
-        out[2 * q] = lp.re;
-        out[2 * q + 1] = lp.im;
-      }
-      continue;
-    }
     double mx = -INFINITY;
     for (int r0 = 0; r0 < G; r0 += RC) {
       const int nr = min(RC, G - r0);
@@ -234,7 +242,8 @@ size_t sym_fwd_lds(const RbmGeom& g, int G) {
 // LDS of alpha, beta chooses RC: rows of 2 H + 1 entries (an odd number of
 // 16-byte units, so rows do not share banks).  TAB: the g table in LDS.
 // 4096 samples, 16 sites x 32 units, 64 elements, Ising chain: 17644 us with
-// materialised rows (4.5e6 forward passes).
+// materialised rows (4.5e6 forward passes), 455 us here (716 with 64 rows and
+// one workgroup per CU).
 template <bool CPX, int RC, bool TAB>
 __global__ void __launch_bounds__(SYM_T, 2) sym_rbm_eloc(RbmGeom g, SymGeom o, const double* __restrict__ P,
                                                          OpDev op, RbmTab tab, const int32_t* __restrict__ cfg,
@@ -249,9 +258,7 @@ __global__ void __launch_bounds__(SYM_T, 2) sym_rbm_eloc(RbmGeom g, SymGeom o, c
   double* red = lds;
   T* ab = (T*)(red + 8);                  // [RC][2 H + 1]
   T* he = ab + (size_t)RC * stride;       // [H][L][2] if TAB
-  // the row-by-row form's [G] sums take the place of alpha, beta and the table
-  const size_t abb = sizeof(T) * ((size_t)RC * stride + (TAB ? (size_t)2 * H * L : 0)), slowb = sizeof(cd) * (size_t)G;
-  cd* wt = (cd*)((char*)ab + (abb > slowb ? abb : slowb));  // [RC]
+  cd* wt = (cd*)(he + (TAB ? (size_t)2 * H * L : 0));  // [RC]
   cd* mel = wt + RC;                      // [nstr] matrix elements
   cd* sum = mel + nstr;                   // [4 gq] sums over the orbit
   int32_t* site = (int32_t*)(sum + 4 * gq);  // [4 gq][2] changed sites, -1: none
@@ -259,8 +266,8 @@ __global__ void __launch_bounds__(SYM_T, 2) sym_rbm_eloc(RbmGeom g, SymGeom o, c
   unsigned short* inv = (unsigned short*)(s + L);  // [RC][L]: position of a site in the row
   unsigned char* rb = (unsigned char*)(inv + RC * L);  // [RC][L]
   const int nl = tab.lead[0];
-  const bool ok = rbmq_ok(g, tab, 2, lane);
-  if (TAB && ok)
+  if (!rbmq_ok(g, tab, 2, lane)) return;  // sym_slow_eloc's
+  if (TAB)
     for (int t = tid; t < 2 * H * L; t += SYM_T) he[t] = ((const T*)tab.he)[t];
   for (int64_t q = blockIdx.x; q < n; q += gridDim.x) {
     const cd lq = {lps[2 * q], lps[2 * q + 1]};
@@ -299,26 +306,6 @@ __global__ void __launch_bounds__(SYM_T, 2) sym_rbm_eloc(RbmGeom g, SymGeom o, c
       sum[j] = {0.0, 0.0};
     }
     ds = block_sum_cd(ds, red);
-    if (!ok) {
-      // every s' from scratch
-      cd acc = {0.0, 0.0};
-      cd* c = (cd*)ab;
-      for (int j = -1; j < nl; ++j) {
-        const cd m = j < 0 ? ds : mel[j];
-        if (j < 0 ? !nonzero(m) : (m.re == 0.0 && m.im == 0.0)) continue;
-        __syncthreads();
-        if (j >= 0 && tid < 2 && site[2 * j + tid] >= 0) s[site[2 * j + tid]] = 1 - s[site[2 * j + tid]];
-        __syncthreads();
-        acc = acc + m * cexp(slow_logpsi(g, o, P, s, c, red) - lq);
-        __syncthreads();
-        if (j >= 0 && tid < 2 && site[2 * j + tid] >= 0) s[site[2 * j + tid]] = 1 - s[site[2 * j + tid]];
-      }
-      if (tid == 0) {
-        out[2 * q] = acc.re;
-        out[2 * q + 1] = acc.im;
-      }
-      continue;
-    }
     cd base = {0.0, 0.0};  // sum_g w_g (threads that own a row's first slice)
     for (int r0 = 0; r0 < G; r0 += RC) {
       const int nr = min(RC, G - r0);
@@ -440,28 +427,30 @@ __global__ void __launch_bounds__(SYM_T, 2) sym_rbm_eloc(RbmGeom g, SymGeom o, c
     }
   }
 }
-size_t sym_eloc_lds(const RbmGeom& g, int G, int RC, bool tabl, int nstr) {
+size_t sym_eloc_lds(const RbmGeom& g, int RC, bool tabl, int nstr) {
   const size_t cw = 8 * (size_t)rbm_cw(g), gq = (nstr + 3) / 4;
   size_t abb = cw * RC * (2 * g.H + 1);
   abb += tabl ? cw * 2 * g.H * g.L : 0;
-  // the row-by-row form keeps [G] sums where alpha, beta and the table are
-  return 64 + std::max(abb, (size_t)16 * G) + 16 * (size_t)RC + 16 * (size_t)nstr + 64 * gq + 32 * gq +
+  return 64 + abb + 16 * (size_t)RC + 16 * (size_t)nstr + 64 * gq + 32 * gq +
          4 * (size_t)g.L + 3 * (size_t)RC * g.L + 16;
 }
 
 // ------------------------------------------------------------------ Metropolis chains
 // A workgroup per chain (sampler.py:264-367), SL threads per row, HT hidden
-// units each: e, alpha, beta live in registers, the spins and the flipped
+// units each: e and alpha live in registers, the spins and the flipped
 // position of every row in LDS.  A proposal: one product per row, a sum over
 // the orbit (one barrier: the partial sums alternate between two slots), the
 // decision, and on acceptance e' = e g and one reciprocal per unit.  Proposals
 // use the Philox counters of the other chain kernels.  theta is recomputed at
-// emissions at least RBMQ_MC_REFRESH proposals apart.
+// emissions at least RBMQ_MC_REFRESH proposals apart.  Registers decide how
+// many chains share a CU: beta = e alpha is not kept (three waves per SIMD
+// instead of one).
 // 1024 chains x 140 proposals, 16 sites x 32 units, 64 elements: 22.0 ms with
-// one batched forward per proposal.
-template <bool CPX, int HT, int MAXT>
-__global__ void __launch_bounds__(MAXT) sym_rbm_mc(RbmGeom g, SymGeom o, const double* __restrict__ P, jv_mc_args a,
-                                                   RbmTab tab, int SL, int tab_lds, int32_t* __restrict__ walkers,
+// one batched forward per proposal, 1.26 ms here (1.34 with beta kept, one
+// workgroup per CU); about 450 FP64 instructions per wave and proposal.
+template <bool CPX, int HT, int MAXT, bool TAB>
+__global__ void __launch_bounds__(MAXT, MAXT == 256 ? 3 : MAXT == 512 ? 2 : 4) sym_rbm_mc(RbmGeom g, SymGeom o, const double* __restrict__ P, jv_mc_args a,
+                                                   RbmTab tab, int SL, int32_t* __restrict__ walkers,
                                                    int32_t* __restrict__ configs, int64_t* __restrict__ counters) {
   typedef typename num_of<CPX>::type T;
   extern __shared__ double lds[];
@@ -469,33 +458,46 @@ __global__ void __launch_bounds__(MAXT) sym_rbm_mc(RbmGeom g, SymGeom o, const d
   const int chain = blockIdx.x;
   double* red = lds;                     // block reductions; [2][16] complex partial sums of the proposals
   cd* part = (cd*)(red + 16);
-  cd* slow = part + 32;                  // [G]
-  T* me = (T*)(slow + G);                // [L][2][H] if tab_lds
-  int32_t* s = (int32_t*)(me + (tab_lds ? (size_t)2 * L * H : 0));
+  cd* pre = part + 32;                   // [L][2]
+  T* me = (T*)(pre + 2 * L);                // [L][2][HP] if TAB, HP odd: rows do not share banks
+  const int HP = H | 1;
+  int32_t* s = (int32_t*)(me + (TAB ? (size_t)2 * L * HP : 0));
   unsigned short* inv = (unsigned short*)(s + L);  // [G][L]: 2 * position + (row holds the flipped spin)
   unsigned char* rb = (unsigned char*)(inv + (size_t)G * L);  // [G][L] spins of the rows (refresh only)
-  const bool ok = rbmq_ok(g, tab, 2, lane);
+  if (!rbmq_ok(g, tab, 2, lane)) return;  // sym_slow_mc's
   for (int i = tid; i < L; i += nt) s[i] = walkers[(int64_t)chain * L + i] > 0;
-  if (tab_lds)
-    for (int t = tid; t < 2 * L * H; t += nt) me[t] = ((const T*)tab.me)[t];
+  for (int t = tid; t < 2 * L; t += nt) {
+    const double* pq = tab.site + 8 * (int64_t)(t / 2) + 2 + 2 * (t % 2);
+    pre[t] = {pq[0], pq[1]};
+  }
+  if constexpr (TAB)
+    for (int t = tid; t < 2 * L * H; t += nt) me[t / H * HP + t % H] = ((const T*)tab.me)[t];
   for (int t = tid; t < G * L; t += nt) {
     const int r = t / L, i = t % L, m = o.map[t];
     inv[r * L + (m >= 0 ? m : -1 - m)] = (unsigned short)(2 * i + (m < 0));
   }
   __syncthreads();
+  // the ratio form keeps the spins in every wave's registers too (bit w of lane
+  // l: site 64 w + l), so one barrier per proposal suffices
+  const int words = (L + WAVE - 1) / WAVE;
+  uint32_t sp = 0;
+  for (int w = 0; w < words; ++w)
+    if (w * WAVE + lane < L && s[w * WAVE + lane]) sp |= 1u << w;
+  auto spins_out = [&]() {  // registers -> s (all threads call)
+    __syncthreads();
+    if (tid < WAVE)
+      for (int w = 0; w < words; ++w)
+        if (w * WAVE + lane < L) s[w * WAVE + lane] = (sp >> w) & 1;
+    __syncthreads();
+  };
   const int r = tid / SL, sl = tid % SL, h0 = sl * HT;
   const bool mine = r < G;
   const int rc = min(r, G - 1);
   const cd b = {o.fac[2 * rc], o.fac[2 * rc + 1]};
-  T e[HT], al[HT], be[HT];
+  T e[HT], al[HT];
   cd wt = {0.0, 0.0};   // b_g psi_net(g s) up to a common factor (every lane of the row)
   double cur2 = 0.0;    // |sum_g wt|^2
-  cd cur = {0.0, 0.0};  // slow form: log psi
-  auto refresh = [&]() {
-    if (!ok) {
-      cur = slow_logpsi(g, o, P, s, slow, red);
-      return;
-    }
+  auto refresh = [&]() __attribute__((always_inline)) {
     __syncthreads();
     for (int t = tid; t < G * L; t += nt) rb[t] = row_spin(o, L, s, t / L, t % L);
     __syncthreads();
@@ -508,17 +510,17 @@ __global__ void __launch_bounds__(MAXT) sym_rbm_mc(RbmGeom g, SymGeom o, const d
       cd th[4];
       theta4<CPX>(g, P, row, h0 + k0, th);
 #pragma unroll
-      for (int k = k0; k < k0 + 4 && k < HT; ++k) {
+      for (int j = 0; j < 4; ++j) {
+        const int k = k0 + j;
         const bool in = h0 + k < H;
-        if constexpr (CPX) e[k] = in ? cexp({-2.0 * th[k - k0].re, -2.0 * th[k - k0].im}) : cd{0.0, 0.0};
-        else e[k] = in ? exp(-2.0 * th[k - k0].re) : 0.0;
+        if constexpr (CPX) e[k] = in ? cexp({-2.0 * th[j].re, -2.0 * th[j].im}) : cd{0.0, 0.0};
+        else e[k] = in ? exp(-2.0 * th[j].re) : 0.0;
         al[k] = recip(plus1(e[k]));
-        be[k] = mulc(e[k], al[k]);
         // cosh theta = e^{theta} (1 + e) / 2 with |1 + e| <= 2 on the side where |e| <= 1
-        const bool neg = th[k - k0].re < 0.0;
+        const bool neg = th[j].re < 0.0;
         if (in) {
-          li = li + (neg ? cd{-th[k - k0].re, -th[k - k0].im} : th[k - k0]);
-          dp = mulc(dp, sel(neg, be[k], al[k]));
+          li = li + (neg ? cd{-th[j].re, -th[j].im} : th[j]);
+          dp = mulc(dp, sel(neg, mulc(e[k], al[k]), al[k]));
         }
       }
     }
@@ -547,56 +549,39 @@ __global__ void __launch_bounds__(MAXT) sym_rbm_mc(RbmGeom g, SymGeom o, const d
     const int site = __builtin_amdgcn_readlane(dsite, k64);
     const double u = __hiloint2double(__builtin_amdgcn_readlane(__double2hiint(du), k64),
                                       __builtin_amdgcn_readlane(__double2loint(du), k64));
-    bool acc;
-    if (!ok) {
-      __syncthreads();
-      if (tid == 0) s[site] = 1 - s[site];
-      __syncthreads();
-      const cd lp = slow_logpsi(g, o, P, s, slow, red);
-      acc = u < exp(a.mu * lp.re - a.mu * cur.re);
-      __syncthreads();
-      if (tid == 0 && !acc) s[site] = 1 - s[site];
-      __syncthreads();
-      if (acc) cur = lp;
-    } else {
-      const int iv = inv[rc * L + site], pos = iv >> 1, v = s[site] ^ (iv & 1);
-      T gq[HT], pr;
-      set_one(pr);
-      const int64_t at = (int64_t)(2 * pos + v) * H;
+    const int up = (__builtin_amdgcn_readlane((int)sp, site & 63) >> (site >> 6)) & 1;
+    const int iv = inv[rc * L + site], pos = iv >> 1, v = up ^ (iv & 1);
+    T en[HT], pr;  // e after the flip; (1 + e') / (1 + e) per unit
+    set_one(pr);
+    const int at = (2 * pos + v) * (TAB ? HP : H);
 #pragma unroll
-      for (int k = 0; k < HT; ++k) {
-        const int hc = min(h0 + k, H - 1);
-        gq[k] = tab_lds ? me[at + hc] : ((const T*)tab.me)[at + hc];
-        pr = mulc(pr, fmac(be[k], gq[k], al[k]));
-      }
-      for (int m = 1; m < SL; m *= 2) pr = mulc(pr, shfl_xor(pr, m));
-      const double* pq = tab.site + 8 * (int64_t)pos + 2 + 2 * v;
-      const cd z = mulc(mulc(to_cd(pr), cd{pq[0], pq[1]}), wt);
-      const double zr = wave_sum(mine && sl == 0 ? z.re : 0.0), zi = o.cpx ? wave_sum(mine && sl == 0 ? z.im : 0.0) : 0.0;
-      cd* slot = part + 16 * (step & 1);
-      if (lane == 0) slot[tid / WAVE] = {zr, zi};
-      __syncthreads();
-      cd S = slot[0];
-      for (int i = 1; i < nw; ++i) S = S + slot[i];
-      const double new2 = !o.cpx && S.re < 0.0 ? NAN : norm2(S);
-      // random.bernoulli(key, P), sampler.py:336-340
-      acc = a.mu == 2.0 ? u * cur2 < new2 : u < exp(a.mu * (0.5 * log(new2) - 0.5 * log(cur2)));
-      if (acc) {
+    for (int k = 0; k < HT; ++k) {
+      const int hc = min(h0 + k, H - 1);
+      if constexpr (TAB) en[k] = mulc(e[k], me[at + hc]);
+      else en[k] = mulc(e[k], ((const T*)tab.me)[at + hc]);
+      pr = mulc(pr, mulc(al[k], plus1(en[k])));
+    }
+    for (int m = 1; m < SL; m *= 2) pr = mulc(pr, shfl_xor(pr, m));
+    const cd z = mulc(to_cd(pr), mulc(pre[2 * pos + v], wt));
+    const double zr = wave_sum(mine && sl == 0 ? z.re : 0.0), zi = o.cpx ? wave_sum(mine && sl == 0 ? z.im : 0.0) : 0.0;
+    cd* slot = part + 16 * (step & 1);
+    if (lane == 0) slot[tid / WAVE] = {zr, zi};
+    __syncthreads();
+    cd S = slot[0];
+    for (int i = 1; i < nw; ++i) S = S + slot[i];
+    const double new2 = !o.cpx && S.re < 0.0 ? NAN : norm2(S);
+    // random.bernoulli(key, P), sampler.py:336-340
+    const bool acc = a.mu == 2.0 ? u * cur2 < new2 : u < exp(a.mu * (0.5 * log(new2) - 0.5 * log(cur2)));
+    if (acc) {
 #pragma unroll
-        for (int k = 0; k < HT; ++k)
-          if (h0 + k < H) {
-            e[k] = mulc(e[k], gq[k]);
-            al[k] = recip(plus1(e[k]));
-            be[k] = mulc(e[k], al[k]);
-          }
-        const double sc = new2 > 0.0 ? 1.0 / sqrt(new2) : 1.0;
-        wt = {z.re * sc, z.im * sc};
-        cur2 = new2 > 0.0 ? 1.0 : 0.0;
-        if (tid == 0) s[site] ^= 1;
+      for (int k = 0; k < HT; ++k) {  // units beyond H: e = 0 stays 0
+        e[k] = en[k];
+        al[k] = recip(plus1(en[k]));
       }
-      // the flip is seen by the other waves after the next barrier; a proposal
-      // at the same site right after needs it now
-      __syncthreads();
+      const double sc = new2 > 0.0 ? 1.0 / sqrt(new2) : 1.0;
+      wt = {z.re * sc, z.im * sc};
+      cur2 = new2 > 0.0 ? 1.0 : 0.0;
+      if (lane == (site & 63)) sp ^= 1u << (site >> 6);
     }
     nacc += acc;
     ++since;
@@ -604,6 +589,7 @@ __global__ void __launch_bounds__(MAXT) sym_rbm_mc(RbmGeom g, SymGeom o, const d
       left = a.sweep_steps;
       int32_t* out = configs + row_out * L;
       row_out += a.num_chains;
+      spins_out();
       for (int i = tid; i < L; i += nt) out[i] = s[i];
       if (since >= RBMQ_MC_REFRESH) {
         refresh();
@@ -611,6 +597,7 @@ __global__ void __launch_bounds__(MAXT) sym_rbm_mc(RbmGeom g, SymGeom o, const d
       }
     }
   }
+  spins_out();
   for (int i = tid; i < L; i += nt) walkers[(int64_t)chain * L + i] = s[i];
   if (tid == 0) {
     atomicAdd((unsigned long long*)&counters[0], (unsigned long long)total);
@@ -618,9 +605,108 @@ __global__ void __launch_bounds__(MAXT) sym_rbm_mc(RbmGeom g, SymGeom o, const d
   }
 }
 size_t sym_mc_lds(const RbmGeom& g, int G, bool tabl) {
-  return 8 * 16 + 16 * 32 + 16 * (size_t)G + (tabl ? 8 * (size_t)rbm_cw(g) * 2 * g.L * g.H : 0) + 4 * (size_t)g.L +
+  return 8 * 16 + 16 * 32 + 32 * (size_t)g.L + (tabl ? 8 * (size_t)rbm_cw(g) * 2 * g.L * (g.H | 1) : 0) + 4 * (size_t)g.L +
          3 * (size_t)G * g.L + 16;
 }
+
+// ------------------------------------------------------------------ parameters out of range
+// Row by row with rbm.hpp's log-cosh, one configuration or chain per
+// workgroup; these kernels return at once where the resident ones above work
+// (and the other way round), so neither carries the other's registers.
+__global__ void __launch_bounds__(SYM_T) sym_slow_forward(RbmGeom g, SymGeom o, const double* __restrict__ P,
+                                                          RbmTab tab, const int32_t* __restrict__ cfg, int64_t n,
+                                                          double* __restrict__ out) {
+  extern __shared__ double lds[];
+  if (rbmq_ok(g, tab, 2, threadIdx.x % WAVE)) return;
+  cd* c = (cd*)(lds + 8);
+  int32_t* s = (int32_t*)(c + o.G);
+  for (int64_t q = blockIdx.x; q < n; q += gridDim.x) {
+    __syncthreads();
+    for (int i = threadIdx.x; i < g.L; i += SYM_T) s[i] = cfg[q * g.L + i];
+    __syncthreads();
+    const cd lp = slow_logpsi(g, o, P, s, c, lds);
+    if (threadIdx.x == 0) {
+      out[2 * q] = lp.re;
+      out[2 * q + 1] = lp.im;
+    }
+  }
+}
+
+__global__ void __launch_bounds__(SYM_T) sym_slow_eloc(RbmGeom g, SymGeom o, const double* __restrict__ P, OpDev op,
+                                                       RbmTab tab, const int32_t* __restrict__ cfg,
+                                                       const double* __restrict__ lps, int64_t n,
+                                                       double* __restrict__ out) {
+  extern __shared__ double lds[];
+  if (rbmq_ok(g, tab, 2, threadIdx.x % WAVE)) return;
+  cd* c = (cd*)(lds + 8);
+  int32_t* s = (int32_t*)(c + o.G);
+  for (int64_t q = blockIdx.x; q < n; q += gridDim.x) {
+    __syncthreads();
+    for (int i = threadIdx.x; i < g.L; i += SYM_T) s[i] = cfg[q * g.L + i];
+    __syncthreads();
+    cd acc = {0.0, 0.0};
+    const int32_t* cq = cfg + q * g.L;
+    const cd dsum = diag_sum(op, cq);
+    for (int j = 0; j < op.num_ops; ++j) {
+      int sites[MAXLEN], vals[MAXLEN], nch;
+      const cd m = merged_m(op, j, apply_string(op, j, cq, sites, vals, nch), dsum);
+      if (!nonzero(m)) continue;
+      __syncthreads();
+      if (threadIdx.x == 0)
+        for (int k = 0; k < nch; ++k) s[sites[k]] = 1 - s[sites[k]];
+      __syncthreads();
+      acc = acc + m * cexp(slow_logpsi(g, o, P, s, c, lds) - cd{lps[2 * q], lps[2 * q + 1]});
+      __syncthreads();
+      if (threadIdx.x == 0)
+        for (int k = 0; k < nch; ++k) s[sites[k]] = 1 - s[sites[k]];
+      __syncthreads();
+    }
+    if (threadIdx.x == 0) {
+      out[2 * q] = acc.re;
+      out[2 * q + 1] = acc.im;
+    }
+  }
+}
+
+__global__ void __launch_bounds__(SYM_T) sym_slow_mc(RbmGeom g, SymGeom o, const double* __restrict__ P, jv_mc_args a,
+                                                     RbmTab tab, int32_t* __restrict__ walkers,
+                                                     int32_t* __restrict__ configs, int64_t* __restrict__ counters) {
+  extern __shared__ double lds[];
+  if (rbmq_ok(g, tab, 2, threadIdx.x % WAVE)) return;
+  const int tid = threadIdx.x, chain = blockIdx.x;
+  cd* c = (cd*)(lds + 8);
+  int32_t* s = (int32_t*)(c + o.G);
+  for (int i = tid; i < g.L; i += SYM_T) s[i] = walkers[(int64_t)chain * g.L + i];
+  __syncthreads();
+  double lacc = a.mu * slow_logpsi(g, o, P, s, c, lds).re;
+  const int total = a.therm_steps + a.samples_per_chain * a.sweep_steps;
+  int64_t nacc = 0;
+  for (int step = 0; step < total; ++step) {
+    int site;
+    double u;
+    mc_draw(a.seed, (uint32_t)step, (uint32_t)chain, a.call_index, a.stream, g.L, site, u);
+    __syncthreads();
+    if (tid == 0) s[site] ^= 1;
+    __syncthreads();
+    const double lnew = a.mu * slow_logpsi(g, o, P, s, c, lds).re;
+    const bool acc = u < exp(lnew - lacc);
+    __syncthreads();
+    if (tid == 0 && !acc) s[site] ^= 1;
+    __syncthreads();
+    if (acc) lacc = lnew;
+    nacc += acc;
+    const int k = step + 1 - a.therm_steps;
+    if (k > 0 && k % a.sweep_steps == 0)
+      for (int i = tid; i < g.L; i += SYM_T)
+        configs[((int64_t)(k / a.sweep_steps - 1) * a.num_chains + chain) * g.L + i] = s[i];
+  }
+  for (int i = tid; i < g.L; i += SYM_T) walkers[(int64_t)chain * g.L + i] = s[i];
+  if (tid == 0) {
+    atomicAdd((unsigned long long*)&counters[0], (unsigned long long)total);
+    atomicAdd((unsigned long long*)&counters[1], (unsigned long long)nacc);
+  }
+}
+size_t sym_slow_lds(const RbmGeom& g, int G) { return 64 + 16 * (size_t)G + 4 * (size_t)g.L; }
 
 __global__ void sym_zero_counters(int64_t* c) {
   if (threadIdx.x < 2) c[threadIdx.x] = 0;
@@ -655,6 +741,10 @@ int sym_rbm_forward_launch(const jv_net* net, const double* params, const jv_orb
   hipLaunchKernelGGL(fn, dim3((unsigned)std::min<int64_t>(n, 1 << 20)), dim3(SYM_T), lds, st, g, o, params, tab, configs,
                      n, logpsi);
   JV_LAUNCH_CHECK("sym_rbm_forward");
+  if ((rc = set_lds_limit((const void*)sym_slow_forward, sym_slow_lds(g, o.G)))) return rc;
+  hipLaunchKernelGGL(sym_slow_forward, dim3((unsigned)std::min<int64_t>(n, 512)), dim3(SYM_T), sym_slow_lds(g, o.G), st,
+                     g, o, params, tab, configs, n, logpsi);
+  JV_LAUNCH_CHECK("sym_slow_forward");
   *done = true;
   return JV_OK;
 }
@@ -668,23 +758,21 @@ int sym_rbm_eloc_launch(const jv_net* net, const double* params, const jv_orbit*
   if (!sym_rbm_geom(net, orbit, g, o) || op->max_len > 2 || op->fermi || !prefactor) return JV_OK;
   const OpDev d = make_opdev(op, prefactor, net->num_sites);
   const int nstr = rbmq_strings(d);
-  // the most rows at once, with the table in LDS where two workgroups still
-  // share a CU (or where it fits at all beside the rows)
+  // two workgroups per CU, with the table in LDS if that leaves room for rows,
+  // then as many rows as fit; else whatever fits one
   int RC = 0;
   bool tabl = false;
   size_t lds = 0;
-  for (int rows : {64, 32, 16}) {
-    if (RC) break;
-    for (bool t : {true, false}) {
-      const size_t b = sym_eloc_lds(g, o.G, rows, t, nstr);
-      if (b <= (size_t)(t ? 80 : 160) * 1024 || (t && rows == 64 && b <= 160 * 1024)) {
-        RC = rows;
-        tabl = t;
-        lds = b;
-        break;
-      }
+  for (int pass = 0; pass < 4 && !RC; ++pass)
+    for (int rows : {64, 32, 16}) {
+      const bool t = pass == 0 || pass == 2;
+      const size_t b = sym_eloc_lds(g, rows, t, nstr);
+      if (b > (size_t)(pass < 2 ? 80 : 160) * 1024) continue;
+      RC = rows;
+      tabl = t;
+      lds = b;
+      break;
     }
-  }
   if (!RC) return JV_OK;
   RbmTab tab;
   int rc = build_rbm_tables(g, params, &d, false, true, st, slot0, &tab);
@@ -699,6 +787,10 @@ int sym_rbm_eloc_launch(const jv_net* net, const double* params, const jv_orbit*
   hipLaunchKernelGGL(fn, dim3((unsigned)std::min<int64_t>(n, 4096)), dim3(SYM_T), lds, st, g, o, params, d, tab, configs,
                      lps, n, nstr, out);
   JV_LAUNCH_CHECK("sym_rbm_eloc");
+  if ((rc = set_lds_limit((const void*)sym_slow_eloc, sym_slow_lds(g, o.G)))) return rc;
+  hipLaunchKernelGGL(sym_slow_eloc, dim3((unsigned)std::min<int64_t>(n, 512)), dim3(SYM_T), sym_slow_lds(g, o.G), st, g,
+                     o, params, d, tab, configs, lps, n, out);
+  JV_LAUNCH_CHECK("sym_slow_eloc");
   *done = true;
   return JV_OK;
 }
@@ -708,7 +800,7 @@ int sym_rbm_mc_launch(const jv_net* net, const double* params, const jv_orbit* o
   *done = false;
   RbmGeom g;
   SymGeom o;
-  if (!sym_rbm_geom(net, orbit, g, o) || g.H > RBMQ_MC_MAX_H) return JV_OK;
+  if (!sym_rbm_geom(net, orbit, g, o) || !rbmq_mc_fits(g)) return JV_OK;
   // hidden units per thread: as many as leave the fewest threads (a power of
   // two of them per row, inside one wave), with registers for 512 threads of
   // eight units or 1024 of four
@@ -729,16 +821,22 @@ int sym_rbm_mc_launch(const jv_net* net, const double* params, const jv_orbit* o
   int rc = build_rbm_tables(g, params, nullptr, true, false, st, slot0, &tab);
   if (rc) return rc;
   const int T = (o.G * SL + WAVE - 1) / WAVE * WAVE;
-  const auto fn = HT == 8 ? (T <= 256 ? (g.cpx ? sym_rbm_mc<true, 8, 256> : sym_rbm_mc<false, 8, 256>)
-                                      : (g.cpx ? sym_rbm_mc<true, 8, 512> : sym_rbm_mc<false, 8, 512>))
-                          : (g.cpx ? sym_rbm_mc<true, 4, 1024> : sym_rbm_mc<false, 4, 1024>);
+#define JV_SYM_MC(HTv, Tv)                                                                                \
+  (g.cpx ? (tabl ? sym_rbm_mc<true, HTv, Tv, true> : sym_rbm_mc<true, HTv, Tv, false>)                    \
+         : (tabl ? sym_rbm_mc<false, HTv, Tv, true> : sym_rbm_mc<false, HTv, Tv, false>))
+  const auto fn = HT == 8 ? (T <= 256 ? JV_SYM_MC(8, 256) : JV_SYM_MC(8, 512)) : JV_SYM_MC(4, 1024);
+#undef JV_SYM_MC
   rc = set_lds_limit((const void*)fn, lds);
   if (rc) return rc;
   hipLaunchKernelGGL(sym_zero_counters, dim3(1), dim3(64), 0, st, counters);
   JV_LAUNCH_CHECK("sym_zero_counters");
-  hipLaunchKernelGGL(fn, dim3((unsigned)a.num_chains), dim3(T), lds, st, g, o, params, a, tab, SL, (int)tabl, walkers,
+  hipLaunchKernelGGL(fn, dim3((unsigned)a.num_chains), dim3(T), lds, st, g, o, params, a, tab, SL, walkers,
                      configs, counters);
   JV_LAUNCH_CHECK("sym_rbm_mc");
+  if ((rc = set_lds_limit((const void*)sym_slow_mc, sym_slow_lds(g, o.G)))) return rc;
+  hipLaunchKernelGGL(sym_slow_mc, dim3((unsigned)a.num_chains), dim3(SYM_T), sym_slow_lds(g, o.G), st, g, o, params, a,
+                     tab, walkers, configs, counters);
+  JV_LAUNCH_CHECK("sym_slow_mc");
   *done = true;
   return JV_OK;
 }
