@@ -758,6 +758,7 @@ int trd_eig_solve(double* S, int n, double* ev, double* c, double* Zbuf, double*
 }
 
 size_t trd_work_doubles(int n);
+int herm_apply_q(const double* S, const double* tau, int n, double* X, hipStream_t st);
 
 // Full eigendecomposition of the real symmetric S (row-major, destroyed):
 // ev ascending, S overwritten with the eigenvectors as rows (the same
@@ -785,7 +786,8 @@ int trd_eigh_full(double* S, int n, double* ev, hipStream_t st) {
 // Full eigendecomposition of the complex Hermitian S (row-major, destroyed):
 // ev ascending, row k of S <- conj(v_k) (the convention of the rocSOLVER path,
 // which decomposes the column-major view conj(S)).  Householder reduction to a
-// real tridiagonal T (trd_step_c), rocSOLVER dstedc for T, zunmtr for Q Z.
+// real tridiagonal T (trd_step_c), divide and conquer for T, Q Z on the matrix
+// cores (herm_apply_q).
 int trdc_eigh_full(double* S, int n, double* ev, hipStream_t st) {
   const int G = trd_groups(n);
   const size_t wd = 13 * (size_t)n + 2 * (size_t)G + 64;
@@ -823,17 +825,13 @@ int trdc_eigh_full(double* S, int n, double* ev, hipStream_t st) {
   }
   int rc = stedc(n, ev, a.e, Z, (rocblas_int*)(work + 13 * (size_t)n + 2 * G + 8), st);
   if (rc) return rc;
-  rocblas_handle h = blas_handle(st);
-  if (!h) return fail(JV_E_SOLVER, "rocblas_create_handle failed");
   const int64_t nn = (int64_t)n * n;
   hipLaunchKernelGGL(trdc_expand, dim3((unsigned)((nn + 255) / 256)), dim3(256), 0, st, Z, nn, Zc);
   JV_LAUNCH_CHECK("trdc_expand");
   {
     ScopedTimer tm("ormtr", st);
-    rocblas_status s = rocsolver_zunmtr(h, rocblas_side_left, rocblas_fill_lower, rocblas_operation_none, n, n,
-                                        (rocblas_double_complex*)S, n, (rocblas_double_complex*)a.tau,
-                                        (rocblas_double_complex*)Zc, n);
-    if (s != rocblas_status_success) return fail(JV_E_SOLVER, "rocsolver_zunmtr status " + std::to_string((int)s));
+    rc = herm_apply_q(S, a.tau, n, Zc, st);
+    if (rc) return rc;
   }
   hipLaunchKernelGGL(trdc_conj, dim3((unsigned)((nn + 255) / 256)), dim3(256), 0, st, Zc, nn, S);
   JV_LAUNCH_CHECK("trdc_conj");

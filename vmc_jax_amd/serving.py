@@ -403,7 +403,8 @@ def footprint_bytes(num_samples, num_real_params, num_sites, complex_params, sol
     route: the Gram's split-sample partial tiles, the shifted copy, the second
     factor and the inverse of the Cholesky route, the eigenvectors, the
     explicit Q and its product, the divide-and-conquer buffers, the complex
-    tridiagonal path's buffers and, where the library's eigendecomposition
+    tridiagonal path's buffers (with the slices of its blocked back
+    transformation) and, where the library's eigendecomposition
     runs, its workspace, plus the solver library handle of the job's thread
     (rocBLAS / rocSOLVER keep ~134 MB of device memory per handle; counted
     for every route, since a real solve needs the library once its spectrum
@@ -418,6 +419,7 @@ def footprint_bytes(num_samples, num_real_params, num_sites, complex_params, sol
         b += n * pr * 16 * 4                              # O (flat layout) and centred O, SNR data Q and R
         b += n * pc * 16 * 2                              # holomorphic G and the SNR projection M
         b += pr * pr * 8 * 5                              # S0 (complex), Z, S
+        b += _q_apply_bytes(pc)
         b += pc * pc * 8 * 10                             # A, eigenvectors, tridiagonal Z and Zc, D&C buffers
         b += pr * pr * 16 * 3                             # library eigendecomposition workspace
         b += _gram_slice_bytes(n, 2 * pr)
@@ -425,6 +427,8 @@ def footprint_bytes(num_samples, num_real_params, num_sites, complex_params, sol
             b += _bf16_gram_bytes(n, 2 * pc)
     elif solver == "minsr":
         b += n * pc * esz * 2                             # O and centred O
+        if complex_params:
+            b += _q_apply_bytes(min(n, pc))
         b += (n // 64 + 1) * pc * esz                     # O^T e partial sums (64-sample chunks)
         if n > pc:                                        # dual form
             m = pc
@@ -443,6 +447,14 @@ def footprint_bytes(num_samples, num_real_params, num_sites, complex_params, sol
         raise ValueError("solver must be 'tdvp' or 'minsr'")
     b += LIBRARY_HANDLE_BYTES
     return int(1.25 * b) + (64 << 20)
+
+
+def _q_apply_bytes(m):
+    """Slices of W, U and the T factors of the complex back transformation
+    (csrc/qapply.hip) for an m x m matrix."""
+    tiles = (m + 63) // 64
+    splits = max(1, min((384 + tiles - 1) // tiles, tiles))
+    return splits * tiles * 64 * 128 * 8 + m * 128 * 8 + tiles * 64 * 64 * 16
 
 
 # device memory a thread's solver library handle holds (measured: 134 MB)
