@@ -414,9 +414,22 @@ int gram_pp_f64(const double* D, int64_t n, int64_t p, int cpx, double* S, hipSt
   if (side > 4096) return fail(JV_E_ARG, "gram_pp_f64: matrix too large");
   const int nts = (int)side;
   const int64_t ntiles = side * (side + 1) / 2;
+  // Slices of the sample axis, by rounds: the chip holds 512 workgroups (two
+  // per CU), so `s` slices take ceil(ntiles s / 512) rounds of nkb / s stages
+  // plus about two stages' worth of writing and reducing a partial tile.  One
+  // slice leaves the second round of the L = 32 complex RBM's 561 tiles nearly
+  // empty (16384 x 2112 complex: 8.7 ms, 5.05 with the slices this picks);
+  // sixteen leave a 1240-column Gram's second round (880 workgroups) a quarter
+  // empty (0.310 ms; nine, one round of 495, 0.260).
   const int64_t nkb = (n + G6K - 1) / G6K;
-  int64_t splits = 1;
-  while (ntiles * splits < 512 && nkb / (splits * 2) >= 16) splits *= 2;
+  int64_t splits = 1, best = INT64_MAX;
+  for (int64_t s = 1; s <= 64 && s * 8 <= std::max<int64_t>(nkb, 8) && (s == 1 || ntiles * s <= 8192); ++s) {
+    const int64_t cost = (ntiles * s + 511) / 512 * ((nkb + s - 1) / s + 2);
+    if (cost < best) {
+      best = cost;
+      splits = s;
+    }
+  }
   const int64_t kchunk = (nkb + splits - 1) / splits * G6K;
   splits = (n + kchunk - 1) / kchunk;
   double* part = (double*)workspace(sizeof(double) * (size_t)splits * ntiles * GT * GT, slot);

@@ -360,13 +360,17 @@ def _cdiv(a, b):
 
 def _gram_slice_bytes(n, q):
     """Partial tiles of the FP64 Gram of an n x q real matrix: 128 x 128 upper
-    tiles, the sample axis cut into slices of whole 32-sample stages while the
-    tiles number fewer than 512 and each slice keeps >= 16 stages (the rule of
-    gram_pp_f64 in csrc/gram_mixed.hip)."""
+    tiles, the sample axis cut into the slices of whole 32-sample stages that
+    gram_pp_f64 in csrc/gram_mixed.hip picks (fewest rounds of 512 workgroups)."""
     side = _cdiv(q, 128)
-    ntiles, nkb, splits = side * (side + 1) // 2, _cdiv(n, 32), 1
-    while ntiles * splits < 512 and nkb // (splits * 2) >= 16:
-        splits *= 2
+    ntiles, nkb = side * (side + 1) // 2, _cdiv(n, 32)
+    splits, best = 1, None
+    for s in range(1, 65):
+        if s > 1 and (s * 8 > nkb or ntiles * s > 8192):
+            break
+        cost = _cdiv(ntiles * s, 512) * (_cdiv(nkb, s) + 2)
+        if best is None or cost < best:
+            splits, best = s, cost
     splits = _cdiv(n, _cdiv(nkb, splits) * 32)
     return splits * ntiles * 128 * 128 * 8
 
