@@ -208,7 +208,8 @@ __global__ void __launch_bounds__(256) cnn_fwd_grad_p(CnnGeom g, const T* __rest
   T* A = x0 + nn;                          // A + l * CM * n: planes [c][p]
   T* D = A + (size_t)g.nl * CM * nn;       // D + l * n * CM: [p][c]
   T* part = D + (size_t)g.nl * CM * nn;    // [nt][CM]
-  short* nbr = (short*)(part + (size_t)cnn_p_items(g, CM, nt) * CM);
+  // log psi alone keeps neither deltas nor partial sums (cnn_p_lds_fwd)
+  short* nbr = (short*)(want_grad ? part + (size_t)cnn_p_items(g, CM, nt) * CM : D);
   short* inv = nbr + nn * g.FF;
   const cst_t<T>* Wp = (const cst_t<T>*)Wpk;
   cnn_build_tables(g, nbr, inv, tid, nt);
@@ -423,11 +424,14 @@ int cnn_p_launch(const CnnGeom& g, const double* params, const int32_t* configs,
   const T* wpk = pack_cnn_weights<T>(g, pk, params, st, slot);
   if (!wpk) return JV_E_NOMEM;
   int rc = JV_OK;
+  // log psi alone takes a third of the LDS, so three times the workgroups
+  // share a CU
+  const size_t need = grad ? lds : cnn_p_lds_fwd(g, cm, (int)sizeof(T));
 #define JV_CNNP(CMv)                                                                                      \
   if (cm == CMv) {                                                                                        \
-    rc = set_lds_limit((const void*)cnn_fwd_grad_p<CMv, T>, lds);                                         \
+    rc = set_lds_limit((const void*)cnn_fwd_grad_p<CMv, T>, need);                                         \
     if (rc) return rc;                                                                                    \
-    hipLaunchKernelGGL((cnn_fwd_grad_p<CMv, T>), dim3((unsigned)blocks), dim3(256), lds, st, g, wpk, pk,   \
+    hipLaunchKernelGGL((cnn_fwd_grad_p<CMv, T>), dim3((unsigned)blocks), dim3(256), need, st, g, wpk, pk,   \
                        configs, n, layout, grad, logpsi);                                                 \
     JV_LAUNCH_CHECK("cnn_fwd_grad_p");                                                                    \
     *done = true;                                                                                         \

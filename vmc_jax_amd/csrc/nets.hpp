@@ -276,6 +276,10 @@ __host__ __device__ inline size_t cnn_p_lds(const CnnGeom& g, int cm, int nt, in
   const size_t t = (size_t)g.n + 2 * (size_t)g.nl * cm * g.n + (size_t)cnn_p_items(g, cm, nt) * cm;
   return 8 * 8 + (size_t)tsize * t + 2 * 2 * (size_t)g.n * g.FF;
 }
+// The same without gradients: no deltas, no partial sums.
+__host__ __device__ inline size_t cnn_p_lds_fwd(const CnnGeom& g, int cm, int tsize) {
+  return 8 * 8 + (size_t)tsize * ((size_t)g.n + (size_t)g.nl * cm * g.n) + 2 * 2 * (size_t)g.n * g.FF;
+}
 
 __device__ __host__ inline int win_ex(const CnnGeom& g, int l) { return l < 0 ? 1 : 1 + (l + 1) * (g.Fx - 1); }
 __device__ __host__ inline int win_ey(const CnnGeom& g, int l) { return l < 0 ? 1 : 1 + (l + 1) * (g.Fy - 1); }
