@@ -228,3 +228,36 @@ def test_sym_resident(cpx, L, H, names, op, big):
         assert np.array_equal(to_np(ms.sample()[0])[0], so)
     assert np.array_equal(to_np(ms.states), mo.states)
     assert float(ms.acceptance_ratio()[0]) == float(np.ravel(mo.acceptance_ratio())[0])
+
+
+def test_eloc_in_a_captured_graph():
+    """A captured call keeps no pointer into the tables' scratch memory: calls
+    with other sizes between the replays do not change its results."""
+    L, H, n = 9, 14, 50
+    rng = np.random.default_rng(8)
+    Hd, Ho = xxz_pair(L, 0.6)
+    P = 0.1 * rng.normal(size=_num(True, L, H, True, False))
+    psi, opsi = _states(True, L, H, True, False, P)
+    s = rng.integers(0, 2, size=(n, L)).astype(np.int32)
+    sd = torch.as_tensor(s[None], device="cuda")
+    lp = psi(sd)
+    eager = Hd.get_O_loc(sd, psi, lp).clone()
+    stream = torch.cuda.Stream()
+    stream.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(stream):
+        Hd.get_O_loc(sd, psi, lp)
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph, stream=stream):
+        out = Hd.get_O_loc(sd, psi, lp)
+    big, _ = _states(True, 40, 90, True, False, 0.05 * rng.normal(size=_num(True, 40, 90, True, False)))
+    Hb, _ = tfim_pair((40,), -1.0, -0.7)
+    sb = torch.as_tensor(rng.integers(0, 2, size=(1, 30, 40)).astype(np.int32), device="cuda")
+    for _ in range(3):
+        with torch.cuda.stream(stream):
+            Hb.get_O_loc(sb, big, big(sb))
+        torch.cuda.synchronize()
+        out.zero_()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert _rel(to_np(out), to_np(eager)) < TOL
