@@ -1159,21 +1159,25 @@ __global__ void tdvp_project_S(const double* __restrict__ S0, int64_t pr, int im
 
 // Per-sample SNR data Q[n][k] = makeReal(-x conj(D[n][k]) e_n / w_n)
 // (stats.py:255-265 covar_data followed by transform, tdvp.py:175-178).
+// -x conj(D_t) e / w: the part of one sample's force the solve mode keeps.
+__device__ inline double tdvp_snr_q(const double* __restrict__ D, int64_t t, double er, double ei, double inv, double xr,
+                                    double xi, int imag) {
+  double dr = D[2 * t], di = -D[2 * t + 1];  // conj(D)
+  double pr_ = dr * er - di * ei, pi_ = dr * ei + di * er;
+  pr_ *= inv;
+  pi_ *= inv;
+  return imag ? -(xr * pi_ + xi * pr_) : -(xr * pr_ - xi * pi_);
+}
+
 __global__ void tdvp_snr_data(const double* __restrict__ D, const double* __restrict__ e,
                               const double* __restrict__ w, int64_t n, int64_t pr, double xr, double xi, int imag,
                               double* __restrict__ Q) {
   int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (t >= n * pr) return;
   int64_t r = t / pr;
-  double dr = D[2 * t], di = -D[2 * t + 1];  // conj(D)
-  double er = e[2 * r], ei = e[2 * r + 1];
-  double pr_ = dr * er - di * ei, pi_ = dr * ei + di * er;
-  double inv = 1.0 / w[r];
-  pr_ *= inv;
-  pi_ *= inv;
-  double qr = -(xr * pr_ - xi * pi_), qi = -(xr * pi_ + xi * pr_);
-  if (imag) { Q[2 * t] = 0.0; Q[2 * t + 1] = qi; }
-  else Q[t] = qr;
+  const double q = tdvp_snr_q(D, t, e[2 * r], e[2 * r + 1], 1.0 / w[r], xr, xi, imag);
+  if (imag) { Q[2 * t] = 0.0; Q[2 * t + 1] = q; }
+  else Q[t] = q;
 }
 
 __global__ void tdvp_snr(const double* __restrict__ VtF, const double* __restrict__ var, int64_t pr, int cpx,
@@ -1347,35 +1351,27 @@ __global__ void holo_eig(const double* __restrict__ R, const double* __restrict_
 // eigenvectors is, per pair k:
 //   'imag': column pc+k = i M / sqrt2, column pc-1-k = i conj(M) / sqrt2;
 //   'real': column 2k = Re M, column 2k+1 = Im M.
-__global__ void holo_qc(const double* __restrict__ Q, int64_t n, int64_t pr, const int64_t* __restrict__ col_g,
-                        const int64_t* __restrict__ col_ig, int64_t pc, int imag, double* __restrict__ Qc) {
-  const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (t >= n * pc) return;
-  const int64_t r = t / pc, c = t - r * pc;
-  const int64_t a = r * pr + col_g[c], b = r * pr + col_ig[c];
-  Qc[2 * t] = imag ? Q[2 * a + 1] : Q[a];
-  Qc[2 * t + 1] = imag ? Q[2 * b + 1] : Q[b];
+// One thread per column, rows over the grid's second dimension.
+__global__ void __launch_bounds__(256) holo_qc(const double* __restrict__ D, const double* __restrict__ e,
+                                               const double* __restrict__ w, int64_t n, int64_t pr,
+                                               const int64_t* __restrict__ col_g, const int64_t* __restrict__ col_ig,
+                                               int64_t pc, double xr, double xi, int imag, double* __restrict__ Qc) {
+  const int64_t c = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (c >= pc) return;
+  const int64_t a = col_g[c], b = col_ig[c];
+  for (int64_t r = blockIdx.y; r < n; r += gridDim.y) {
+    const double er = e[2 * r], ei = e[2 * r + 1], inv = 1.0 / w[r];
+    Qc[2 * (r * pc + c)] = tdvp_snr_q(D, r * pr + a, er, ei, inv, xr, xi, imag);
+    Qc[2 * (r * pc + c) + 1] = tdvp_snr_q(D, r * pr + b, er, ei, inv, xr, xi, imag);
+  }
 }
 
-__global__ void holo_snr_scatter(const double* __restrict__ M, int64_t n, int64_t pc, int imag,
-                                 double* __restrict__ R) {
-  const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (t >= n * pc) return;
-  const int64_t r = t / pc, k = t - r * pc;
-  const double mr = M[2 * t], mi = M[2 * t + 1];
-  const int64_t pr = 2 * pc;
-  if (imag) {
-    const double h = 0.70710678118654752440;
-    double* p = R + 2 * (r * pr + pc + k);  // i M / sqrt2
-    p[0] = -h * mi;
-    p[1] = h * mr;
-    p = R + 2 * (r * pr + pc - 1 - k);      // i conj(M) / sqrt2
-    p[0] = h * mi;
-    p[1] = h * mr;
-  } else {
-    R[r * pr + 2 * k] = mr;
-    R[r * pr + 2 * k + 1] = mi;
-  }
+// 'imag': the projections on the two eigenvectors of a pair are i M / sqrt2
+// (column pc + k) and i conj(M) / sqrt2 (column pc - 1 - k): half M's variance each.
+__global__ void holo_var(const double* __restrict__ vm, int64_t pc, double* __restrict__ var) {
+  const int64_t k = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (k >= pc) return;
+  var[pc + k] = var[pc - 1 - k] = 0.5 * vm[k];
 }
 
 __global__ void sum_vec(const double* __restrict__ v, int64_t n, double* __restrict__ out) {
@@ -1437,8 +1433,8 @@ static int tdvp_solve_impl(const double* D, const double* e, const double* w, in
   double* raw = (double*)workspace(sizeof(double) * 2 * pr, 22);
   double* F0 = (double*)workspace(sizeof(double) * 2 * pr, 23);
   double* VtF = (double*)workspace(sizeof(double) * 2 * pr, 24);
-  double* Q = (double*)workspace(sizeof(double) * (imag ? 2 : 1) * (size_t)n * pr, 25);
-  double* R = (double*)workspace(sizeof(double) * (imag ? 2 : 1) * (size_t)n * pr, 26);
+  double* Q = holo ? nullptr : (double*)workspace(sizeof(double) * (imag ? 2 : 1) * (size_t)n * pr, 25);
+  double* R = holo ? nullptr : (double*)workspace(sizeof(double) * (imag ? 2 : 1) * (size_t)n * pr, 26);
   double* mean = (double*)workspace(sizeof(double) * 2 * pr, 27);
   double* var = (double*)workspace(sizeof(double) * pr, 28);
   double* scal = (double*)workspace(sizeof(double) * 8, 29);  // fnorm, evar, tdvp_error
@@ -1446,7 +1442,7 @@ static int tdvp_solve_impl(const double* D, const double* e, const double* w, in
   double* ucpx = (double*)workspace(sizeof(double) * 2 * pr, 31);
   double* S0u = (double*)workspace(sizeof(double) * 2 * pr, 32);
   double* Fr = (double*)workspace(sizeof(double) * pr, 33);
-  if (!S0 || !Z || !raw || !F0 || !VtF || !Q || !R || !mean || !var || !scal || !cvec || !ucpx || !S0u || !Fr)
+  if (!S0 || !Z || !raw || !F0 || !VtF || (!holo && (!Q || !R)) || !mean || !var || !scal || !cvec || !ucpx || !S0u || !Fr)
     return fail(JV_E_NOMEM, "jv_tdvp_solve: workspace allocation failed");
   const unsigned bp = (unsigned)((pr + 255) / 256);
   int rc;
@@ -1497,26 +1493,37 @@ static int tdvp_solve_impl(const double* D, const double* e, const double* w, in
     if ((rc = gemv(false, Z, Fr, pr, pr, 0, 0, 1.0, VtF, st, 34))) return rc;
   }
   // SNR (tdvp.py:173-181): rho = Q conj(V) = Q Z^T, weighted variance per column
-  hipLaunchKernelGGL(tdvp_snr_data, dim3((unsigned)((n * pr + 255) / 256)), dim3(256), 0, st, D, e, w, n, pr, xr,
-                     xi, imag, Q);
-  JV_LAUNCH_CHECK("tdvp_snr_data");
   if (holo) {
+    // straight from D to the pairs' coefficients and from their projection to
+    // the variances: the flat n x 2 Pc data and projections (1.1 GB each at
+    // 16384 x 4224) are neither written nor read
     double* Qc = (double*)workspace(sizeof(double) * 2 * (size_t)n * pc, 38);
     double* M = (double*)workspace(sizeof(double) * 2 * (size_t)n * pc, 45);
     if (!Qc || !M) return fail(JV_E_NOMEM, "jv_tdvp_solve: workspace allocation failed");
-    const unsigned nb = (unsigned)((n * pc + 255) / 256);
-    hipLaunchKernelGGL(holo_qc, dim3(nb), dim3(256), 0, st, Q, n, pr, col_g, col_ig, pc, imag, Qc);
+    hipLaunchKernelGGL(holo_qc, dim3((unsigned)((pc + 255) / 256), (unsigned)std::min<int64_t>(n, 4096)), dim3(256), 0,
+                       st, D, e, w, n, pr, col_g, col_ig, pc, xr, xi, imag, Qc);
     JV_LAUNCH_CHECK("holo_qc");
     GemmArgs g{n, pc, pc, Qc, pc, 1, 0, A, 1, pc, 0, M, pc, 1, 0, 1.0};
     if ((rc = gemm(g, st))) return rc;
-    hipLaunchKernelGGL(holo_snr_scatter, dim3(nb), dim3(256), 0, st, M, n, pc, imag, R);
-    JV_LAUNCH_CHECK("holo_snr_scatter");
+    if (imag) {
+      if ((rc = center(M, w, n, pc, 1, mean, M, st))) return rc;
+      if ((rc = col_norm2(M, n, pc, 1, cvec, st, 35))) return rc;
+      hipLaunchKernelGGL(holo_var, dim3((unsigned)((pc + 255) / 256)), dim3(256), 0, st, cvec, pc, var);
+      JV_LAUNCH_CHECK("holo_var");
+    } else {
+      // columns (2k, 2k + 1) of the real projection are M's (re, im): its own layout
+      if ((rc = center(M, w, n, pr, 0, mean, M, st))) return rc;
+      if ((rc = col_norm2(M, n, pr, 0, var, st, 35))) return rc;
+    }
   } else {
+    hipLaunchKernelGGL(tdvp_snr_data, dim3((unsigned)((n * pr + 255) / 256)), dim3(256), 0, st, D, e, w, n, pr, xr, xi,
+                       imag, Q);
+    JV_LAUNCH_CHECK("tdvp_snr_data");
     GemmArgs g{n, pr, pr, Q, pr, 1, 0, Z, 1, pr, 0, R, pr, imag, 0, 1.0};
     if ((rc = gemm(g, st))) return rc;
+    if ((rc = center(R, w, n, pr, imag, mean, R, st))) return rc;
+    if ((rc = col_norm2(R, n, pr, imag, var, st, 35))) return rc;
   }
-  if ((rc = center(R, w, n, pr, imag, mean, R, st))) return rc;
-  if ((rc = col_norm2(R, n, pr, imag, var, st, 35))) return rc;
   hipLaunchKernelGGL(tdvp_snr, dim3(bp), dim3(256), 0, st, VtF, var, pr, imag, glob_num_samples, snr);
   JV_LAUNCH_CHECK("tdvp_snr");
   // ||F||, Var E = sum |e|^2
