@@ -101,6 +101,23 @@ def test_eloc(cpx, L, H, bias, vbias, op, n):
     assert _rel(e, ref) < TOL
 
 
+@pytest.mark.parametrize("H,L,op", [(257, 6, "mixed"), (300, 48, "tfim"), (900, 17, "xxz")])
+def test_eloc_two_sample_tiles(H, L, op):
+    """More than 256 hidden units: two samples per workgroup of four waves, many
+    full tiles; every sample keeps its own amplitude."""
+    n = 301
+    rng = np.random.default_rng(H)
+    P = 0.3 / np.sqrt(L) * rng.normal(size=_num(True, L, H, True, False))
+    P[2 * H:] *= 0.3  # |Re theta| and the sites' summed |Re W| stay in range
+    psi, opsi = _states(True, L, H, True, False, P)
+    Hd, Ho = OPS[op](L)
+    s = rng.integers(0, 2, size=(n, L)).astype(np.int32)
+    sd = torch.as_tensor(s[None], device="cuda")
+    e = to_np(Hd.get_O_loc(sd, psi, psi(sd)))[0]
+    ref = Ho.get_O_loc(s, opsi, opsi(s))
+    assert np.max(np.abs(e - ref)) < TOL * np.max(np.abs(ref))
+
+
 @pytest.mark.parametrize("big", [10.0, 60.0])
 def test_eloc_out_of_range(big):
     """A site whose summed |Re W| (80, 480) or a unit whose |Re theta| leaves the

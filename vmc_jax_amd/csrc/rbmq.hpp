@@ -365,7 +365,11 @@ __device__ inline void rbmq_eloc_tile(const RbmGeom& g, const double* __restrict
   const double* Wr = P + g.ow;
   const double* Wi = Wr + (int64_t)L * H;
   cd acc[SPW];
-  {
+#pragma unroll
+  for (int k = 0; k < SPW; ++k) acc[k] = {0.0, 0.0};
+  // (S < RBMQ_WAVES: the waves without a sample skip this; the spins of another
+  // wave's sample are only ordered by the barrier of the first pass)
+  if (S >= RBMQ_WAVES || w < S) {
     double lin_re[SPW] = {}, lin_im[SPW] = {};
     T dprod[SPW];
 #pragma unroll
@@ -438,7 +442,6 @@ __device__ inline void rbmq_eloc_tile(const RbmGeom& g, const double* __restrict
       const cd x = {fma(-(double)H, LN2, wave_sum(vr)) - lps[2 * sc], wave_sum(vi) - lps[2 * sc + 1]};
       const cd a = mulc(to_cd(wave_prod(dprod[k])), cexp(x));
       if (lane == 0) amp[s] = a;
-      acc[k] = {0.0, 0.0};
       if (op.num_diag > 1) {
         cd ds = {0.0, 0.0};
         for (int d = lane; d < op.num_diag; d += WAVE) {
