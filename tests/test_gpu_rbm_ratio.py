@@ -118,6 +118,37 @@ def test_eloc_two_sample_tiles(H, L, op):
     assert np.max(np.abs(e - ref)) < TOL * np.max(np.abs(ref))
 
 
+def _late_pair(L, where):
+    """A transverse field with one string that flips no spin (two Sx on one
+    site) at position `where` of the list."""
+    from vmc_jax_amd import operator as dop
+    out = []
+    for o in (dop, oop):
+        H = o.BranchFreeOperator()
+        for k in range(2 * L):
+            if k == where:
+                H.add(o.scal_opstr(0.9, (o.Sx(1), o.Sx(1))))
+            H.add(o.scal_opstr(0.3 + 0.01 * k, (o.Sx(k % L),)))
+        out.append(H)
+    return out
+
+
+@pytest.mark.parametrize("L,H,n,where", [(2, 1, 9000, 0), (2, 1, 40, 3), (50, 5, 60, 0), (50, 5, 60, 63),
+                                         (50, 5, 60, 64), (50, 5, 60, 99)])
+def test_eloc_string_that_flips_nothing(L, H, n, where):
+    """The workgroup's flag for such strings, set in the first pass of 64 strings
+    or in a later one, with a theta phase too short to hide a late clear."""
+    rng = np.random.default_rng(where)
+    P = 0.3 * rng.normal(size=_num(True, L, H, True, False))
+    psi, opsi = _states(True, L, H, True, False, P)
+    Hd, Ho = _late_pair(L, where)
+    s = rng.integers(0, 2, size=(n, L)).astype(np.int32)
+    sd = torch.as_tensor(s[None], device="cuda")
+    e = to_np(Hd.get_O_loc(sd, psi, psi(sd)))[0]
+    ref = Ho.get_O_loc(s, opsi, opsi(s))
+    assert np.max(np.abs(e - ref) / np.abs(ref)) < TOL
+
+
 @pytest.mark.parametrize("big", [10.0, 60.0])
 def test_eloc_out_of_range(big):
     """A site whose summed |Re W| (80, 480) or a unit whose |Re theta| leaves the

@@ -360,15 +360,14 @@ __device__ inline void rbmq_eloc_tile(const RbmGeom& g, const double* __restrict
   for (int s = w; s < S; s += RBMQ_WAVES)
     for (int i = lane; i < L; i += WAVE) sp[s * L + i] = cfg[(int64_t)min(s, ns - 1) * L + i];
   if (threadIdx.x == 0) *odd = 0;
-  wave_sync();
+  __syncthreads();  // the clear comes before any wave's set in the first pass
   // hidden units of the wave's samples: lane = unit
   const double* Wr = P + g.ow;
   const double* Wi = Wr + (int64_t)L * H;
   cd acc[SPW];
 #pragma unroll
   for (int k = 0; k < SPW; ++k) acc[k] = {0.0, 0.0};
-  // (S < RBMQ_WAVES: the waves without a sample skip this; the spins of another
-  // wave's sample are only ordered by the barrier of the first pass)
+  // (S < RBMQ_WAVES: the waves without a sample skip this)
   if (S >= RBMQ_WAVES || w < S) {
     double lin_re[SPW] = {}, lin_im[SPW] = {};
     T dprod[SPW];
