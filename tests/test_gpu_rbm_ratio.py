@@ -167,6 +167,45 @@ def test_eloc_out_of_range(big):
     assert np.max(np.abs(e - ref) / np.abs(ref)) < TOL
 
 
+def _hop_pair(L):
+    """Hopping strings (they keep the number of up spins) and a diagonal one."""
+    from vmc_jax_amd import operator as dop
+    out = []
+    for o in (dop, oop):
+        H = o.BranchFreeOperator()
+        for i in range(L):
+            j = (i + 1) % L
+            H.add(o.scal_opstr(0.7, (o.Sp(i), o.Sm(j))))
+            H.add(o.scal_opstr(0.7, (o.Sm(i), o.Sp(j))))
+        H.add(o.scal_opstr(1.1, (o.Sz(1),)))
+        out.append(H)
+    return out
+
+
+@pytest.mark.parametrize("mu", [2.0, 0.0])
+def test_large_visible_bias(mu):
+    """|Re a| = 400 on every site: the factor of one flipped site over- or
+    underflows, that of a hop (and every log) does not; with mu = 0 every
+    proposal is accepted whatever the ratio."""
+    L, H = 6, 8
+    rng = np.random.default_rng(13)
+    P = 0.1 * rng.normal(size=_num(True, L, H, True, True))
+    P[-2 * L:-L] = 400.0  # Re a
+    psi, opsi = _states(True, L, H, True, True, P)
+    Hd, Ho = _hop_pair(L)
+    s = rng.integers(0, 2, size=(20, L)).astype(np.int32)
+    sd = torch.as_tensor(s[None], device="cuda")
+    e = to_np(Hd.get_O_loc(sd, psi, psi(sd)))[0]
+    ref = Ho.get_O_loc(s, opsi, opsi(s))
+    assert np.all(np.isfinite(ref))
+    # log psi is 2400 in size: its rounding error is the exponent's
+    assert np.max(np.abs(e - ref) / np.abs(ref)) < 1e-10
+    kw = dict(numChains=3, numSamples=9, thermalizationSweeps=2, sweepSteps=20, mu=mu)
+    ms = jv.sampler.MCSampler(psi, (L,), 17, updateProposer=jv.sampler.propose_spin_flip, **kw)
+    mo = osamp.MCSampler(opsi, (L,), 17, **kw)
+    assert np.array_equal(to_np(ms.sample()[0])[0], mo.sample()[0])
+
+
 def test_eloc_nan_parameters():
     L, H = 6, 8
     P = 0.1 * np.random.default_rng(4).normal(size=_num(True, L, H, True, False))

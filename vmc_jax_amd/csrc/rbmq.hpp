@@ -12,9 +12,9 @@
 // relative accuracy, so nothing cancels that does not cancel in cosh(theta').
 //
 // Range: the routines below are used when |Re theta_h| <= RBMQ_THETA for every
-// configuration and 4 n sum_h |Re W_ih| <= 600 for strings of n sites (the
-// products then stay inside the double range); rbm.hpp's log-cosh routines
-// serve everything else.  The kernels read the two bounds from the table, so
+// configuration and sum_h |Re W_ih| + |Re a_i| <= 150 / n for strings of n
+// sites (pre_j and the products over units then stay inside the double range);
+// rbm.hpp's log-cosh routines serve everything else.  The kernels read the two bounds from the table, so
 // no host synchronisation is needed and NaN parameters take the log route.
 #pragma once
 #include "rbm.hpp"
@@ -33,7 +33,7 @@ constexpr int RBMQ_MAX_H = 900;  // prod_h (1 + e_h) <= 2^H
 struct RbmTab {
   double* me;     // [L][2][H]: g of a flip, for the chains (null: not built)
   double* he;     // [H][L][2]: g of a flip, for the local energies (null: not built)
-  double* site;   // [L][8]: |pre|^2 for v = 0, 1; pre for v = 0 (re, im), v = 1; sum_h |Re W_ih|
+  double* site;   // [L][8]: |pre|^2 for v = 0, 1; pre for v = 0 (re, im), v = 1; sum_h |Re W_ih| + |Re a_i|
   double* row;    // [H]: |Re b_h| + sum_i |Re W_ih|
   int32_t* lead;  // [0]: count; then 16 * string + followers (strings behind it that flip the same sites)
   int32_t* mark;  // [num_ops]: 1 for merged diagonal strings
@@ -109,6 +109,7 @@ __device__ inline void rbm_tab_build(const RbmGeom& g, const double* __restrict_
       if (g.oa >= 0) {
         sr += P[g.oa + i];
         si += P[g.oa + g.L + i];
+        sa += fabs(P[g.oa + i]);
       }
       const double sg = tid ? 1.0 : -1.0;
       const cd pre = cexp({-2.0 * sg * sr, -2.0 * sg * si});
