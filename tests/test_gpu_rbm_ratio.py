@@ -317,6 +317,36 @@ def test_sym_resident(cpx, L, H, names, op, big):
     assert float(ms.acceptance_ratio()[0]) == float(np.ravel(mo.acceptance_ratio())[0])
 
 
+@pytest.mark.parametrize("cpx", [True, False])
+def test_sym_rows_that_are_no_permutation(cpx):
+    """An orbit element may read a site twice, or never: (g s)_i = s_{m_i} all
+    the same."""
+    from oracle import symmetries as osym
+    L, H, n = 6, 5, 30
+    maps = np.array([[0, 1, 2, 3, 4, 5], [0, 0, 2, 3, 4, 5], [1, 2, 2, 2, 0, 3], [5, 4, 3, 2, 1, 0]])
+    signs = np.array([[1] * 6, [1, 1, -1, 1, 1, -1], [1, -1, 1, 1, 1, -1], [-1] * 6])
+    orb = jv.util.symmetries.LatticeSymmetry(maps=maps, signs=signs, factor=np.array([1.0, 0.5, 0.25, 2.0]))
+    net, onet = (jv.nets.CpxRBM(H, bias=True), onets.CpxRBM((L,), H, bias=True)) if cpx else \
+        (jv.nets.RBM(H, bias=True), onets.RBM((L,), H, bias=True))
+    rng = np.random.default_rng(21)
+    P = 0.3 * rng.normal(size=_num(cpx, L, H, True, False))
+    psi = jv.NQS(net, orbit=orb)
+    psi(torch.zeros((1, 1, L), dtype=torch.int32))
+    psi.set_parameters(P)
+    opsi = onets.NQS(osym.SymNet(onet, orb.orbit, orb.factor, "exp"), P)
+    s = rng.integers(0, 2, size=(n, L)).astype(np.int32)
+    sd = torch.as_tensor(s[None], device="cuda")
+    lp, lpo = psi(sd), opsi(s)
+    assert np.max(np.abs(to_np(lp)[0] - lpo)) < TOL * np.max(np.abs(lpo))
+    for op in ("tfim", "mixed"):
+        Hd, Ho = OPS[op](L)
+        assert _rel(to_np(Hd.get_O_loc(sd, psi, lp))[0], Ho.get_O_loc(s, opsi, lpo)) < TOL
+    kw = dict(numChains=5, numSamples=20, thermalizationSweeps=3, sweepSteps=50)
+    ms = jv.sampler.MCSampler(psi, (L,), 5, updateProposer=jv.sampler.propose_spin_flip, **kw)
+    mo = osamp.MCSampler(opsi, (L,), 5, **kw)
+    assert np.array_equal(to_np(ms.sample()[0])[0], mo.sample()[0])
+
+
 def test_eloc_in_a_captured_graph():
     """A captured call keeps no pointer into the tables' scratch memory: calls
     with other sizes between the replays do not change its results."""

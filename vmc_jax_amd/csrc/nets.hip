@@ -76,22 +76,28 @@ __global__ void __launch_bounds__(256) rbm_fwd_grad(RbmGeom g, const double* __r
 }
 
 // ------------------------------------------------------------------ RBM ratio tables
-__global__ void __launch_bounds__(256) rbm_tables(RbmGeom g, const double* __restrict__ P, OpDev op, RbmTab t) {
+__global__ void __launch_bounds__(256) rbm_tables(RbmGeom g, const double* __restrict__ P, OpDev op, RbmTab t,
+                                                  const int32_t* __restrict__ map) {
   __shared__ double red[4];
   __shared__ int wcnt[4];
-  rbm_tab_build(g, P, t, &op, blockIdx.x, red, wcnt);
+  __shared__ uint32_t bits[RBM_ORBIT_MAX_L / 32];
+  const int own = rbm_tab_blocks(g, t.lead ? op.num_ops : 0);
+  if ((int)blockIdx.x >= own) rbm_tab_perm(map, g.L, blockIdx.x - own, t.perm, bits);
+  else rbm_tab_build(g, P, t, &op, blockIdx.x, red, wcnt);
 }
 
 // Tables of one parameter vector in the stream's scratch buffer (op: null for
-// the chains' tables, else the operator whose strings are listed).
+// the chains' tables, else the operator whose strings are listed; map: null, or
+// the site maps of G orbit elements, L <= RBM_ORBIT_MAX_L, to be checked).
 int build_rbm_tables(const RbmGeom& g, const double* params, const OpDev* op, bool me, bool he, hipStream_t st,
-                     int slot0, RbmTab* out) {
+                     int slot0, RbmTab* out, const int32_t* map, int G) {
   const int nops = op ? op->num_ops : 0;
-  double* base = (double*)stream_workspace(sizeof(double) * rbm_tab_doubles(g, me, he, nops), slot0, st);
+  if (!map) G = 0;
+  double* base = (double*)stream_workspace(sizeof(double) * rbm_tab_doubles(g, me, he, nops, G), slot0, st);
   if (!base) return fail(JV_E_NOMEM, "RBM ratio tables: workspace allocation failed");
-  *out = rbm_tab_at(g, base, me, he, nops);
-  hipLaunchKernelGGL(rbm_tables, dim3((unsigned)rbm_tab_blocks(g, nops)), dim3(256), 0, st, g, params,
-                     op ? *op : OpDev(), *out);
+  *out = rbm_tab_at(g, base, me, he, nops, G);
+  hipLaunchKernelGGL(rbm_tables, dim3((unsigned)(rbm_tab_blocks(g, nops) + G)), dim3(256), 0, st, g, params,
+                     op ? *op : OpDev(), *out, map);
   JV_LAUNCH_CHECK("rbm_tables");
   return JV_OK;
 }

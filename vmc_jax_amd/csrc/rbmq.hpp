@@ -26,6 +26,7 @@ constexpr double RBMQ_THETA = 150.0;
 // the chains (which a step may run on different streams).
 constexpr int WS_RBMQ_ELOC = 130, WS_RBMQ_MC = 140;
 constexpr int RBMQ_MAX_H = 900;  // prod_h (1 + e_h) <= 2^H
+constexpr int RBM_ORBIT_MAX_L = 16384;  // sites of an orbit's map (positions in 16 bits)
 
 // Device tables of one parameter vector (and one operator).  Elements of me /
 // he are complex for complex networks, real otherwise; index v is the spin
@@ -37,14 +38,18 @@ struct RbmTab {
   double* row;    // [H]: |Re b_h| + sum_i |Re W_ih|
   int32_t* lead;  // [0]: count; then 16 * string + followers (strings behind it that flip the same sites)
   int32_t* mark;  // [num_ops]: 1 for merged diagonal strings
+  int32_t* perm;  // [orbit elements]: 1 where every site is read once (null: no orbit)
 };
 
 __host__ __device__ inline int rbm_cw(const RbmGeom& g) { return g.cpx ? 2 : 1; }
-// Doubles of a table set (num_ops = 0: without the operator's lists).
-__host__ __device__ inline size_t rbm_tab_doubles(const RbmGeom& g, bool me, bool he, int num_ops) {
-  return (size_t)(me + he) * 2 * g.L * g.H * rbm_cw(g) + 8 * (size_t)g.L + g.H + (size_t)num_ops + 1;
+// Doubles of a table set (num_ops = 0: without the operator's lists; G: orbit
+// elements to check, 0 without an orbit).
+__host__ __device__ inline size_t rbm_tab_doubles(const RbmGeom& g, bool me, bool he, int num_ops, int G = 0) {
+  return (size_t)(me + he) * 2 * g.L * g.H * rbm_cw(g) + 8 * (size_t)g.L + g.H + (size_t)num_ops + 1 +
+         ((size_t)G + 1) / 2;
 }
-__host__ __device__ inline RbmTab rbm_tab_at(const RbmGeom& g, double* base, bool me, bool he, int num_ops) {
+__host__ __device__ inline RbmTab rbm_tab_at(const RbmGeom& g, double* base, bool me, bool he, int num_ops,
+                                             int G = 0) {
   RbmTab t;
   const size_t q = (size_t)2 * g.L * g.H * rbm_cw(g);
   t.me = me ? base : nullptr;
@@ -56,6 +61,7 @@ __host__ __device__ inline RbmTab rbm_tab_at(const RbmGeom& g, double* base, boo
   int32_t* i = (int32_t*)(t.row + g.H);
   t.lead = num_ops > 0 ? i : nullptr;
   t.mark = num_ops > 0 ? i + 1 + num_ops : nullptr;
+  t.perm = G > 0 ? i + 2 * ((size_t)num_ops + 1) : nullptr;
   return t;
 }
 // Workgroups that build a table set: one per site, one per 256 hidden units,
@@ -175,6 +181,9 @@ __device__ inline void rbm_tab_build(const RbmGeom& g, const double* __restrict_
   if (tid == 0) t.lead[0] = cnt;
 }
 
+int build_rbm_tables(const RbmGeom& g, const double* params, const OpDev* op, bool me, bool he, hipStream_t st,
+                     int slot0, RbmTab* out, const int32_t* map = nullptr, int G = 0);
+
 // Whether the products stay in range for strings changing up to `nch` sites
 // (same answer in every lane; false for NaN parameters).
 __device__ inline bool rbmq_ok(const RbmGeom& g, const RbmTab& t, int nch, int lane) {
@@ -183,6 +192,20 @@ __device__ inline bool rbmq_ok(const RbmGeom& g, const RbmTab& t, int nch, int l
   for (int i = lane; i < g.L; i += WAVE) ok = ok && t.site[8 * (int64_t)i + 6] <= lim;
   for (int h = lane; h < g.H; h += WAVE) ok = ok && t.row[h] <= RBMQ_THETA;
   return __all(ok);
+}
+
+// Whether orbit element r reads every site once: perm[r] (workgroup of 256
+// threads; bits: one bit per site in LDS).
+__device__ inline void rbm_tab_perm(const int32_t* __restrict__ map, int L, int r, int32_t* perm, uint32_t* bits) {
+  for (int i = threadIdx.x; i < (L + 31) / 32; i += 256) bits[i] = 0;
+  __syncthreads();
+  int bad = 0;
+  for (int i = threadIdx.x; i < L; i += 256) {
+    const int m = map[(int64_t)r * L + i], j = m >= 0 ? m : -1 - m;
+    if (j >= L || (atomicOr(&bits[j / 32], 1u << (j % 32)) >> (j % 32) & 1)) bad = 1;
+  }
+  bad = __syncthreads_or(bad);
+  if (threadIdx.x == 0) perm[r] = !bad;
 }
 
 // ------------------------------------------------------------------ arithmetic

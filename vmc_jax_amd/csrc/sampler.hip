@@ -10,8 +10,6 @@ namespace jv {
 bool make_rbm_geom(const jv_net* net, RbmGeom& g);
 bool make_cnn_geom(const jv_net* net, CnnGeom& g);
 int set_lds_limit(const void* fn, size_t bytes);
-int build_rbm_tables(const RbmGeom& g, const double* params, const OpDev* op, bool me, bool he, hipStream_t st,
-                     int slot0, RbmTab* out);
 
 __global__ void zero_i64(int64_t* p, int n) {
   int i = blockIdx.x * blockDim.x + threadIdx.x;

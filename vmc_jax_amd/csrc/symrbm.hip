@@ -6,8 +6,9 @@
 // psi(s) = sum_g b_g psi_net(g s).  Flipping site i flips one site of every row
 // g s, so psi(s') / psi(s) = sum_g w_g r_g with w_g = b_g psi_net(g s) / psi(s)
 // and r_g the RBM ratio of rbmq.hpp: eight FP64 operations per row, hidden
-// unit and flip.  Parameters outside the ratio form's range are evaluated row
-// by row with rbm.hpp's log-cosh (slow_* below).
+// unit and flip.  Parameters outside the ratio form's range, and orbits with a
+// row that reads a site twice, are evaluated row by row with rbm.hpp's log-cosh
+// (slow_* below).
 #include <algorithm>
 #include <cmath>
 #include <string>
@@ -17,8 +18,6 @@
 namespace jv {
 
 int set_lds_limit(const void* fn, size_t bytes);
-int build_rbm_tables(const RbmGeom& g, const double* params, const OpDev* op, bool me, bool he, hipStream_t st,
-                     int slot0, RbmTab* out);
 bool make_rbm_geom(const jv_net* net, RbmGeom& g);
 OpDev make_opdev(const jv_optable* op, const double* pref, int L);
 
@@ -37,6 +36,15 @@ constexpr int SYM_T = 256;       // threads of the forward and local-energy work
 __device__ inline int row_spin(const SymGeom& o, int L, const int32_t* s, int r, int i) {
   const int m = o.map[(int64_t)r * L + i];
   return m >= 0 ? (s[m] > 0) : !(s[-1 - m] > 0);
+}
+
+// Whether the resident chains and local energies apply: parameters in range,
+// and every row a permutation of the sites (they look up where a flipped site
+// sits in a row; log psi only reads the rows).
+__device__ inline bool sym_ok(const RbmGeom& g, const SymGeom& o, const RbmTab& t, int lane) {
+  bool ok = true;
+  for (int r = lane; r < o.G; r += WAVE) ok = ok && t.perm[r];
+  return __all(ok) && rbmq_ok(g, t, 2, lane);
 }
 
 struct quad {
@@ -266,7 +274,7 @@ __global__ void __launch_bounds__(SYM_T, 2) sym_rbm_eloc(RbmGeom g, SymGeom o, c
   unsigned short* inv = (unsigned short*)(s + L);  // [RC][L]: position of a site in the row
   unsigned char* rb = (unsigned char*)(inv + RC * L);  // [RC][L]
   const int nl = tab.lead[0];
-  if (!rbmq_ok(g, tab, 2, lane)) return;  // sym_slow_eloc's
+  if (!sym_ok(g, o, tab, lane)) return;  // sym_slow_eloc's
   if (TAB)
     for (int t = tid; t < 2 * H * L; t += SYM_T) he[t] = ((const T*)tab.he)[t];
   for (int64_t q = blockIdx.x; q < n; q += gridDim.x) {
@@ -464,7 +472,7 @@ __global__ void __launch_bounds__(MAXT, MAXT == 256 ? 3 : MAXT == 512 ? 2 : 4) s
   int32_t* s = (int32_t*)(me + (TAB ? (size_t)2 * L * HP : 0));
   unsigned short* inv = (unsigned short*)(s + L);  // [G][L]: 2 * position + (row holds the flipped spin)
   unsigned char* rb = (unsigned char*)(inv + (size_t)G * L);  // [G][L] spins of the rows (refresh only)
-  if (!rbmq_ok(g, tab, 2, lane)) return;  // sym_slow_mc's
+  if (!sym_ok(g, o, tab, lane)) return;  // sym_slow_mc's
   for (int i = tid; i < L; i += nt) s[i] = walkers[(int64_t)chain * L + i] > 0;
   for (int t = tid; t < 2 * L; t += nt) {
     const double* pq = tab.site + 8 * (int64_t)(t / 2) + 2 + 2 * (t % 2);
@@ -609,7 +617,7 @@ size_t sym_mc_lds(const RbmGeom& g, int G, bool tabl) {
          3 * (size_t)G * g.L + 16;
 }
 
-// ------------------------------------------------------------------ parameters out of range
+// ------------------------------------------------------------------ parameters out of range, other maps
 // Row by row with rbm.hpp's log-cosh, one configuration or chain per
 // workgroup; these kernels return at once where the resident ones above work
 // (and the other way round), so neither carries the other's registers.
@@ -637,7 +645,7 @@ __global__ void __launch_bounds__(SYM_T) sym_slow_eloc(RbmGeom g, SymGeom o, con
                                                        const double* __restrict__ lps, int64_t n,
                                                        double* __restrict__ out) {
   extern __shared__ double lds[];
-  if (rbmq_ok(g, tab, 2, threadIdx.x % WAVE)) return;
+  if (sym_ok(g, o, tab, threadIdx.x % WAVE)) return;
   cd* c = (cd*)(lds + 8);
   int32_t* s = (int32_t*)(c + o.G);
   for (int64_t q = blockIdx.x; q < n; q += gridDim.x) {
@@ -672,7 +680,7 @@ __global__ void __launch_bounds__(SYM_T) sym_slow_mc(RbmGeom g, SymGeom o, const
                                                      RbmTab tab, int32_t* __restrict__ walkers,
                                                      int32_t* __restrict__ configs, int64_t* __restrict__ counters) {
   extern __shared__ double lds[];
-  if (rbmq_ok(g, tab, 2, threadIdx.x % WAVE)) return;
+  if (sym_ok(g, o, tab, threadIdx.x % WAVE)) return;
   const int tid = threadIdx.x, chain = blockIdx.x;
   cd* c = (cd*)(lds + 8);
   int32_t* s = (int32_t*)(c + o.G);
@@ -718,7 +726,7 @@ bool sym_rbm_geom(const jv_net* net, const jv_orbit* orbit, RbmGeom& g, SymGeom&
   o.cpx = net->is_complex || orbit->complex_factor;
   o.map = orbit->map;
   o.fac = orbit->factor;
-  return o.G <= SYM_MAX_G && g.H <= RBMQ_MAX_H && g.L <= 16384;
+  return o.G <= SYM_MAX_G && g.H <= RBMQ_MAX_H && g.L <= RBM_ORBIT_MAX_L;
 }
 
 }  // namespace
@@ -775,7 +783,7 @@ int sym_rbm_eloc_launch(const jv_net* net, const double* params, const jv_orbit*
     }
   if (!RC) return JV_OK;
   RbmTab tab;
-  int rc = build_rbm_tables(g, params, &d, false, true, st, slot0, &tab);
+  int rc = build_rbm_tables(g, params, &d, false, true, st, slot0, &tab, o.map, o.G);
   if (rc) return rc;
 #define JV_SYM_ELO(RCv)                                                                           \
   (g.cpx ? (tabl ? sym_rbm_eloc<true, RCv, true> : sym_rbm_eloc<true, RCv, false>)                \
@@ -818,7 +826,7 @@ int sym_rbm_mc_launch(const jv_net* net, const double* params, const jv_orbit* o
   const size_t lds = sym_mc_lds(g, o.G, tabl);
   if (lds > 160 * 1024) return JV_OK;
   RbmTab tab;
-  int rc = build_rbm_tables(g, params, nullptr, true, false, st, slot0, &tab);
+  int rc = build_rbm_tables(g, params, nullptr, true, false, st, slot0, &tab, o.map, o.G);
   if (rc) return rc;
   const int T = (o.G * SL + WAVE - 1) / WAVE * WAVE;
 #define JV_SYM_MC(HTv, Tv)                                                                                \
