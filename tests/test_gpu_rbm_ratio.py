@@ -317,6 +317,24 @@ def test_sym_resident(cpx, L, H, names, op, big):
     assert float(ms.acceptance_ratio()[0]) == float(np.ravel(mo.acceptance_ratio())[0])
 
 
+@pytest.mark.parametrize("big", [0.0, 90.0])
+@pytest.mark.parametrize("cpx,L,H,names", [
+    (True, 10, 1, ("reflection",)), (True, 11, 200, ("reflection",)), (False, 6, 300, ("reflection",)),
+    (True, 8, 130, ("translation",)), (True, 16, 33, ("translation",)), (True, 24, 8, ALL), (False, 16, 32, ALL)])
+def test_sym_log_psi(cpx, L, H, names, big):
+    """log psi over every split of a row between threads (4 to 64 threads, one
+    or four units each), weights of ordinary size and far outside the ratio
+    form's range."""
+    rng = np.random.default_rng(L * 1000 + H)
+    P = 0.3 / np.sqrt(L) * rng.normal(size=_num(cpx, L, H, True, False))
+    if big:
+        P[(2 if cpx else 1) * H] = big
+    psi, opsi = _sym_states(cpx, L, H, names, P)
+    s = rng.integers(0, 2, size=(13, L)).astype(np.int32)
+    lp, lpo = to_np(psi(torch.as_tensor(s[None], device="cuda")))[0], opsi(s)
+    assert np.max(np.abs(lp - lpo)) < TOL * np.max(np.abs(lpo))
+
+
 @pytest.mark.parametrize("cpx", [True, False])
 def test_sym_rows_that_are_no_permutation(cpx):
     """An orbit element may read a site twice, or never: (g s)_i = s_{m_i} all

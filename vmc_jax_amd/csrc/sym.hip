@@ -20,7 +20,7 @@ namespace jv {
 int check_op(const jv_optable* op, const double* pref);
 // Resident forms for RBMs under avgFun_Coefficients_Exp (symrbm.hip).
 int sym_rbm_forward_launch(const jv_net* net, const double* params, const jv_orbit* orbit, const int32_t* configs,
-                           int64_t n, double* logpsi, hipStream_t st, int slot0, bool* done);
+                           int64_t n, double* logpsi, hipStream_t st, bool* done);
 int sym_rbm_eloc_launch(const jv_net* net, const double* params, const jv_orbit* orbit, const jv_optable* op,
                         const double* prefactor, const int32_t* configs, const double* lps, int64_t n, double* out,
                         hipStream_t st, int slot0, bool* done);
@@ -29,7 +29,7 @@ int sym_rbm_mc_launch(const jv_net* net, const double* params, const jv_orbit* o
 
 namespace {
 // first slots of the resident forms' tables in stream_workspace
-constexpr int WS_SYM_FWD_TAB = 150, WS_SYM_ELOC_TAB = 160, WS_SYM_MC_TAB = 170;
+constexpr int WS_SYM_ELOC_TAB = 150, WS_SYM_MC_TAB = 160;
 // workspace slots of this file.  jv_sym_eloc may run on a side stream while
 // jv_sym_gradients runs on the main stream, so the forward pass inside
 // jv_sym_eloc has rows / log-psi slots of its own (WS_EROWS, WS_ELP).
@@ -312,7 +312,7 @@ int sym_forward(const jv_net* net, const double* params, const jv_orbit* orbit, 
   if (n == 0) return JV_OK;
   hipStream_t st = (hipStream_t)stream;
   bool done = false;
-  rc = sym_rbm_forward_launch(net, params, orbit, configs, n, logpsi, st, WS_SYM_FWD_TAB, &done);
+  rc = sym_rbm_forward_launch(net, params, orbit, configs, n, logpsi, st, &done);
   if (rc || done) return rc;
   const int L = net->num_sites, G = orbit->num_elements;
   const int64_t cs = std::min<int64_t>(n, rows_per_chunk(net, orbit, 0));

@@ -61,27 +61,33 @@ __device__ inline quad load4(const double* __restrict__ p, int h, int H) {
   }
   return q;
 }
-// theta of hidden units h .. h + 3 (clamped to H - 1) for one row's spins.
-template <bool CPX>
-__device__ inline void theta4(const RbmGeom& g, const double* __restrict__ P, const unsigned char* row, int h,
-                              cd* th) {
+// theta of hidden units h .. h + U - 1 (clamped to H - 1; U = 4 or 1) for one
+// row's spins.
+template <bool CPX, int U = 4>
+__device__ inline void theta_of(const RbmGeom& g, const double* __restrict__ P, const unsigned char* row, int h,
+                                cd* th) {
   const double* Wr = P + g.ow;
   const double* Wi = Wr + (int64_t)g.L * g.H;
 #pragma unroll
-  for (int k = 0; k < 4; ++k) {
+  for (int k = 0; k < U; ++k) {
     const int hc = min(h + k, g.H - 1);
     th[k] = {g.ob >= 0 ? P[g.ob + hc] : 0.0, CPX && g.ob >= 0 ? P[g.ob + g.H + hc] : 0.0};
   }
-#pragma unroll 4
+#pragma unroll(U == 4 ? 4 : 8)
   for (int i = 0; i < g.L; ++i) {
     const double sg = row[i] ? 1.0 : -1.0;
-    const quad wr = load4(Wr + (int64_t)i * g.H, h, g.H);
-    quad wm = wr;
-    if (CPX) wm = load4(Wi + (int64_t)i * g.H, h, g.H);
+    if constexpr (U == 4) {
+      const quad wr = load4(Wr + (int64_t)i * g.H, h, g.H);
+      quad wm = wr;
+      if (CPX) wm = load4(Wi + (int64_t)i * g.H, h, g.H);
 #pragma unroll
-    for (int k = 0; k < 4; ++k) {
-      th[k].re = fma(sg, wr.v[k], th[k].re);
-      if (CPX) th[k].im = fma(sg, wm.v[k], th[k].im);
+      for (int k = 0; k < 4; ++k) {
+        th[k].re = fma(sg, wr.v[k], th[k].re);
+        if (CPX) th[k].im = fma(sg, wm.v[k], th[k].im);
+      }
+    } else {
+      th[0].re = fma(sg, Wr[(int64_t)i * g.H + h], th[0].re);
+      if (CPX) th[0].im = fma(sg, Wi[(int64_t)i * g.H + h], th[0].im);
     }
   }
 }
@@ -165,80 +171,106 @@ __device__ __forceinline__ cd slow_logpsi(const RbmGeom& g, const SymGeom& o, co
 }
 
 // ------------------------------------------------------------------ log psi
-// A workgroup per configuration: four threads per row, four hidden units at a
-// time.  FP64 issue (exp and sincos of every theta) sets its time: 4096
-// samples, 16 sites x 32 units, 64 elements 600 -> 100 us.
-template <bool CPX>
-__global__ void __launch_bounds__(SYM_T, 2) sym_rbm_forward(RbmGeom g, SymGeom o, const double* __restrict__ P,
-                                                            RbmTab tab, const int32_t* __restrict__ cfg, int64_t n,
-                                                            double* __restrict__ out) {
+// log psi of the spins s (LDS) by the whole workgroup: SL threads per row, U
+// hidden units at a time (sym_lanes).  A row's amplitude is
+// e^{lin} prod_h d_h / 2^H with Re lin >= 0 and |d_h| <= 2 (rbm_ab), whatever
+// the size of theta: no logarithm per unit and no range to test.  lin, dd: [G];
+// rb: [threads / SL][L].  Same value in every thread.
+template <bool CPX, int U, int SLC>
+__device__ __forceinline__ cd block_logpsi(const RbmGeom& g, const SymGeom& o, const double* __restrict__ P,
+                                           const int32_t* s, int SLr, cd* lin, cd* dd, unsigned char* rb, double* red) {
   typedef typename num_of<CPX>::type T;
+  const int SL = SLC > 0 ? SLC : SLr;
+  const int L = g.L, H = g.H, G = o.G, tid = threadIdx.x, nt = blockDim.x, RC = nt / SL;
+  const int r = tid / SL, sl = tid % SL;
+  double mx = -INFINITY;
+  __syncthreads();  // s is set
+  for (int r0 = 0; r0 < G; r0 += RC) {
+    if (r < min(RC, G - r0)) {
+      unsigned char* row = rb + r * L;  // of this row's threads, all in one wave
+      wave_sync();
+      for (int i = sl; i < L; i += SL) row[i] = row_spin(o, L, s, r0 + r, i);
+      wave_sync();
+      cd li = visible(g, P, row, sl, SL);
+      T dp;
+      set_one(dp);
+      for (int h = U * sl; h < H; h += U * SL) {
+        cd th[U];
+        theta_of<CPX, U>(g, P, row, h, th);
+#pragma unroll
+        for (int k = 0; k < U; ++k)
+          if (h + k < H) {
+            T al, be, d;
+            cd l;
+            ab_of<CPX>(th[k], al, be, l, d);
+            li = li + l;
+            dp = mulc(dp, d);
+          }
+      }
+      for (int m = 1; m < SL; m *= 2) {
+        li = li + shfl_xor(li, m);
+        dp = mulc(dp, shfl_xor(dp, m));
+      }
+      if (sl == 0) {
+        lin[r0 + r] = li;
+        dd[r0 + r] = to_cd(dp);
+      }
+      if (o.fac[2 * (r0 + r)] != 0.0 || o.fac[2 * (r0 + r) + 1] != 0.0) mx = fmax(mx, li.re);
+    }
+  }
+  mx = block_max(mx, red);
+  if (!isfinite(mx)) mx = 0.0;
+  cd S = {0.0, 0.0};
+  for (int q = tid; q < G; q += nt) {
+    const cd b = {o.fac[2 * q], o.fac[2 * q + 1]};
+    if (b.re == 0.0 && b.im == 0.0) continue;
+    const double x = fma(-(double)H, LN2, lin[q].re - mx);
+    if (o.cpx) S = S + mulc(mulc(cexp({x, lin[q].im}), dd[q]), b);
+    else S.re += exp(x) * dd[q].re * b.re;
+  }
+  return log_of_sum(block_sum_cd(S, red), mx, o.cpx);
+}
+
+// Threads per row and hidden units at a time (*four: 4, else 1).  Four units a
+// thread share a row's spins and signs; one where rows have fewer than 16 units
+// or all rows' units fit one wave.  As many threads as the units fill within
+// 256 a configuration: with four per row whatever the group, 64 sites x 200
+// units of a two-element group took 1701 us for 4096 samples (165 with 64, 258
+// by one wave per materialised row); 512 a configuration: 274 against 188 us
+// for 64 elements of 16 sites x 32 units.
+int sym_lanes(int G, int H, bool* four) {
+  int p2 = 4, sl = 4;
+  while (p2 < H && p2 < WAVE) p2 *= 2;
+  *four = H >= 16 && (H > WAVE || G * p2 > WAVE);
+  while (sl < WAVE && (*four ? 4 * sl : sl) < H && 2 * sl * G <= SYM_T) sl *= 2;
+  return sl;
+}
+int sym_threads(int G, int SL, int most) { return std::min(most, (G * SL + WAVE - 1) / WAVE * WAVE); }
+
+// A workgroup per configuration.  FP64 issue (exp and sincos of every theta)
+// sets its time: 4096 samples, 16 sites x 32 units, 64 elements: 589 us with
+// materialised rows, 188 here (a call and its wait).
+template <bool CPX, int U, int SLC>
+__global__ void __launch_bounds__(SYM_T, 2) sym_rbm_forward(RbmGeom g, SymGeom o, const double* __restrict__ P, int SL,
+                                                            const int32_t* __restrict__ cfg, int64_t n,
+                                                            double* __restrict__ out) {
   extern __shared__ double lds[];
-  constexpr int SL = 4, RC = SYM_T / SL;
-  const int L = g.L, H = g.H, G = o.G, tid = threadIdx.x;
   double* red = lds;
   cd* lin = (cd*)(red + 8);  // [G]
-  cd* dd = lin + G;          // [G]
-  int32_t* s = (int32_t*)(dd + G);
-  unsigned char* rb = (unsigned char*)(s + L);  // [RC][L]
-  if (!rbmq_ok(g, tab, 2, tid % WAVE)) return;  // sym_slow_forward's
+  cd* dd = lin + o.G;        // [G]
+  int32_t* s = (int32_t*)(dd + o.G);
+  unsigned char* rb = (unsigned char*)(s + g.L);
   for (int64_t q = blockIdx.x; q < n; q += gridDim.x) {
-    __syncthreads();
-    for (int i = tid; i < L; i += SYM_T) s[i] = cfg[q * L + i];
-    __syncthreads();
-    double mx = -INFINITY;
-    for (int r0 = 0; r0 < G; r0 += RC) {
-      const int nr = min(RC, G - r0);
-      for (int t = tid; t < nr * L; t += SYM_T) rb[t] = row_spin(o, L, s, r0 + t / L, t % L);
-      __syncthreads();
-      const int r = tid / SL, sl = tid % SL;
-      if (r < nr) {
-        const unsigned char* row = rb + r * L;
-        cd li = visible(g, P, row, sl, SL);
-        T dp;
-        set_one(dp);
-        for (int h = 4 * sl; h < H; h += 4 * SL) {
-          cd th[4];
-          theta4<CPX>(g, P, row, h, th);
-#pragma unroll
-          for (int k = 0; k < 4; ++k)
-            if (h + k < H) {
-              T al, be, d;
-              cd l;
-              ab_of<CPX>(th[k], al, be, l, d);
-              li = li + l;
-              dp = mulc(dp, d);
-            }
-        }
-        for (int m = 1; m < SL; m *= 2) {
-          li = li + shfl_xor(li, m);
-          dp = mulc(dp, shfl_xor(dp, m));
-        }
-        if (sl == 0) {
-          lin[r0 + r] = li;
-          dd[r0 + r] = to_cd(dp);
-        }
-        if (o.fac[2 * (r0 + r)] != 0.0 || o.fac[2 * (r0 + r) + 1] != 0.0) mx = fmax(mx, li.re);
-      }
-      __syncthreads();
-    }
-    mx = block_max(mx, red);
-    if (!isfinite(mx)) mx = 0.0;
-    cd S = {0.0, 0.0};
-    for (int r = tid; r < G; r += SYM_T) {
-      const cd b = {o.fac[2 * r], o.fac[2 * r + 1]};
-      if (b.re == 0.0 && b.im == 0.0) continue;
-      S = S + mulc(mulc(cexp({fma(-(double)H, LN2, lin[r].re - mx), lin[r].im}), dd[r]), b);
-    }
-    const cd lp = log_of_sum(block_sum_cd(S, red), mx, o.cpx);
-    if (tid == 0) {
+    for (int i = threadIdx.x; i < g.L; i += blockDim.x) s[i] = cfg[q * g.L + i];
+    const cd lp = block_logpsi<CPX, U, SLC>(g, o, P, s, SL, lin, dd, rb, red);
+    if (threadIdx.x == 0) {
       out[2 * q] = lp.re;
       out[2 * q + 1] = lp.im;
     }
   }
 }
-size_t sym_fwd_lds(const RbmGeom& g, int G) {
-  return 8 * 8 + 32 * (size_t)G + 4 * (size_t)g.L + (size_t)(SYM_T / 4) * g.L + 16;
+size_t sym_rows_lds(const RbmGeom& g, int G, int T, int SL) {
+  return 8 * 8 + 32 * (size_t)G + 4 * (size_t)g.L + (size_t)(T / SL) * g.L + 16;
 }
 
 // ------------------------------------------------------------------ local energies
@@ -333,7 +365,7 @@ __global__ void __launch_bounds__(SYM_T, 2) sym_rbm_eloc(RbmGeom g, SymGeom o, c
           set_one(dp);
           for (int h = 4 * sl; h < H; h += 4 * SL) {
             cd th[4];
-            theta4<CPX>(g, P, row, h, th);
+            theta_of<CPX>(g, P, row, h, th);
 #pragma unroll
             for (int k = 0; k < 4; ++k)
               if (h + k < H) {
@@ -516,7 +548,7 @@ __global__ void __launch_bounds__(MAXT, MAXT == 256 ? 3 : MAXT == 512 ? 2 : 4) s
 #pragma unroll
     for (int k0 = 0; k0 < HT; k0 += 4) {
       cd th[4];
-      theta4<CPX>(g, P, row, h0 + k0, th);
+      theta_of<CPX>(g, P, row, h0 + k0, th);
 #pragma unroll
       for (int j = 0; j < 4; ++j) {
         const int k = k0 + j;
@@ -621,25 +653,6 @@ size_t sym_mc_lds(const RbmGeom& g, int G, bool tabl) {
 // Row by row with rbm.hpp's log-cosh, one configuration or chain per
 // workgroup; these kernels return at once where the resident ones above work
 // (and the other way round), so neither carries the other's registers.
-__global__ void __launch_bounds__(SYM_T) sym_slow_forward(RbmGeom g, SymGeom o, const double* __restrict__ P,
-                                                          RbmTab tab, const int32_t* __restrict__ cfg, int64_t n,
-                                                          double* __restrict__ out) {
-  extern __shared__ double lds[];
-  if (rbmq_ok(g, tab, 2, threadIdx.x % WAVE)) return;
-  cd* c = (cd*)(lds + 8);
-  int32_t* s = (int32_t*)(c + o.G);
-  for (int64_t q = blockIdx.x; q < n; q += gridDim.x) {
-    __syncthreads();
-    for (int i = threadIdx.x; i < g.L; i += SYM_T) s[i] = cfg[q * g.L + i];
-    __syncthreads();
-    const cd lp = slow_logpsi(g, o, P, s, c, lds);
-    if (threadIdx.x == 0) {
-      out[2 * q] = lp.re;
-      out[2 * q + 1] = lp.im;
-    }
-  }
-}
-
 __global__ void __launch_bounds__(SYM_T) sym_slow_eloc(RbmGeom g, SymGeom o, const double* __restrict__ P, OpDev op,
                                                        RbmTab tab, const int32_t* __restrict__ cfg,
                                                        const double* __restrict__ lps, int64_t n,
@@ -734,25 +747,24 @@ bool sym_rbm_geom(const jv_net* net, const jv_orbit* orbit, RbmGeom& g, SymGeom&
 // Each returns JV_OK with *done = true when the resident form applies (RBM,
 // avgFun_Coefficients_Exp, LDS and registers suffice), else *done = false.
 int sym_rbm_forward_launch(const jv_net* net, const double* params, const jv_orbit* orbit, const int32_t* configs,
-                           int64_t n, double* logpsi, hipStream_t st, int slot0, bool* done) {
+                           int64_t n, double* logpsi, hipStream_t st, bool* done) {
   *done = false;
   RbmGeom g;
   SymGeom o;
   if (!sym_rbm_geom(net, orbit, g, o)) return JV_OK;
-  const size_t lds = sym_fwd_lds(g, o.G);
+  bool four;
+  const int SL = sym_lanes(o.G, g.H, &four), T = sym_threads(o.G, SL, SYM_T);
+  const size_t lds = sym_rows_lds(g, o.G, T, SL);
   if (lds > 160 * 1024) return JV_OK;
-  RbmTab tab;
-  int rc = build_rbm_tables(g, params, nullptr, false, false, st, slot0, &tab);
-  const auto fn = g.cpx ? sym_rbm_forward<true> : sym_rbm_forward<false>;
-  if (!rc) rc = set_lds_limit((const void*)fn, lds);
+#define JV_SYM_FWD(CPX)                                                                  \
+  (four ? (SL == 4 ? sym_rbm_forward<CPX, 4, 4> : sym_rbm_forward<CPX, 4, 0>) : sym_rbm_forward<CPX, 1, 0>)
+  const auto fn = g.cpx ? JV_SYM_FWD(true) : JV_SYM_FWD(false);
+#undef JV_SYM_FWD
+  const int rc = set_lds_limit((const void*)fn, lds);
   if (rc) return rc;
-  hipLaunchKernelGGL(fn, dim3((unsigned)std::min<int64_t>(n, 1 << 20)), dim3(SYM_T), lds, st, g, o, params, tab, configs,
-                     n, logpsi);
+  hipLaunchKernelGGL(fn, dim3((unsigned)std::min<int64_t>(n, 1 << 20)), dim3((unsigned)T), lds, st, g, o, params, SL,
+                     configs, n, logpsi);
   JV_LAUNCH_CHECK("sym_rbm_forward");
-  if ((rc = set_lds_limit((const void*)sym_slow_forward, sym_slow_lds(g, o.G)))) return rc;
-  hipLaunchKernelGGL(sym_slow_forward, dim3((unsigned)std::min<int64_t>(n, 512)), dim3(SYM_T), sym_slow_lds(g, o.G), st,
-                     g, o, params, tab, configs, n, logpsi);
-  JV_LAUNCH_CHECK("sym_slow_forward");
   *done = true;
   return JV_OK;
 }
