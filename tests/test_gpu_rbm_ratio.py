@@ -335,6 +335,34 @@ def test_sym_log_psi(cpx, L, H, names, big):
     assert np.max(np.abs(lp - lpo)) < TOL * np.max(np.abs(lpo))
 
 
+@pytest.mark.parametrize("cpx,L,H,names,op,mu", [
+    (True, 10, 1, ("reflection",), "tfim", 2.0), (True, 11, 200, ("reflection",), "xxz", 2.0),
+    (False, 6, 300, ("reflection",), "mixed", 1.0), (True, 8, 40, ("translation",), "mixed", 2.0),
+    (True, 24, 8, ALL, "tfim", 0.5), (False, 16, 32, ALL, "xxz", 2.0)])
+def test_sym_out_of_range(cpx, L, H, names, op, mu):
+    """Local energies and chains with a weight far outside the ratio form's
+    range, over the splits of a row between threads."""
+    rng = np.random.default_rng(L * 1000 + H)
+    P = 0.3 / np.sqrt(L) * rng.normal(size=_num(cpx, L, H, True, False))
+    P[(2 if cpx else 1) * H] = 90.0
+    psi, opsi = _sym_states(cpx, L, H, names, P)
+    s = rng.integers(0, 2, size=(13, L)).astype(np.int32)
+    sd = torch.as_tensor(s[None], device="cuda")
+    Hd, Ho = OPS[op](L)
+    lpo = opsi(s)
+    e = to_np(Hd.get_O_loc(sd, psi, torch.as_tensor(lpo[None], device="cuda")))[0]
+    ref = Ho.get_O_loc(s, opsi, lpo)
+    # log psi is some 1e3 in size: its rounding error is the exponent's
+    assert np.max(np.abs(e - ref)) < 1e-10 * np.max(np.abs(ref))
+    kw = dict(numChains=3, numSamples=9, thermalizationSweeps=2, sweepSteps=30, mu=mu)
+    ms = jv.sampler.MCSampler(psi, (L,), 5, updateProposer=jv.sampler.propose_spin_flip, **kw)
+    mo = osamp.MCSampler(opsi, (L,), 5, **kw)
+    for _ in range(2):
+        assert np.array_equal(to_np(ms.sample()[0])[0], mo.sample()[0])
+    assert np.array_equal(to_np(ms.states), mo.states)
+    assert float(ms.acceptance_ratio()[0]) == float(np.ravel(mo.acceptance_ratio())[0])
+
+
 @pytest.mark.parametrize("cpx", [True, False])
 def test_sym_rows_that_are_no_permutation(cpx):
     """An orbit element may read a site twice, or never: (g s)_i = s_{m_i} all

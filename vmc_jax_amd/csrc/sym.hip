@@ -23,13 +23,13 @@ int sym_rbm_forward_launch(const jv_net* net, const double* params, const jv_orb
                            int64_t n, double* logpsi, hipStream_t st, bool* done);
 int sym_rbm_eloc_launch(const jv_net* net, const double* params, const jv_orbit* orbit, const jv_optable* op,
                         const double* prefactor, const int32_t* configs, const double* lps, int64_t n, double* out,
-                        hipStream_t st, int slot0, bool* done);
+                        hipStream_t st, int slot0, int slot1, bool* done);
 int sym_rbm_mc_launch(const jv_net* net, const double* params, const jv_orbit* orbit, const jv_mc_args& a,
                       int32_t* walkers, int32_t* configs, int64_t* counters, hipStream_t st, int slot0, bool* done);
 
 namespace {
-// first slots of the resident forms' tables in stream_workspace
-constexpr int WS_SYM_ELOC_TAB = 150, WS_SYM_MC_TAB = 160;
+// first slots of the resident forms' tables and partial sums in stream_workspace
+constexpr int WS_SYM_ELOC_TAB = 150, WS_SYM_MC_TAB = 160, WS_SYM_ELOC_PART = 170;
 // workspace slots of this file.  jv_sym_eloc may run on a side stream while
 // jv_sym_gradients runs on the main stream, so the forward pass inside
 // jv_sym_eloc has rows / log-psi slots of its own (WS_EROWS, WS_ELP).
@@ -398,7 +398,8 @@ int jv_sym_eloc(const jv_net* net, const double* params, const jv_orbit* orbit, 
   if ((rc = check_op(op, prefactor))) return rc;
   ScopedTimer tm("sym_eloc", st);
   bool done = false;
-  rc = sym_rbm_eloc_launch(net, params, orbit, op, prefactor, configs, logpsi_s, n, out, st, WS_SYM_ELOC_TAB, &done);
+  rc = sym_rbm_eloc_launch(net, params, orbit, op, prefactor, configs, logpsi_s, n, out, st, WS_SYM_ELOC_TAB, WS_SYM_ELOC_PART,
+                           &done);
   if (rc || done) return rc;
   const int L = net->num_sites, nops = op->num_ops;
   // s' of cs samples are cs * nops configurations, each expanded |orbit| times by jv_sym_forward

@@ -7,8 +7,8 @@
 // g s, so psi(s') / psi(s) = sum_g w_g r_g with w_g = b_g psi_net(g s) / psi(s)
 // and r_g the RBM ratio of rbmq.hpp: eight FP64 operations per row, hidden
 // unit and flip.  Parameters outside the ratio form's range, and orbits with a
-// row that reads a site twice, are evaluated row by row with rbm.hpp's log-cosh
-// (slow_* below).
+// row that reads a site twice, are evaluated row by row from scratch
+// (sym_rows_*).
 #include <algorithm>
 #include <cmath>
 #include <string>
@@ -132,44 +132,6 @@ __device__ inline cd log_of_sum(cd S, double shift, int cpx) {
   return {S.re < 0.0 ? NAN : log(fabs(S.re)) + shift, 0.0};
 }
 
-// log psi of the spins s (LDS) by the whole workgroup, one row per thread at a
-// time, log-cosh per hidden unit; c: [G] scratch.  Same value in every thread.
-__device__ __forceinline__ cd slow_logpsi(const RbmGeom& g, const SymGeom& o, const double* __restrict__ P, const int32_t* s,
-                                 cd* c, double* red) {
-  double mx = -INFINITY;
-  for (int r = threadIdx.x; r < o.G; r += blockDim.x) {
-    cd a = {0.0, 0.0};
-    for (int h = 0; h < g.H; ++h) {
-      cd th = {g.ob >= 0 ? P[g.ob + h] : 0.0, g.cpx && g.ob >= 0 ? P[g.ob + g.H + h] : 0.0};
-      for (int i = 0; i < g.L; ++i) {
-        const double sg = row_spin(o, g.L, s, r, i) ? 1.0 : -1.0;
-        const int64_t w = g.ow + (int64_t)i * g.H + h;
-        th.re = fma(sg, P[w], th.re);
-        if (g.cpx) th.im = fma(sg, P[w + (int64_t)g.L * g.H], th.im);
-      }
-      a = a + (g.cpx ? log_cosh(th) : cd{log_cosh(th.re), 0.0});
-    }
-    if (g.oa >= 0)
-      for (int i = 0; i < g.L; ++i) {
-        const double sg = row_spin(o, g.L, s, r, i) ? 1.0 : -1.0;
-        a.re = fma(sg, P[g.oa + i], a.re);
-        a.im = fma(sg, P[g.oa + g.L + i], a.im);
-      }
-    c[r] = a;
-    if (o.fac[2 * r] != 0.0 || o.fac[2 * r + 1] != 0.0) mx = fmax(mx, a.re);
-  }
-  mx = block_max(mx, red);
-  if (!isfinite(mx)) mx = 0.0;
-  cd S = {0.0, 0.0};
-  for (int r = threadIdx.x; r < o.G; r += blockDim.x) {
-    const cd b = {o.fac[2 * r], o.fac[2 * r + 1]};
-    if (b.re == 0.0 && b.im == 0.0) continue;
-    const double e = exp(c[r].re - mx);
-    S = S + (o.cpx ? cd{e * cos(c[r].im), e * sin(c[r].im)} * b : cd{e * b.re, 0.0});
-  }
-  return log_of_sum(block_sum_cd(S, red), mx, o.cpx);
-}
-
 // ------------------------------------------------------------------ log psi
 // log psi of the spins s (LDS) by the whole workgroup: SL threads per row, U
 // hidden units at a time (sym_lanes).  A row's amplitude is
@@ -245,7 +207,15 @@ int sym_lanes(int G, int H, bool* four) {
   while (sl < WAVE && (*four ? 4 * sl : sl) < H && 2 * sl * G <= SYM_T) sl *= 2;
   return sl;
 }
-int sym_threads(int G, int SL, int most) { return std::min(most, (G * SL + WAVE - 1) / WAVE * WAVE); }
+size_t sym_rows_lds(const RbmGeom& g, int G, int T, int SL) {
+  return 8 * 8 + 32 * (size_t)G + 4 * (size_t)g.L + (size_t)(T / SL) * g.L + 16;
+}
+// Threads of the workgroup: no more than the rows fill or the LDS takes.
+int sym_threads(const RbmGeom& g, int G, int SL) {
+  int T = std::min(SYM_T, (G * SL + WAVE - 1) / WAVE * WAVE);
+  while (T > WAVE && sym_rows_lds(g, G, T, SL) > 160 * 1024) T -= WAVE;
+  return T;
+}
 
 // A workgroup per configuration.  FP64 issue (exp and sincos of every theta)
 // sets its time: 4096 samples, 16 sites x 32 units, 64 elements: 589 us with
@@ -269,9 +239,6 @@ __global__ void __launch_bounds__(SYM_T, 2) sym_rbm_forward(RbmGeom g, SymGeom o
     }
   }
 }
-size_t sym_rows_lds(const RbmGeom& g, int G, int T, int SL) {
-  return 8 * 8 + 32 * (size_t)G + 4 * (size_t)g.L + (size_t)(T / SL) * g.L + 16;
-}
 
 // ------------------------------------------------------------------ local energies
 // A workgroup per configuration.  The orbit in chunks of RC rows: four (eight,
@@ -288,6 +255,7 @@ template <bool CPX, int RC, bool TAB>
 __global__ void __launch_bounds__(SYM_T, 2) sym_rbm_eloc(RbmGeom g, SymGeom o, const double* __restrict__ P,
                                                          OpDev op, RbmTab tab, const int32_t* __restrict__ cfg,
                                                          const double* __restrict__ lps, int64_t n, int nstr,
+                                                         const double* __restrict__ part, int K,
                                                          double* __restrict__ out) {
   typedef typename num_of<CPX>::type T;
   extern __shared__ double lds[];
@@ -306,7 +274,15 @@ __global__ void __launch_bounds__(SYM_T, 2) sym_rbm_eloc(RbmGeom g, SymGeom o, c
   unsigned short* inv = (unsigned short*)(s + L);  // [RC][L]: position of a site in the row
   unsigned char* rb = (unsigned char*)(inv + RC * L);  // [RC][L]
   const int nl = tab.lead[0];
-  if (!sym_ok(g, o, tab, lane)) return;  // sym_slow_eloc's
+  if (!sym_ok(g, o, tab, lane)) {  // sym_rows_eloc's
+    if (K > 1)
+      for (int64_t q = blockIdx.x * (int64_t)SYM_T + tid; q < 2 * n; q += (int64_t)gridDim.x * SYM_T) {
+        double v = 0.0;
+        for (int k = 0; k < K; ++k) v += part[2 * n * k + q];
+        out[q] = v;
+      }
+    return;
+  }
   if (TAB)
     for (int t = tid; t < 2 * H * L; t += SYM_T) he[t] = ((const T*)tab.he)[t];
   for (int64_t q = blockIdx.x; q < n; q += gridDim.x) {
@@ -504,7 +480,7 @@ __global__ void __launch_bounds__(MAXT, MAXT == 256 ? 3 : MAXT == 512 ? 2 : 4) s
   int32_t* s = (int32_t*)(me + (TAB ? (size_t)2 * L * HP : 0));
   unsigned short* inv = (unsigned short*)(s + L);  // [G][L]: 2 * position + (row holds the flipped spin)
   unsigned char* rb = (unsigned char*)(inv + (size_t)G * L);  // [G][L] spins of the rows (refresh only)
-  if (!sym_ok(g, o, tab, lane)) return;  // sym_slow_mc's
+  if (!sym_ok(g, o, tab, lane)) return;  // sym_rows_mc's
   for (int i = tid; i < L; i += nt) s[i] = walkers[(int64_t)chain * L + i] > 0;
   for (int t = tid; t < 2 * L; t += nt) {
     const double* pq = tab.site + 8 * (int64_t)(t / 2) + 2 + 2 * (t % 2);
@@ -650,84 +626,95 @@ size_t sym_mc_lds(const RbmGeom& g, int G, bool tabl) {
 }
 
 // ------------------------------------------------------------------ parameters out of range, other maps
-// Row by row with rbm.hpp's log-cosh, one configuration or chain per
-// workgroup; these kernels return at once where the resident ones above work
-// (and the other way round), so neither carries the other's registers.
-__global__ void __launch_bounds__(SYM_T) sym_slow_eloc(RbmGeom g, SymGeom o, const double* __restrict__ P, OpDev op,
-                                                       RbmTab tab, const int32_t* __restrict__ cfg,
-                                                       const double* __restrict__ lps, int64_t n,
-                                                       double* __restrict__ out) {
+// log psi of every configuration from scratch (block_logpsi), one configuration
+// or chain per workgroup; these kernels return at once where the resident ones
+// above work (and the other way round), so neither carries the other's
+// registers.  Against a launch per step over materialised rows (4096 samples or
+// 1024 chains x 128 proposals, one |Re W| = 90): 16 x 32, 64 elements E_loc
+// 17.8 -> 3.9 ms, chains 20.3 -> 5.3; 64 x 200, two elements 30.1 -> 11.2, 8.9
+// -> 4.2.
+// Few samples: the strings over gridDim.y workgroups each, whose sums [K][n]
+// sym_rbm_eloc, launched behind, adds up (16 samples of 64 x 200, two elements:
+// 1746 us with one workgroup a sample, 238 so; 659 with materialised rows).
+template <bool CPX, int U>
+__global__ void __launch_bounds__(SYM_T, 2) sym_rows_eloc(RbmGeom g, SymGeom o, const double* __restrict__ P, OpDev op,
+                                                          RbmTab tab, int SL, const int32_t* __restrict__ cfg,
+                                                          const double* __restrict__ lps, int64_t n,
+                                                          double* __restrict__ out) {
   extern __shared__ double lds[];
   if (sym_ok(g, o, tab, threadIdx.x % WAVE)) return;
-  cd* c = (cd*)(lds + 8);
-  int32_t* s = (int32_t*)(c + o.G);
+  out += 2 * n * blockIdx.y;
+  double* red = lds;
+  cd* lin = (cd*)(red + 8);
+  cd* dd = lin + o.G;
+  int32_t* s = (int32_t*)(dd + o.G);
+  unsigned char* rb = (unsigned char*)(s + g.L);
   for (int64_t q = blockIdx.x; q < n; q += gridDim.x) {
-    __syncthreads();
-    for (int i = threadIdx.x; i < g.L; i += SYM_T) s[i] = cfg[q * g.L + i];
-    __syncthreads();
-    cd acc = {0.0, 0.0};
     const int32_t* cq = cfg + q * g.L;
+    for (int i = threadIdx.x; i < g.L; i += blockDim.x) s[i] = cq[i];
+    cd acc = {0.0, 0.0};
     const cd dsum = diag_sum(op, cq);
-    for (int j = 0; j < op.num_ops; ++j) {
+    for (int j = blockIdx.y; j < op.num_ops; j += gridDim.y) {
       int sites[MAXLEN], vals[MAXLEN], nch;
       const cd m = merged_m(op, j, apply_string(op, j, cq, sites, vals, nch), dsum);
       if (!nonzero(m)) continue;
-      __syncthreads();
+      __syncthreads();  // s is set
       if (threadIdx.x == 0)
-        for (int k = 0; k < nch; ++k) s[sites[k]] = 1 - s[sites[k]];
-      __syncthreads();
-      acc = acc + m * cexp(slow_logpsi(g, o, P, s, c, lds) - cd{lps[2 * q], lps[2 * q + 1]});
-      __syncthreads();
+        for (int k = 0; k < nch; ++k) s[sites[k]] = vals[k];
+      const cd lp = block_logpsi<CPX, U, 0>(g, o, P, s, SL, lin, dd, rb, red);
+      acc = acc + m * cexp(lp - cd{lps[2 * q], lps[2 * q + 1]});
       if (threadIdx.x == 0)
-        for (int k = 0; k < nch; ++k) s[sites[k]] = 1 - s[sites[k]];
-      __syncthreads();
+        for (int k = 0; k < nch; ++k) s[sites[k]] = cq[sites[k]];
     }
     if (threadIdx.x == 0) {
       out[2 * q] = acc.re;
       out[2 * q + 1] = acc.im;
     }
+    __syncthreads();
   }
 }
 
-__global__ void __launch_bounds__(SYM_T) sym_slow_mc(RbmGeom g, SymGeom o, const double* __restrict__ P, jv_mc_args a,
-                                                     RbmTab tab, int32_t* __restrict__ walkers,
-                                                     int32_t* __restrict__ configs, int64_t* __restrict__ counters) {
+template <bool CPX, int U>
+__global__ void __launch_bounds__(SYM_T, 2) sym_rows_mc(RbmGeom g, SymGeom o, const double* __restrict__ P, jv_mc_args a,
+                                                        RbmTab tab, int SL, int32_t* __restrict__ walkers,
+                                                        int32_t* __restrict__ configs, int64_t* __restrict__ counters) {
   extern __shared__ double lds[];
   if (sym_ok(g, o, tab, threadIdx.x % WAVE)) return;
-  const int tid = threadIdx.x, chain = blockIdx.x;
-  cd* c = (cd*)(lds + 8);
-  int32_t* s = (int32_t*)(c + o.G);
-  for (int i = tid; i < g.L; i += SYM_T) s[i] = walkers[(int64_t)chain * g.L + i];
-  __syncthreads();
-  double lacc = a.mu * slow_logpsi(g, o, P, s, c, lds).re;
+  const int tid = threadIdx.x, nt = blockDim.x, chain = blockIdx.x;
+  double* red = lds;
+  cd* lin = (cd*)(red + 8);
+  cd* dd = lin + o.G;
+  int32_t* s = (int32_t*)(dd + o.G);
+  unsigned char* rb = (unsigned char*)(s + g.L);
+  for (int i = tid; i < g.L; i += nt) s[i] = walkers[(int64_t)chain * g.L + i];
+  double lacc = a.mu * block_logpsi<CPX, U, 0>(g, o, P, s, SL, lin, dd, rb, red).re;
   const int total = a.therm_steps + a.samples_per_chain * a.sweep_steps;
   int64_t nacc = 0;
   for (int step = 0; step < total; ++step) {
     int site;
     double u;
     mc_draw(a.seed, (uint32_t)step, (uint32_t)chain, a.call_index, a.stream, g.L, site, u);
-    __syncthreads();
     if (tid == 0) s[site] ^= 1;
-    __syncthreads();
-    const double lnew = a.mu * slow_logpsi(g, o, P, s, c, lds).re;
+    const double lnew = a.mu * block_logpsi<CPX, U, 0>(g, o, P, s, SL, lin, dd, rb, red).re;
     const bool acc = u < exp(lnew - lacc);
-    __syncthreads();
     if (tid == 0 && !acc) s[site] ^= 1;
-    __syncthreads();
     if (acc) lacc = lnew;
     nacc += acc;
     const int k = step + 1 - a.therm_steps;
-    if (k > 0 && k % a.sweep_steps == 0)
-      for (int i = tid; i < g.L; i += SYM_T)
+    if (k > 0 && k % a.sweep_steps == 0) {
+      __syncthreads();
+      for (int i = tid; i < g.L; i += nt)
         configs[((int64_t)(k / a.sweep_steps - 1) * a.num_chains + chain) * g.L + i] = s[i];
+      __syncthreads();
+    }
   }
-  for (int i = tid; i < g.L; i += SYM_T) walkers[(int64_t)chain * g.L + i] = s[i];
+  __syncthreads();
+  for (int i = tid; i < g.L; i += nt) walkers[(int64_t)chain * g.L + i] = s[i];
   if (tid == 0) {
     atomicAdd((unsigned long long*)&counters[0], (unsigned long long)total);
     atomicAdd((unsigned long long*)&counters[1], (unsigned long long)nacc);
   }
 }
-size_t sym_slow_lds(const RbmGeom& g, int G) { return 64 + 16 * (size_t)G + 4 * (size_t)g.L; }
 
 __global__ void sym_zero_counters(int64_t* c) {
   if (threadIdx.x < 2) c[threadIdx.x] = 0;
@@ -753,7 +740,7 @@ int sym_rbm_forward_launch(const jv_net* net, const double* params, const jv_orb
   SymGeom o;
   if (!sym_rbm_geom(net, orbit, g, o)) return JV_OK;
   bool four;
-  const int SL = sym_lanes(o.G, g.H, &four), T = sym_threads(o.G, SL, SYM_T);
+  const int SL = sym_lanes(o.G, g.H, &four), T = sym_threads(g, o.G, SL);
   const size_t lds = sym_rows_lds(g, o.G, T, SL);
   if (lds > 160 * 1024) return JV_OK;
 #define JV_SYM_FWD(CPX)                                                                  \
@@ -771,7 +758,7 @@ int sym_rbm_forward_launch(const jv_net* net, const double* params, const jv_orb
 
 int sym_rbm_eloc_launch(const jv_net* net, const double* params, const jv_orbit* orbit, const jv_optable* op,
                         const double* prefactor, const int32_t* configs, const double* lps, int64_t n, double* out,
-                        hipStream_t st, int slot0, bool* done) {
+                        hipStream_t st, int slot0, int slot1, bool* done) {
   *done = false;
   RbmGeom g;
   SymGeom o;
@@ -793,7 +780,10 @@ int sym_rbm_eloc_launch(const jv_net* net, const double* params, const jv_orbit*
       lds = b;
       break;
     }
-  if (!RC) return JV_OK;
+  bool four;
+  const int SL = sym_lanes(o.G, g.H, &four), T = sym_threads(g, o.G, SL);
+  const size_t rlds = sym_rows_lds(g, o.G, T, SL);
+  if (!RC || rlds > 160 * 1024) return JV_OK;
   RbmTab tab;
   int rc = build_rbm_tables(g, params, &d, false, true, st, slot0, &tab, o.map, o.G);
   if (rc) return rc;
@@ -804,13 +794,18 @@ int sym_rbm_eloc_launch(const jv_net* net, const double* params, const jv_orbit*
 #undef JV_SYM_ELO
   rc = set_lds_limit((const void*)fn, lds);
   if (rc) return rc;
+  const auto rf = g.cpx ? (four ? sym_rows_eloc<true, 4> : sym_rows_eloc<true, 1>)
+                        : (four ? sym_rows_eloc<false, 4> : sym_rows_eloc<false, 1>);
+  if ((rc = set_lds_limit((const void*)rf, rlds))) return rc;
+  const int K = n <= 256 ? std::min(d.num_ops, 512 / (int)n) : 1;
+  double* part = K > 1 ? (double*)stream_workspace(16 * (size_t)K * n, slot1, st) : out;
+  if (!part) return fail(JV_E_NOMEM, "jv_sym_eloc: workspace allocation failed");
+  hipLaunchKernelGGL(rf, dim3((unsigned)std::min<int64_t>(n, 512 * SYM_T / T), (unsigned)K), dim3((unsigned)T), rlds, st, g, o,
+                     params, d, tab, SL, configs, lps, n, part);
+  JV_LAUNCH_CHECK("sym_rows_eloc");
   hipLaunchKernelGGL(fn, dim3((unsigned)std::min<int64_t>(n, 4096)), dim3(SYM_T), lds, st, g, o, params, d, tab, configs,
-                     lps, n, nstr, out);
+                     lps, n, nstr, part, K, out);
   JV_LAUNCH_CHECK("sym_rbm_eloc");
-  if ((rc = set_lds_limit((const void*)sym_slow_eloc, sym_slow_lds(g, o.G)))) return rc;
-  hipLaunchKernelGGL(sym_slow_eloc, dim3((unsigned)std::min<int64_t>(n, 512)), dim3(SYM_T), sym_slow_lds(g, o.G), st, g,
-                     o, params, d, tab, configs, lps, n, out);
-  JV_LAUNCH_CHECK("sym_slow_eloc");
   *done = true;
   return JV_OK;
 }
@@ -836,7 +831,10 @@ int sym_rbm_mc_launch(const jv_net* net, const double* params, const jv_orbit* o
   if (!HT) return JV_OK;
   const bool tabl = sym_mc_lds(g, o.G, true) <= 64 * 1024;
   const size_t lds = sym_mc_lds(g, o.G, tabl);
-  if (lds > 160 * 1024) return JV_OK;
+  bool four;
+  const int rSL = sym_lanes(o.G, g.H, &four), rT = sym_threads(g, o.G, rSL);
+  const size_t rlds = sym_rows_lds(g, o.G, rT, rSL);
+  if (lds > 160 * 1024 || rlds > 160 * 1024) return JV_OK;
   RbmTab tab;
   int rc = build_rbm_tables(g, params, nullptr, true, false, st, slot0, &tab, o.map, o.G);
   if (rc) return rc;
@@ -853,10 +851,12 @@ int sym_rbm_mc_launch(const jv_net* net, const double* params, const jv_orbit* o
   hipLaunchKernelGGL(fn, dim3((unsigned)a.num_chains), dim3(T), lds, st, g, o, params, a, tab, SL, walkers,
                      configs, counters);
   JV_LAUNCH_CHECK("sym_rbm_mc");
-  if ((rc = set_lds_limit((const void*)sym_slow_mc, sym_slow_lds(g, o.G)))) return rc;
-  hipLaunchKernelGGL(sym_slow_mc, dim3((unsigned)a.num_chains), dim3(SYM_T), sym_slow_lds(g, o.G), st, g, o, params, a,
-                     tab, walkers, configs, counters);
-  JV_LAUNCH_CHECK("sym_slow_mc");
+  const auto rf = g.cpx ? (four ? sym_rows_mc<true, 4> : sym_rows_mc<true, 1>)
+                        : (four ? sym_rows_mc<false, 4> : sym_rows_mc<false, 1>);
+  if ((rc = set_lds_limit((const void*)rf, rlds))) return rc;
+  hipLaunchKernelGGL(rf, dim3((unsigned)a.num_chains), dim3((unsigned)rT), rlds, st, g, o, params, a, tab, rSL, walkers,
+                     configs, counters);
+  JV_LAUNCH_CHECK("sym_rows_mc");
   *done = true;
   return JV_OK;
 }
