@@ -167,6 +167,43 @@ def test_eloc_out_of_range(big):
     assert np.max(np.abs(e - ref) / np.abs(ref)) < TOL
 
 
+@pytest.mark.parametrize("cpx,L,H,vbias,op,n", [
+    (True, 5, 1, False, "tfim", 3), (False, 7, 65, False, "mixed", 9), (True, 9, 130, True, "long", 10),
+    (True, 6, 257, False, "xxz", 5), (False, 5, 900, False, "mixed", 7), (True, 4, 6, True, "mixed", 8200)])
+def test_eloc_out_of_range_sizes(cpx, L, H, vbias, op, n):
+    """The form for parameters out of range over units per lane, samples per
+    workgroup, real networks and strings of more than two sites."""
+    rng = np.random.default_rng(L * 1000 + H)
+    P = 0.3 / np.sqrt(L) * rng.normal(size=_num(cpx, L, H, True, vbias))
+    P[(2 if cpx else 1) * H] = 90.0
+    psi, opsi = _states(cpx, L, H, True, vbias, P)
+    Hd, Ho = OPS[op](L)
+    s = rng.integers(0, 2, size=(n, L)).astype(np.int32)
+    lpo = opsi(s)
+    e = to_np(Hd.get_O_loc(torch.as_tensor(s[None], device="cuda"), psi, torch.as_tensor(lpo[None], device="cuda")))[0]
+    ref = Ho.get_O_loc(s, opsi, lpo)
+    assert np.max(np.abs(e - ref)) < TOL * np.max(np.abs(ref))
+    big = np.abs(ref) > 1e-3 * np.max(np.abs(ref))
+    assert np.max(np.abs(e - ref)[big] / np.abs(ref)[big]) < 1e-10
+
+
+@pytest.mark.parametrize("cpx,L,H,vbias,mu", [
+    (True, 70, 1, False, 2.0), (False, 12, 65, False, 1.0), (True, 9, 128, True, 2.0), (True, 8, 256, False, 0.5),
+    (False, 6, 256, False, 0.0)])
+def test_chains_out_of_range_sizes(cpx, L, H, vbias, mu):
+    rng = np.random.default_rng(L * 100 + H)
+    P = 0.3 / np.sqrt(L) * rng.normal(size=_num(cpx, L, H, True, vbias))
+    P[(2 if cpx else 1) * H] = 90.0
+    psi, opsi = _states(cpx, L, H, True, vbias, P)
+    kw = dict(numChains=6, numSamples=24, thermalizationSweeps=5, sweepSteps=45, mu=mu)
+    ms = jv.sampler.MCSampler(psi, (L,), 17, updateProposer=jv.sampler.propose_spin_flip, **kw)
+    mo = osamp.MCSampler(opsi, (L,), 17, **kw)
+    for _ in range(2):
+        assert np.array_equal(to_np(ms.sample()[0])[0], mo.sample()[0])
+    assert np.array_equal(to_np(ms.states), mo.states)
+    assert abs(float(ms.acceptance_ratio()[0]) - float(np.ravel(mo.acceptance_ratio())[0])) < 1e-15
+
+
 def _hop_pair(L):
     """Hopping strings (they keep the number of up spins) and a diagonal one."""
     from vmc_jax_amd import operator as dop

@@ -80,7 +80,7 @@ __global__ void __launch_bounds__(512) batch_sample(const BatchInst* __restrict_
   const int w = __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE);
   const int chain = (blockIdx.x - I.wg[0]) * nw + w;
   if (chain >= I.a.num_chains) return;
-  const int64_t nacc = rbmq_mc(I.g, I.P, I.a, I.tab, I.walkers, I.configs, chain, lane, lds + (size_t)w * lds_per_wave);
+  const int64_t nacc = rbmq_mc_any(I.g, I.P, I.a, I.tab, I.walkers, I.configs, chain, lane, lds + (size_t)w * lds_per_wave);
   if (lane == 0) {
     const int total = I.a.therm_steps + I.a.samples_per_chain * I.a.sweep_steps;
     atomicAdd((unsigned long long*)&I.counters[0], (unsigned long long)total);

@@ -14,8 +14,9 @@
 // Range: the routines below are used when |Re theta_h| <= RBMQ_THETA for every
 // configuration and sum_h |Re W_ih| + |Re a_i| <= 150 / n for strings of n
 // sites (pre_j and the products over units then stay inside the double range);
-// rbm.hpp's log-cosh routines serve everything else.  The kernels read the two bounds from the table, so
-// no host synchronisation is needed and NaN parameters take the log route.
+// the rbmq_*_direct routines serve everything else.  The kernels read the two
+// bounds from the table, so no host synchronisation is needed and NaN
+// parameters count as out of range.
 #pragma once
 #include "rbm.hpp"
 
@@ -318,7 +319,7 @@ __host__ __device__ inline size_t rbmq_eloc_lds_doubles(const RbmGeom& g, int ns
   const size_t S = rbmq_tile(g, n), jp = rbmq_jp(nstr), cw = rbm_cw(g);
   return S * (2 * cw * g.H + 2 + 2 * jp + RBMQ_WAVES * cw * jp + (g.L + 1) / 2) + 2;
 }
-// ... of either form (rbm.hpp's log-cosh form serves what is out of range).
+// ... of any form.
 __host__ __device__ inline size_t rbmq_block_lds_doubles(const RbmGeom& g, int nstr, int64_t n) {
   const size_t log_form = (size_t)RBMQ_WAVES * 4 * g.H;
   if (g.H > RBMQ_MAX_H) return log_form;
@@ -640,9 +641,109 @@ __device__ inline void rbmq_eloc_tile(const RbmGeom& g, const double* __restrict
   }
 }
 
+// theta of unit h for the spins s and its value on the side where Re >= 0;
+// d = 1 + e^{-2 lin}, so that cosh(theta) = e^{lin} d / 2.
+__device__ inline void rbm_lin(cd th, cd& lin, cd& d) {
+  lin = th.re < 0.0 ? cd{-th.re, -th.im} : th;
+  d = plus1(cexp({-2.0 * lin.re, -2.0 * lin.im}));
+}
+__device__ inline void rbm_lin(double th, double& lin, double& d) {
+  lin = fabs(th);
+  d = 1.0 + exp(-2.0 * lin);
+}
+
+// O_loc of one sample by one wave for parameters out of the ratio form's range:
+// psi(s') = e^{sum lin'} prod d' per string, an exponential per hidden unit and
+// no logarithm (H <= RBMQ_MAX_H keeps the product in range whatever theta).
+// 2000 samples of 100 x 200: 3.0 ms with rbm.hpp's log-cosh form inside this
+// kernel, whose registers and LDS leave it half the waves, 1.53 so (1.74 in
+// eloc_rbm).  th: H complex (real) of LDS.
+template <bool CPX>
+__device__ inline void rbmq_eloc_direct(const RbmGeom& g, const double* __restrict__ P, const OpDev& op,
+                                        const int32_t* c, const double* lps_s, double* out_s, double* lds, int lane) {
+  typedef typename num_of<CPX>::type T;
+  T* th = (T*)lds;
+  const double* Wr = P + g.ow;
+  const double* Wi = Wr + (int64_t)g.L * g.H;
+  T lin0, prod;
+  set_one(prod);
+  lin0 = prod - prod;
+  wave_sync();  // the previous sample is done
+  for (int h = lane; h < g.H; h += WAVE) {
+    const cd t = rbm_theta(g, P, c, h);
+    T x, lin, d;
+    if constexpr (CPX) x = t;
+    else x = t.re;
+    th[h] = x;
+    rbm_lin(x, lin, d);
+    lin0 = lin0 + lin;
+    prod = mulc(prod, d);
+  }
+  cd base = to_cd(lin0);
+  if (g.oa >= 0)
+    for (int i = lane; i < g.L; i += WAVE) {
+      const double sg = (double)(2 * c[i] - 1);
+      base.re = fma(sg, P[g.oa + i], base.re);
+      base.im = fma(sg, P[g.oa + g.L + i], base.im);
+    }
+  // e^{base} prod d = psi(s) / e^{log psi given by the caller} (base.py:164)
+  base = {fma(-(double)g.H, LN2, wave_sum(base.re)) - lps_s[0], wave_sum(base.im) - lps_s[1]};
+  const T prod0 = wave_prod(prod);
+  wave_sync();
+  const cd dsum = diag_sum(op, c);
+  cd acc = {0.0, 0.0};
+  int sites[MAXLEN], vals[MAXLEN], nch;
+  for (int o = 0; o < op.num_ops; ++o) {
+    const cd m = merged_m(op, o, apply_string(op, o, c, sites, vals, nch), dsum);
+    if (!nonzero(m)) continue;
+    cd x = base;
+    T dp = prod0;
+    if (nch > 0) {
+      T dl;
+      set_one(dp);
+      dl = dp - dp;
+      for (int h = lane; h < g.H; h += WAVE) {
+        const T t0 = th[h];
+        cd t = to_cd(t0);
+        for (int j = 0; j < nch; ++j) {
+          const double f = 2.0 * (double)(vals[j] - c[sites[j]]);
+          const int64_t wi = (int64_t)sites[j] * g.H + h;
+          t.re = fma(f, Wr[wi], t.re);
+          if (CPX) t.im = fma(f, Wi[wi], t.im);
+        }
+        T lin, d, l0;
+        if constexpr (CPX) {
+          rbm_lin(t, lin, d);
+          l0 = t0.re < 0.0 ? cd{-t0.re, -t0.im} : t0;
+        } else {
+          rbm_lin(t.re, lin, d);
+          l0 = fabs(t0);
+        }
+        dl = dl + (lin - l0);
+        dp = mulc(dp, d);
+      }
+      const cd dc = to_cd(dl);
+      x.re += wave_sum(dc.re);
+      if (CPX) x.im += wave_sum(dc.im);
+      dp = wave_prod(dp);
+      if (g.oa >= 0)
+        for (int j = 0; j < nch; ++j) {
+          const double f = 2.0 * (double)(vals[j] - c[sites[j]]);
+          x.re = fma(f, P[g.oa + sites[j]], x.re);
+          x.im = fma(f, P[g.oa + g.L + sites[j]], x.im);
+        }
+    }
+    acc = acc + mulc(m, mulc(to_cd(dp), cexp(x)));
+  }
+  if (lane == 0) {
+    out_s[0] = acc.re;
+    out_s[1] = acc.im;
+  }
+}
+
 // Samples [s0, s0 + cnt) by one workgroup of RBMQ_WAVES waves, S at a time:
-// the ratio form where the parameters' range allows it, rbm.hpp's log-cosh
-// form otherwise (S = 0: always).
+// the ratio form where the parameters' range allows it, string by string
+// otherwise (S = 0: rbm.hpp's log-cosh form always).
 template <bool CPX, bool SMALL, int S>
 __device__ inline void rbmq_eloc_range(const RbmGeom& g, const double* __restrict__ P, const OpDev& op,
                                        const RbmTab& tab, const int32_t* __restrict__ cfg, int64_t s0, int64_t cnt,
@@ -658,6 +759,10 @@ __device__ inline void rbmq_eloc_range(const RbmGeom& g, const double* __restric
       }
       return;
     }
+    for (int64_t k = w; k < cnt; k += RBMQ_WAVES)
+      rbmq_eloc_direct<CPX>(g, P, op, cfg + (s0 + k) * g.L, lps + 2 * (s0 + k), out + 2 * (s0 + k),
+                            lds + (size_t)w * rbm_cw(g) * g.H, lane);
+    return;
   }
   for (int64_t k = w; k < cnt; k += RBMQ_WAVES)
     eloc_rbm_sample(g, P, op, cfg + (s0 + k) * g.L, lps + 2 * (s0 + k), out + 2 * (s0 + k),
@@ -826,21 +931,110 @@ __device__ inline int64_t rbmq_mc_chain(const RbmGeom& g, const double* __restri
   return nacc;
 }
 
-// The chain in the form the parameters' range and the sizes allow
-// (lds: mc_rbm_lds_doubles(g), used by the log-cosh form).
+// The chain for parameters out of that range, H <= RBMQ_MC_MAX_H: theta in LDS
+// (2 H doubles), |cosh theta|^2 = e^{2 a} q / 4 with a = |Re theta| and
+// q = |1 + e^{-2 theta}|^2 in [0, 4], so a proposal costs an exponential and a
+// cosine per unit, a sum of a' - a and a product of q', and no logarithm per
+// unit.  1024 chains x 320 proposals, 32 x 64: 609 us with rbm.hpp's log-cosh
+// form here, 467 so (541 in mc_rbm); 4096 chains, 8 x 8: 2.61 ms, 0.99 (1.54).
+template <bool CPX>
+__device__ inline int64_t rbmq_mc_direct(const RbmGeom& g, const double* __restrict__ P, const jv_mc_args& a,
+                                         int32_t* __restrict__ walkers, int32_t* __restrict__ configs, int chain,
+                                         int lane, double* lds) {
+  typedef typename num_of<CPX>::type T;
+  T* th = (T*)lds;
+  int32_t* s = (int32_t*)(lds + rbm_cw(g) * g.H);
+  const double* Wr = P + g.ow;
+  const double* Wi = Wr + (int64_t)g.L * g.H;
+  for (int i = lane; i < g.L; i += WAVE) s[i] = walkers[(int64_t)chain * g.L + i];
+  wave_sync();
+  auto q_of = [](T t) {
+    if constexpr (CPX) {
+      const double e = exp(-2.0 * fabs(t.re));
+      return 1.0 + fma(2.0 * e, cos(2.0 * t.im), e * e);
+    } else {
+      const double e = 1.0 + exp(-2.0 * fabs(t));
+      return e * e;
+    }
+  };
+  double Q;  // product of q over the units
+  auto refresh = [&]() {
+    double p = 1.0;
+    for (int h = lane; h < g.H; h += WAVE) {
+      const cd t = rbm_theta(g, P, s, h);
+      if constexpr (CPX) th[h] = t;
+      else th[h] = t.re;
+      p *= q_of(th[h]);
+    }
+    Q = wave_prod(p);
+  };
+  refresh();
+  auto moved = [&](int site, double d, int h) {
+    const int64_t wi = (int64_t)site * g.H + h;
+    if constexpr (CPX) return cd{fma(d, Wr[wi], th[h].re), fma(d, Wi[wi], th[h].im)};
+    else return fma(d, Wr[wi], th[h]);
+  };
+  int64_t nacc = 0;
+  const int total = a.therm_steps + a.samples_per_chain * a.sweep_steps;
+  for (int step = 0; step < total; ++step) {
+    int site;
+    double u;
+    mc_draw(a.seed, (uint32_t)step, (uint32_t)chain, a.call_index, a.stream, g.L, site, u);
+    const double d = -2.0 * (double)(2 * s[site] - 1);
+    double dl = 0.0, p = 1.0;
+    for (int h = lane; h < g.H; h += WAVE) {
+      const T t = moved(site, d, h);
+      dl += fabs(to_cd(t).re) - fabs(to_cd(th[h]).re);
+      p *= q_of(t);
+    }
+    dl = wave_sum(dl);
+    p = wave_prod(p);
+    if (g.oa >= 0) dl = fma(d, P[g.oa + site], dl);
+    // random.bernoulli(key, P), sampler.py:336-340
+    const bool acc = a.mu == 2.0 ? u < exp(2.0 * dl) * (p / Q) : u < exp(a.mu * fma(0.5, log(p / Q), dl));
+    if (acc) {
+      for (int h = lane; h < g.H; h += WAVE) th[h] = moved(site, d, h);
+      Q = p;
+      wave_sync();
+      if (lane == 0) s[site] ^= 1;
+      ++nacc;
+    }
+    wave_sync();
+    const int k = step + 1 - a.therm_steps;
+    if (k > 0 && k % a.sweep_steps == 0) {
+      const int64_t t = k / a.sweep_steps - 1;
+      int32_t* out = configs + (t * a.num_chains + chain) * g.L;
+      for (int i = lane; i < g.L; i += WAVE) out[i] = s[i];
+      refresh();
+      wave_sync();
+    }
+  }
+  for (int i = lane; i < g.L; i += WAVE) walkers[(int64_t)chain * g.L + i] = s[i];
+  return nacc;
+}
+
+// The chain in the form the parameters' range allows, sizes as rbmq_mc_fits
+// (lds: mc_rbm_lds_doubles(g), used out of range).
+template <bool CPX, int NH>
 __device__ inline int64_t rbmq_mc(const RbmGeom& g, const double* __restrict__ P, const jv_mc_args& a,
                                   const RbmTab& tab, int32_t* __restrict__ walkers, int32_t* __restrict__ configs,
                                   int chain, int lane, double* lds) {
-  if (rbmq_mc_fits(g) && rbmq_ok(g, tab, 2, lane)) {  // squared moduli: twice the exponent of one flip
-#define JV_RBMQ_MC(NHv)                                                                         \
-  return g.cpx ? rbmq_mc_chain<true, NHv>(g, P, a, tab, walkers, configs, chain, lane)          \
-               : rbmq_mc_chain<false, NHv>(g, P, a, tab, walkers, configs, chain, lane)
-    if (g.H <= 64) JV_RBMQ_MC(1);
-    if (g.H <= 128) JV_RBMQ_MC(2);
-    JV_RBMQ_MC(4);
+  if (rbmq_ok(g, tab, 2, lane))  // squared moduli: twice the exponent of one flip
+    return rbmq_mc_chain<CPX, NH>(g, P, a, tab, walkers, configs, chain, lane);
+  return rbmq_mc_direct<CPX>(g, P, a, walkers, configs, chain, lane, lds);
+}
+// The same for any sizes (the batch's instances differ).
+__device__ inline int64_t rbmq_mc_any(const RbmGeom& g, const double* __restrict__ P, const jv_mc_args& a,
+                                      const RbmTab& tab, int32_t* __restrict__ walkers, int32_t* __restrict__ configs,
+                                      int chain, int lane, double* lds) {
+  if (!rbmq_mc_fits(g)) return mc_rbm_chain(g, P, a, walkers, configs, chain, lane, lds);
+#define JV_RBMQ_MC(NHv)                                                                        \
+  return g.cpx ? rbmq_mc<true, NHv>(g, P, a, tab, walkers, configs, chain, lane, lds)          \
+               : rbmq_mc<false, NHv>(g, P, a, tab, walkers, configs, chain, lane, lds)
+  if (g.H <= 64) JV_RBMQ_MC(1);
+  if (g.H <= 128) JV_RBMQ_MC(2);
+  JV_RBMQ_MC(4);
 #undef JV_RBMQ_MC
-  }
-  return mc_rbm_chain(g, P, a, walkers, configs, chain, lane, lds);
 }
 
 }  // namespace jv

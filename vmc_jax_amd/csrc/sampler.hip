@@ -33,7 +33,11 @@ __global__ void __launch_bounds__(256) mc_rbm(RbmGeom g, const double* __restric
   }
 }
 
-// The same with ratio tables (rbmq_mc in rbmq.hpp).
+// The same with ratio tables (rbmq_mc in rbmq.hpp, for sizes that rbmq_mc_fits
+// allows).  A kernel per NH: the registers of four units a lane would leave
+// 4096 chains of 8 x 8 a wave per SIMD (320 proposals: 527 us, 332 so; out of
+// range 1.82 ms, 0.99 so).
+template <bool CPX, int NH>
 __global__ void __launch_bounds__(256, 1) mc_rbmq(RbmGeom g, const double* __restrict__ P, jv_mc_args a, RbmTab tab,
                                                   int32_t* __restrict__ walkers, int32_t* __restrict__ configs,
                                                   int64_t* __restrict__ counters) {
@@ -42,7 +46,7 @@ __global__ void __launch_bounds__(256, 1) mc_rbmq(RbmGeom g, const double* __res
   const int w = __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE);
   const int chain = blockIdx.x * nw + w;
   if (chain >= a.num_chains) return;
-  const int64_t nacc = rbmq_mc(g, P, a, tab, walkers, configs, chain, lane, lds + (size_t)w * mc_rbm_lds_doubles(g));
+  const int64_t nacc = rbmq_mc<CPX, NH>(g, P, a, tab, walkers, configs, chain, lane, lds + (size_t)w * mc_rbm_lds_doubles(g));
   if (lane == 0) {
     const int total = a.therm_steps + a.samples_per_chain * a.sweep_steps;
     atomicAdd((unsigned long long*)&counters[0], (unsigned long long)total);
@@ -644,19 +648,22 @@ int jv_mc_sample(const jv_net* net, const double* params, const jv_mc_args* args
     const bool q = rbmq_mc_fits(rg) && !stream_capturing(st);
     const int nw = q && a.num_chains <= 256 ? 1 : 4;
     size_t lds = nw * 8 * mc_rbm_lds_doubles(rg);
-    int rc = set_lds_limit(q ? (const void*)mc_rbmq : (const void*)mc_rbm, lds);
+#define JV_RBMQ_MC(CPX) (rg.H <= 64 ? mc_rbmq<CPX, 1> : rg.H <= 128 ? mc_rbmq<CPX, 2> : mc_rbmq<CPX, 4>)
+    const auto fn = rg.cpx ? JV_RBMQ_MC(true) : JV_RBMQ_MC(false);
+#undef JV_RBMQ_MC
+    int rc = set_lds_limit(q ? (const void*)fn : (const void*)mc_rbm, lds);
     if (rc) return rc;
     if (q) {
       RbmTab tab;
       rc = build_rbm_tables(rg, params, nullptr, true, false, st, WS_RBMQ_MC, &tab);
       if (rc) return rc;
-      hipLaunchKernelGGL(mc_rbmq, dim3((unsigned)((a.num_chains + nw - 1) / nw)), dim3(64 * nw), lds, st, rg, params,
+      hipLaunchKernelGGL(fn, dim3((unsigned)((a.num_chains + nw - 1) / nw)), dim3(64 * nw), lds, st, rg, params,
                          a, tab, walkers, configs, counters);
       JV_LAUNCH_CHECK("mc_rbmq");
     } else {
-    hipLaunchKernelGGL(mc_rbm, dim3((unsigned)((a.num_chains + nw - 1) / nw)), dim3(64 * nw), lds, st, rg,
-                       params, a, walkers, configs, counters);
-    JV_LAUNCH_CHECK("mc_rbm");
+      hipLaunchKernelGGL(mc_rbm, dim3((unsigned)((a.num_chains + nw - 1) / nw)), dim3(64 * nw), lds, st, rg, params, a,
+                         walkers, configs, counters);
+      JV_LAUNCH_CHECK("mc_rbm");
     }
   } else if (make_cnn_geom(net, cg) && win_ok(cg) && cnn_cmax(cg) > 0 && mc_win_cs(cg) > 0 &&
              mc_win_bytes(cg, cnn_cmax(cg), mc_win_cs(cg), net->precision == JV_PREC_MIXED ? 4 : 8) <= 160 * 1024) {
