@@ -400,6 +400,25 @@ def test_sym_out_of_range(cpx, L, H, names, op, mu):
     assert float(ms.acceptance_ratio()[0]) == float(np.ravel(mo.acceptance_ratio())[0])
 
 
+@pytest.mark.parametrize("cpx,seed", [(True, 5), (True, 6), (False, 7)])
+def test_sym_chain_rows_far_apart(cpx, seed):
+    """Two rows (a chain and its mirror image) whose weights differ by e^{860}
+    at the start, parameters in range: the lighter one still counts once flips
+    during the thermalisation have made it the heavier."""
+    L, H = 24, 16
+    rng = np.random.default_rng(seed)
+    k = 2 if cpx else 1
+    P = 0.01 * rng.normal(size=_num(cpx, L, H, True, False))
+    P[k * H:k * H + 12 * H] = 4.5  # Re W of the left half
+    psi, opsi = _sym_states(cpx, L, H, ("reflection",), P)
+    init = np.array([1] * 12 + [0, 1] * 6, dtype=np.int32)
+    kw = dict(numChains=4, numSamples=8, thermalizationSweeps=40, sweepSteps=50, mu=0.01, initState=init)
+    ms = jv.sampler.MCSampler(psi, (L,), seed, updateProposer=jv.sampler.propose_spin_flip, **kw)
+    mo = osamp.MCSampler(opsi, (L,), seed, **kw)
+    assert np.array_equal(to_np(ms.sample()[0])[0], mo.sample()[0])
+    assert float(ms.acceptance_ratio()[0]) == float(np.ravel(mo.acceptance_ratio())[0])
+
+
 @pytest.mark.parametrize("cpx", [True, False])
 def test_sym_rows_that_are_no_permutation(cpx):
     """An orbit element may read a site twice, or never: (g s)_i = s_{m_i} all

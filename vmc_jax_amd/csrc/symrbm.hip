@@ -452,6 +452,18 @@ size_t sym_eloc_lds(const RbmGeom& g, int RC, bool tabl, int nstr) {
 }
 
 // ------------------------------------------------------------------ Metropolis chains
+// Moves the power of two of a row's weight into its exponent (0, infinities
+// and NaN stay as they are).
+__device__ inline void scale_row(cd& wt, int& ex) {
+  const double m = fmax(fabs(wt.re), fabs(wt.im));
+  if (m > 0.0 && m < INFINITY) {
+    int e;
+    (void)frexp(m, &e);
+    wt = {ldexp(wt.re, -e), ldexp(wt.im, -e)};
+    ex += e;
+  }
+}
+
 // A workgroup per chain (sampler.py:264-367), SL threads per row, HT hidden
 // units each: e and alpha live in registers, the spins and the flipped
 // position of every row in LDS.  A proposal: one product per row, a sum over
@@ -511,7 +523,11 @@ __global__ void __launch_bounds__(MAXT, MAXT == 256 ? 3 : MAXT == 512 ? 2 : 4) s
   const int rc = min(r, G - 1);
   const cd b = {o.fac[2 * rc], o.fac[2 * rc + 1]};
   T e[HT], al[HT];
-  cd wt = {0.0, 0.0};   // b_g psi_net(g s) up to a common factor (every lane of the row)
+  // b_g psi_net(g s) up to a common factor, wt 2^ex (every lane of the row): rows
+  // differ by more than the double range, and a row that counts for nothing now
+  // may count for everything some flips later
+  cd wt = {0.0, 0.0};
+  int ex = 0;
   double cur2 = 0.0;    // |sum_g wt|^2
   auto refresh = [&]() __attribute__((always_inline)) {
     __syncthreads();
@@ -547,8 +563,12 @@ __global__ void __launch_bounds__(MAXT, MAXT == 256 ? 3 : MAXT == 512 ? 2 : 4) s
     const bool on = mine && (b.re != 0.0 || b.im != 0.0);
     double mx = block_max(on ? li.re : -INFINITY, red);
     if (!isfinite(mx)) mx = 0.0;
-    wt = on ? mulc(mulc(cexp({fma(-(double)H, LN2, li.re - mx), li.im}), to_cd(recip(dp))), b) : cd{0.0, 0.0};
-    const cd S = block_sum_cd(sl == 0 ? wt : cd{0.0, 0.0}, red);
+    const double x = fma(-(double)H, LN2, li.re - mx), k = on ? rint(x * 1.4426950408889634) : 0.0;
+    const double xr = fma(-k, 2.31904681384629955842e-17, fma(-k, 6.93147180559945286227e-01, x));
+    wt = on ? mulc(mulc(cexp({xr, li.im}), to_cd(recip(dp))), b) : cd{0.0, 0.0};
+    ex = (int)k;
+    scale_row(wt, ex);
+    const cd S = block_sum_cd(sl == 0 ? cd{ldexp(wt.re, ex), ldexp(wt.im, ex)} : cd{0.0, 0.0}, red);
     cur2 = !o.cpx && S.re < 0.0 ? NAN : norm2(S);
   };
   refresh();
@@ -579,7 +599,8 @@ __global__ void __launch_bounds__(MAXT, MAXT == 256 ? 3 : MAXT == 512 ? 2 : 4) s
     }
     for (int m = 1; m < SL; m *= 2) pr = mulc(pr, shfl_xor(pr, m));
     const cd z = mulc(to_cd(pr), mulc(pre[2 * pos + v], wt));
-    const double zr = wave_sum(mine && sl == 0 ? z.re : 0.0), zi = o.cpx ? wave_sum(mine && sl == 0 ? z.im : 0.0) : 0.0;
+    const double zr = wave_sum(mine && sl == 0 ? ldexp(z.re, ex) : 0.0);
+    const double zi = o.cpx ? wave_sum(mine && sl == 0 ? ldexp(z.im, ex) : 0.0) : 0.0;
     cd* slot = part + 16 * (step & 1);
     if (lane == 0) slot[tid / WAVE] = {zr, zi};
     __syncthreads();
@@ -596,6 +617,7 @@ __global__ void __launch_bounds__(MAXT, MAXT == 256 ? 3 : MAXT == 512 ? 2 : 4) s
       }
       const double sc = new2 > 0.0 ? 1.0 / sqrt(new2) : 1.0;
       wt = {z.re * sc, z.im * sc};
+      scale_row(wt, ex);
       cur2 = new2 > 0.0 ? 1.0 : 0.0;
       if (lane == (site & 63)) sp ^= 1u << (site >> 6);
     }
