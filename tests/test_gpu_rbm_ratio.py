@@ -149,6 +149,24 @@ def test_eloc_string_that_flips_nothing(L, H, n, where):
     assert np.max(np.abs(e - ref) / np.abs(ref)) < TOL
 
 
+def test_eloc_more_tiles_than_a_launch_has_workgroups():
+    """2^24 tiles and a few samples: as many workgroups of 256 threads are more
+    threads than a launch takes."""
+    L, H, n = 2, 1, (1 << 24) * 8 + 37
+    rng = np.random.default_rng(2)
+    P = 0.3 * rng.normal(size=_num(False, L, H, True, False))
+    psi, opsi = _states(False, L, H, True, False, P)
+    Hd, Ho = tfim_pair((L,), -1.0, -0.7)
+    basis = np.array([[0, 0], [0, 1], [1, 0], [1, 1]], dtype=np.int32)
+    table = torch.as_tensor(Ho.get_O_loc(basis, opsi, np.zeros(4)), device="cuda").to(torch.complex128)
+    s = torch.randint(0, 2, (1, n, L), dtype=torch.int32, device="cuda")
+    e = Hd.get_O_loc(s, psi, torch.zeros((1, n), dtype=torch.complex128, device="cuda"))[0]
+    for a in range(0, n, 1 << 24):
+        b = min(n, a + (1 << 24))
+        ref = table[(2 * s[0, a:b, 0] + s[0, a:b, 1]).long()]
+        assert float((e[a:b] - ref).abs().max()) < TOL
+
+
 @pytest.mark.parametrize("big", [10.0, 60.0])
 def test_eloc_out_of_range(big):
     """A site whose summed |Re W| (80, 480) or a unit whose |Re theta| leaves the

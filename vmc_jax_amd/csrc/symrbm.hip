@@ -850,7 +850,8 @@ int sym_rbm_mc_launch(const jv_net* net, const double* params, const jv_orbit* o
       SL = sl;
     }
   }
-  if (!HT) return JV_OK;
+  const int64_t most = (1 << 22) - 1;  // workgroups of 1024 threads in a launch (fewer than 2^32 threads)
+  if (!HT || a.num_chains > most) return JV_OK;
   const bool tabl = sym_mc_lds(g, o.G, true) <= 64 * 1024;
   const size_t lds = sym_mc_lds(g, o.G, tabl);
   bool four;
