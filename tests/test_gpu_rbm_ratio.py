@@ -321,6 +321,18 @@ def test_chains(cpx, L, H, bias, vbias, mu, big):
     assert abs(float(ms.acceptance_ratio()[0]) - float(np.ravel(mo.acceptance_ratio())[0])) < 1e-15
 
 
+def _xxz_bond(L):
+    """XXZ on one bond."""
+    from vmc_jax_amd import operator as dop
+    out = []
+    for o in (dop, oop):
+        H = o.BranchFreeOperator()
+        for c, a in ((1.0, o.Sx), (1.0, o.Sy), (0.5, o.Sz)):
+            H.add(o.scal_opstr(c, (a(1), a(2))))
+        out.append(H)
+    return out
+
+
 def _sym_states(cpx, L, H, names, P, **kw):
     import warnings
 
@@ -416,6 +428,28 @@ def test_sym_out_of_range(cpx, L, H, names, op, mu):
         assert np.array_equal(to_np(ms.sample()[0])[0], mo.sample()[0])
     assert np.array_equal(to_np(ms.states), mo.states)
     assert float(ms.acceptance_ratio()[0]) == float(np.ravel(mo.acceptance_ratio())[0])
+
+
+def test_sym_eloc_negative_sums():
+    """A real network's negative sums have no logarithm: the local energy is NaN
+    where any string with a matrix element leads to one, also where it cancels
+    against another string with the same s' (X X against Y Y)."""
+    L, H = 7, 5
+    P = 0.5 * np.random.default_rng(3).normal(size=_num(False, L, H, True, False))
+    psi, opsi = _sym_states(False, L, H, ("reflection",), P, reflection_factor=-1.0)
+    s = ((np.arange(2 ** L)[:, None] >> np.arange(L)) & 1).astype(np.int32)
+    sp = s.copy()
+    sp[:, 1:3] ^= 1
+    asym = np.any(s != s[:, ::-1], axis=1) & np.any(sp != sp[:, ::-1], axis=1)  # sums that do not cancel
+    s = s[asym & np.isfinite(opsi(s))]
+    lpo = opsi(s)
+    Hd, Ho = _xxz_bond(L)
+    e = to_np(Hd.get_O_loc(torch.as_tensor(s[None], device="cuda"), psi, torch.as_tensor(lpo[None], device="cuda")))[0]
+    ref = Ho.get_O_loc(s, opsi, lpo)
+    assert np.isnan(ref).any() and np.isfinite(ref).any()
+    assert np.array_equal(np.isnan(e), np.isnan(ref))
+    ok = np.isfinite(ref)
+    assert np.max(np.abs(e - ref)[ok]) < TOL * np.max(np.abs(ref[ok]))
 
 
 @pytest.mark.parametrize("cpx,seed", [(True, 5), (True, 6), (False, 7)])

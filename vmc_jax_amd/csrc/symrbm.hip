@@ -269,7 +269,7 @@ __global__ void __launch_bounds__(SYM_T, 2) sym_rbm_eloc(RbmGeom g, SymGeom o, c
   cd* wt = (cd*)(he + (TAB ? (size_t)2 * H * L : 0));  // [RC]
   cd* mel = wt + RC;                      // [nstr] matrix elements
   cd* sum = mel + nstr;                   // [4 gq] sums over the orbit
-  int32_t* site = (int32_t*)(sum + 4 * gq);  // [4 gq][2] changed sites, -1: none
+  int32_t* site = (int32_t*)(sum + 4 * gq);  // [4 gq][2] changed sites, negative: none
   int32_t* s = site + 8 * gq;
   unsigned short* inv = (unsigned short*)(s + L);  // [RC][L]: position of a site in the row
   unsigned char* rb = (unsigned char*)(inv + RC * L);  // [RC][L]
@@ -299,7 +299,7 @@ __global__ void __launch_bounds__(SYM_T, 2) sym_rbm_eloc(RbmGeom g, SymGeom o, c
       }
     for (int j = tid; j < 4 * gq; j += SYM_T) {
       cd m = {0.0, 0.0};
-      int sa = -1, sb = -1;
+      int sa = -2, sb = -1;  // -2: no string applies to this sample
       if (j < nl) {
         const int code = tab.lead[1 + j], st = code >> 4, fol = code & 15;
         for (int f = 0; f <= fol; ++f) {
@@ -431,8 +431,8 @@ __global__ void __launch_bounds__(SYM_T, 2) sym_rbm_eloc(RbmGeom g, SymGeom o, c
     // a negative sum of real terms has no logarithm (jax's logsumexp): NaN
     cd acc = {0.0, 0.0};
     for (int j = tid; j < nl; j += SYM_T) {
-      const cd m = mel[j];
-      if (m.re == 0.0 && m.im == 0.0) continue;
+      if (site[2 * j] == -2) continue;
+      const cd m = mel[j];  // 0 where strings cancel; a NaN counts all the same
       acc = acc + (!o.cpx && sum[j].re < 0.0 ? cd{NAN, NAN} : mulc(m, sum[j]));
     }
     if (tid == 0 && nonzero(ds)) acc = acc + (!o.cpx && base.re < 0.0 ? cd{NAN, NAN} : mulc(ds, base));
