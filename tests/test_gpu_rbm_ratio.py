@@ -532,3 +532,45 @@ def test_eloc_in_a_captured_graph():
         graph.replay()
         torch.cuda.synchronize()
         assert _rel(to_np(out), to_np(eager)) < TOL
+
+
+@pytest.mark.parametrize("n", [50, 300])
+def test_sym_calls_in_a_captured_graph(n):
+    """Captured on a stream that no call has used before (a warm call on another
+    one has sized the scratch memory); larger calls between the replays leave
+    the captured ones' buffers alone.  n: with and without strings spread over
+    several workgroups."""
+    L, H = 8, 6
+    rng = np.random.default_rng(9)
+    Hd, Ho = xxz_pair(L, 0.6)
+    P = 0.1 * rng.normal(size=_num(True, L, H, True, False))
+    psi, opsi = _sym_states(True, L, H, ALL, P)
+    s = rng.integers(0, 2, size=(n, L)).astype(np.int32)
+    sd = torch.as_tensor(s[None], device="cuda")
+    kw = dict(numChains=6, numSamples=24, thermalizationSweeps=2, sweepSteps=20)
+    ms = jv.sampler.MCSampler(psi, (L,), 17, updateProposer=jv.sampler.propose_spin_flip, **kw)
+    first = to_np(ms.sample()[0]).copy()
+    lp = psi(sd).clone()
+    eager = Hd.get_O_loc(sd, psi, lp).clone()
+    ms.callIndex = 0
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph, stream=torch.cuda.Stream()):
+        e = Hd.get_O_loc(sd, psi, lp)
+        lp2 = psi(sd)
+        c = ms.sample()[0]
+    big, _ = _sym_states(True, 20, 40, ALL, 0.05 * rng.normal(size=_num(True, 20, 40, True, False)))
+    Hb, _ = tfim_pair((20,), -1.0, -0.7)
+    sb = torch.as_tensor(rng.integers(0, 2, size=(1, 30, 20)).astype(np.int32), device="cuda")
+    for _ in range(3):
+        Hb.get_O_loc(sb, big, big(sb))
+        torch.cuda.synchronize()
+        e.zero_()
+        lp2.zero_()
+        ms.states.zero_()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(e, eager)
+        assert torch.equal(lp2, lp)
+        assert np.array_equal(to_np(c), first)
+    assert _rel(to_np(e)[0], Ho.get_O_loc(s, opsi, opsi(s))) < TOL

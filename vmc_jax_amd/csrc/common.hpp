@@ -30,6 +30,8 @@ void* workspace(size_t bytes, int slot);
 // The same per stream (WS_STREAMS slots from slot0 on).
 constexpr int WS_STREAMS = 8;
 void* stream_workspace(size_t bytes, int slot0, hipStream_t st);
+// The same for calls that may be captured (one more slot behind those).
+void* capturable_workspace(size_t bytes, int slot0, hipStream_t st);
 bool stream_capturing(hipStream_t st);
 
 // Optional event timing of named kernels (jv_timer_enable / jv_timer_read).

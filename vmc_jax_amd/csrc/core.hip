@@ -34,6 +34,8 @@ struct DeviceState {
   hipStream_t ws_stream[WS_STREAMS] = {};  // owners of stream_workspace's buffers
   uint64_t ws_used[WS_STREAMS] = {};       // time of last use (0: free)
   uint64_t ws_clock = 0;
+  std::vector<bool> kept;                // slots whose buffer a captured graph may read
+  std::vector<std::pair<void*, size_t>> retired;  // such buffers, outgrown
   hipEvent_t ev[2] = {nullptr, nullptr};
 };
 // Workspaces and solver handles are per host thread and device, so threads
@@ -54,8 +56,11 @@ void release(DeviceState& s, int d) {
   (void)hipDeviceSynchronize();
   for (void* p : s.ptr)
     if (p) (void)hipFree(p);
+  for (auto& r : s.retired) (void)hipFree(r.first);
   s.ptr.clear();
   s.size.clear();
+  s.kept.clear();
+  s.retired.clear();
   for (auto& u : s.ws_used) u = 0;
   if (s.blas) rocblas_destroy_handle(s.blas);
   s.blas = nullptr;
@@ -151,8 +156,13 @@ void* workspace(size_t bytes, int slot) {
   }
   if (s.size[slot] < bytes) {
     if (s.ptr[slot]) {
-      (void)hipDeviceSynchronize();
-      (void)hipFree(s.ptr[slot]);
+      if (slot < (int)s.kept.size() && s.kept[slot]) {
+        s.retired.push_back({s.ptr[slot], s.size[slot]});
+        s.kept[slot] = false;
+      } else {
+        (void)hipDeviceSynchronize();
+        (void)hipFree(s.ptr[slot]);
+      }
       s.ptr[slot] = nullptr;
       s.size[slot] = 0;
     }
@@ -194,6 +204,23 @@ bool stream_capturing(hipStream_t st) {
     return true;
   }
   return cs != hipStreamCaptureStatusNone;
+}
+
+// stream_workspace for calls that a graph capture may record: captured calls use
+// one buffer per slot0, which every other call (on any stream) reserves, since a
+// capture must not allocate.  A buffer handed to a capture is not freed when a
+// larger call outgrows it, so a graph's replays stay valid until jv_shutdown;
+// graphs of one thread share it, so their replays must not overlap.
+void* capturable_workspace(size_t bytes, int slot0, hipStream_t st) {
+  const int slot = slot0 + WS_STREAMS;
+  if (!stream_capturing(st)) return workspace(bytes, slot) ? stream_workspace(bytes, slot0, st) : nullptr;
+  void* p = workspace(bytes, slot);
+  if (p) {
+    DeviceState& s = state();
+    if ((int)s.kept.size() <= slot) s.kept.resize(slot + 1, false);
+    s.kept[slot] = true;
+  }
+  return p;
 }
 
 // The calling thread's auxiliary stream on the current device (default
@@ -264,6 +291,7 @@ int jv_workspace_bytes(int64_t* bytes) {
   if ((int)jv::t_state.dev.size() > d) {
     const auto& s = jv::t_state.dev[d];
     for (size_t b : s.size) total += b;
+    for (auto& r : s.retired) total += r.second;
     size_t lib = 0;  // the solver library handle's own device memory
     if (s.blas && rocblas_get_device_memory_size(s.blas, &lib) == rocblas_status_success) total += lib;
   }

@@ -93,7 +93,9 @@ int build_rbm_tables(const RbmGeom& g, const double* params, const OpDev* op, bo
                      int slot0, RbmTab* out, const int32_t* map, int G) {
   const int nops = op ? op->num_ops : 0;
   if (!map) G = 0;
-  double* base = (double*)stream_workspace(sizeof(double) * rbm_tab_doubles(g, me, he, nops, G), slot0, st);
+  // symmetrised networks' calls may be captured, the others have other kernels then
+  const size_t bytes = sizeof(double) * rbm_tab_doubles(g, me, he, nops, G);
+  double* base = (double*)(G > 0 ? capturable_workspace(bytes, slot0, st) : stream_workspace(bytes, slot0, st));
   if (!base) return fail(JV_E_NOMEM, "RBM ratio tables: workspace allocation failed");
   *out = rbm_tab_at(g, base, me, he, nops, G);
   hipLaunchKernelGGL(rbm_tables, dim3((unsigned)(rbm_tab_blocks(g, nops) + G)), dim3(256), 0, st, g, params,

@@ -820,7 +820,7 @@ int sym_rbm_eloc_launch(const jv_net* net, const double* params, const jv_orbit*
                         : (four ? sym_rows_eloc<false, 4> : sym_rows_eloc<false, 1>);
   if ((rc = set_lds_limit((const void*)rf, rlds))) return rc;
   const int K = n <= 256 ? std::min(d.num_ops, 512 / (int)n) : 1;
-  double* part = K > 1 ? (double*)stream_workspace(16 * (size_t)K * n, slot1, st) : out;
+  double* part = K > 1 ? (double*)capturable_workspace(16 * (size_t)K * n, slot1, st) : out;
   if (!part) return fail(JV_E_NOMEM, "jv_sym_eloc: workspace allocation failed");
   hipLaunchKernelGGL(rf, dim3((unsigned)std::min<int64_t>(n, 512 * SYM_T / T), (unsigned)K), dim3((unsigned)T), rlds, st, g, o,
                      params, d, tab, SL, configs, lps, n, part);
