@@ -295,6 +295,39 @@ def test_eloc_streams():
         assert all(torch.equal(o, ref[k]) for o in out[k])
 
 
+def test_eloc_many_streams():
+    """Calls in turn on more streams than eight do not wait for the device."""
+    L, H = 10, 20
+    rng = np.random.default_rng(6)
+    Hd, _ = tfim_pair((L,), -1.0, -0.7)
+    psi, _ = _states(True, L, H, True, False, 0.1 * rng.normal(size=_num(True, L, H, True, False)))
+    sd = torch.as_tensor(rng.integers(0, 2, size=(1, 40, L)).astype(np.int32), device="cuda")
+    lp = psi(sd)
+    ref = Hd.get_O_loc(sd, psi, lp)
+    streams = [torch.cuda.Stream() for _ in range(20)]
+    busy = torch.cuda.Stream()
+    torch.cuda.synchronize()
+
+    def turn():
+        out = []
+        for st in streams:
+            with torch.cuda.stream(st):
+                out.append(Hd.get_O_loc(sd, psi, lp))
+        return out
+
+    turn()  # buffers of every stream
+    torch.cuda.synchronize()
+    done = torch.cuda.Event()
+    with torch.cuda.stream(busy):
+        torch.cuda._sleep(200_000_000)  # 2 s at the 100 MHz counter, less at the core clock
+        done.record()
+    out = turn()
+    waited = done.query()
+    torch.cuda.synchronize()
+    assert all(torch.equal(o, ref) for o in out)
+    assert not waited
+
+
 @pytest.mark.parametrize("cpx,L,H,bias,vbias,mu,big", [
     (True, 10, 20, True, True, 2.0, 0.0), (True, 7, 1, False, False, 1.0, 0.0), (False, 12, 65, True, False, 2.0, 0.0),
     (True, 65, 130, True, False, 2.0, 0.0), (False, 9, 256, False, False, 0.5, 0.0), (True, 6, 257, True, False, 2.0, 0.0),

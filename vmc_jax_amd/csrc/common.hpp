@@ -28,7 +28,7 @@ int hip_fail(hipError_t e, const char* what);
 // Per-device scratch arena (grown on demand, released by jv_shutdown).
 void* workspace(size_t bytes, int slot);
 // The same per stream (WS_STREAMS slots from slot0 on).
-constexpr int WS_STREAMS = 8;
+constexpr int WS_STREAMS = 40;
 void* stream_workspace(size_t bytes, int slot0, hipStream_t st);
 // The same for calls that may be captured (one more slot behind those).
 void* capturable_workspace(size_t bytes, int slot0, hipStream_t st);

@@ -178,8 +178,9 @@ void* workspace(size_t bytes, int slot) {
 
 // Scratch buffer of a stream: calls on different streams of one thread get
 // buffers of their own (slots slot0 .. slot0 + WS_STREAMS - 1), so they may
-// overlap.  Beyond WS_STREAMS streams the longest unused one's buffer passes
-// to the new stream after a device synchronisation.
+// overlap.  Beyond WS_STREAMS streams (torch's pool has 32 per device) the
+// longest unused one's buffer passes to the new stream after a device
+// synchronisation.
 void* stream_workspace(size_t bytes, int slot0, hipStream_t st) {
   DeviceState& s = state();
   int k = -1, old = 0;

@@ -25,7 +25,7 @@ namespace jv {
 constexpr double RBMQ_THETA = 150.0;
 // First slots of the tables in stream_workspace, for the local energies and
 // the chains (which a step may run on different streams).
-constexpr int WS_RBMQ_ELOC = 130, WS_RBMQ_MC = 140;
+constexpr int WS_RBMQ_ELOC = 130, WS_RBMQ_MC = WS_RBMQ_ELOC + WS_STREAMS;
 constexpr int RBMQ_MAX_H = 900;  // prod_h (1 + e_h) <= 2^H
 constexpr int RBM_ORBIT_MAX_L = 16384;  // sites of an orbit's map (positions in 16 bits)
 

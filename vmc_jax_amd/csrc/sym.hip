@@ -29,7 +29,9 @@ int sym_rbm_mc_launch(const jv_net* net, const double* params, const jv_orbit* o
 
 namespace {
 // first slots of the resident forms' tables and partial sums in stream_workspace
-constexpr int WS_SYM_ELOC_TAB = 150, WS_SYM_MC_TAB = 160, WS_SYM_ELOC_PART = 170;
+// (and one more slot each, capturable_workspace), behind WS_RBMQ_*
+constexpr int WS_SYM_ELOC_TAB = 130 + 2 * WS_STREAMS, WS_SYM_MC_TAB = WS_SYM_ELOC_TAB + WS_STREAMS + 1,
+              WS_SYM_ELOC_PART = WS_SYM_MC_TAB + WS_STREAMS + 1;
 // workspace slots of this file.  jv_sym_eloc may run on a side stream while
 // jv_sym_gradients runs on the main stream, so the forward pass inside
 // jv_sym_eloc has rows / log-psi slots of its own (WS_EROWS, WS_ELP).
