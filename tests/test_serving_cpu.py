@@ -115,3 +115,19 @@ def test_footprint_grows_with_problem_size():
     large = serving.footprint_bytes(16384, 1240, 144, False, "minsr", 1024)
     tdvp = serving.footprint_bytes(16384, 4224, 32, True, "tdvp", 1024)
     assert small < large < tdvp
+
+
+def test_footprint_of_the_holomorphic_solve():
+    """Per sample, a holomorphic TDVP job holds O, the centred O (flat layout) and
+    two arrays of half the columns; without the pair structure (real
+    parameters, or too few) the SNR data and their projection come on top."""
+    n, pr = 16384, 4224
+    row = n * pr * 16
+
+    def grown(pr, cpx, gram):
+        f = [serving.footprint_bytes(m, pr, 32, cpx, "tdvp", 1024) / 1.25 - serving._gram_slice_bytes(m, gram)
+             for m in (n, 1)]
+        return f[0] - f[1]
+    assert 3.0 * row <= grown(pr, True, pr) <= 3.1 * row
+    assert grown(pr, False, 2 * pr) >= 4.0 * row
+    assert grown(200, True, 400) >= 4.0 * n * 200 * 16

@@ -39,6 +39,8 @@ import time
 import numpy as np
 import torch
 
+from .util.tdvp import HOLOMORPHIC_SOLVE
+
 
 class Job:
     """One VMC job.  ``make`` builds (psi, hamiltonian, equation, stepper) on
@@ -420,13 +422,16 @@ def footprint_bytes(num_samples, num_real_params, num_sites, complex_params, sol
     b = n * num_sites * 4 * 6 + chains * num_sites * 4    # samples, s' slots of the operator, walkers
     b += n * 16 * 8                                       # log psi, E_loc, weights, centred E_loc copies
     if solver == "tdvp":
-        b += n * pr * 16 * 4                              # O (flat layout) and centred O, SNR data Q and R
-        b += n * pc * 16 * 2                              # holomorphic G and the SNR projection M
+        pairs = complex_params and pc >= HOLOMORPHIC_SOLVE["real"]
+        b += n * pr * 16 * 2                              # O (flat layout) and centred O
+        if not pairs:
+            b += n * pr * 16 * 2                          # SNR data Q and R
+        b += n * pc * 16 * 2                              # holomorphic G (then the SNR data Qc) and the projection M
         b += pr * pr * 8 * 5                              # S0 (complex), Z, S
         b += _q_apply_bytes(pc)
         b += pc * pc * 8 * 10                             # A, eigenvectors, tridiagonal Z and Zc, D&C buffers
         b += pr * pr * 16 * 3                             # library eigendecomposition workspace
-        b += _gram_slice_bytes(n, 2 * pr)
+        b += _gram_slice_bytes(n, 2 * pc if pairs else 2 * pr)
         if precision == "mixed":
             b += _bf16_gram_bytes(n, 2 * pc)
     elif solver == "minsr":
