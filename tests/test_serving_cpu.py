@@ -117,6 +117,25 @@ def test_footprint_grows_with_problem_size():
     assert small < large < tdvp
 
 
+def test_batch_shapes_of_the_local_energies():
+    """The O_loc phase has four waves per workgroup whatever the shape says: every
+    candidate differs, and shapes cached under the meaning they had before
+    (samples per wave) are not found."""
+    import hashlib
+    import json
+
+    from vmc_jax_amd import batch
+    shapes = batch.BatchedSweep.SHAPES["eloc"]
+    assert all(w == 4 for w, _ in shapes) and len({t for _, t in shapes}) == len(shapes)
+
+    class Inst:
+        def signature(self):
+            return [8, 16, 1, 24, 512, 64, 1]
+    b = object.__new__(batch.BatchedSweep)
+    b.inst = [Inst()]
+    assert b.key() != hashlib.sha1(json.dumps(sorted(i.signature() for i in b.inst)).encode()).hexdigest()
+
+
 def test_footprint_of_the_holomorphic_solve():
     """Per sample, a holomorphic TDVP job holds O, the centred O (flat layout) and
     two arrays of half the columns; without the pair structure (real

@@ -9,9 +9,10 @@ MinSR equation and an Euler step); the reference runs each as its own driver
 * sampling, log psi + O_k and O_loc of **all** instances are one launch each
   (``jv_batch_step``: a device-resident instance table maps every workgroup to
   one instance), captured once into a HIP graph and replayed every step;
-* the launch shape of each phase (waves per workgroup, samples per wave) is
-  chosen by ``autotune`` from timed trials on the actual instance mix and kept
-  in a JSON cache keyed by the mix;
+* the launch shape of each phase (waves per workgroup; samples per wave of the
+  O_k phase, tiles of samples per workgroup of the O_loc phase) is chosen by
+  ``autotune`` from timed trials on the actual instance mix and kept in a JSON
+  cache keyed by the mix;
 * the per-instance solves (FP64 eigendecomposition / Cholesky) run on a pool
   of worker threads, each with its own HIP stream, after the graph's event,
   and update the parameters in place (the graph reads them at replay).
@@ -134,7 +135,10 @@ def _load_cache(path):
 class BatchedSweep:
     SHAPES = {"sample": [(w, 1) for w in (1, 2, 4, 8)],
               "grad": [(w, s) for w in (1, 2, 4, 8) for s in (1, 2, 4, 8)],
-              "eloc": [(w, s) for w in (1, 2, 4, 8) for s in (1, 2, 4, 8)]}
+              "eloc": [(4, t) for t in (1, 2, 4, 8)]}  # always four waves; tiles of samples per workgroup
+    # Part of the cache key: what a shape's numbers mean.  2: O_loc shapes count
+    # tiles (1: samples per wave).
+    SHAPE_VERSION = 2
 
     def __init__(self, instances, workers=8, tune=True, graph=True, pool=None):
         """tune: True runs the trials unless the mix is in the cache; "cache" uses
@@ -166,7 +170,7 @@ class BatchedSweep:
         self._phase_events = []
 
     def key(self):
-        sig = json.dumps(sorted(i.signature() for i in self.inst))
+        sig = json.dumps([self.SHAPE_VERSION, sorted(i.signature() for i in self.inst)])
         return hashlib.sha1(sig.encode()).hexdigest()
 
     def _set_shape(self, batch, phase, shape):
