@@ -54,6 +54,19 @@ def test_complex_eigh_large(n):
         assert np.abs(ev - ref).max() <= 1e-12 * np.abs(ref).max()
 
 
+@pytest.mark.parametrize("n", [128, 129, 130, 193, 257])
+def test_complex_eigh_reflector_blocks(n):
+    """n - 1 reflectors below, at and above whole blocks of 64 (the back
+    transformation's); residual and orthogonality as above."""
+    A = _hermitian(n, n)
+    V, w = _eigh(A)
+    V, ev = V.cpu().numpy(), w.cpu().numpy()
+    assert np.linalg.norm(A @ V - V * ev[None, :]) < 1e-12 * np.linalg.norm(A)
+    assert np.linalg.norm(V.conj().T @ V - np.eye(n)) < 1e-13 * np.sqrt(n)
+    ref = np.linalg.eigvalsh(A)
+    assert np.abs(ev - ref).max() <= 1e-12 * np.abs(ref).max()
+
+
 def test_complex_minsr_t_form_cut_large():
     """T = D D^H (N = 2600 samples, 1200 complex parameters) has rank 1200: the
     pseudo-inverse cuts the rest, so the eigendecomposition of T (the large-n

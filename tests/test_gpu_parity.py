@@ -367,7 +367,7 @@ def test_large_products_through_blas(cpx):
 def test_eigh(cpx, n, stedc):
     """rocSOLVER below 128; from 128 up the Householder tridiagonalisation
     (real: dsytrd conventions; complex Hermitian: zhetrd conventions, real T)
-    + divide and conquer + dormtr / zunmtr."""
+    + divide and conquer + dormtr (real) or reflector blocks (complex)."""
     rng = np.random.default_rng(21)
     A = rng.normal(size=(n, n)) + (1j * rng.normal(size=(n, n)) if cpx else 0)
     A = A + A.conj().T

@@ -463,6 +463,47 @@ def test_sym_out_of_range(cpx, L, H, names, op, mu):
     assert float(ms.acceptance_ratio()[0]) == float(np.ravel(mo.acceptance_ratio())[0])
 
 
+@pytest.mark.parametrize("cpx,L,H,mu", [(True, 9, 12, 1.0), (False, 9, 33, 0.5), (True, 8, 5, 0.0)])
+def test_sym_chains_mu(cpx, L, H, mu):
+    rng = np.random.default_rng(L * 100 + H)
+    P = 0.3 / np.sqrt(L) * rng.normal(size=_num(cpx, L, H, True, False))
+    psi, opsi = _sym_states(cpx, L, H, ALL, P)
+    kw = dict(numChains=3, numSamples=9, thermalizationSweeps=3, sweepSteps=50, mu=mu)
+    ms = jv.sampler.MCSampler(psi, (L,), 5, updateProposer=jv.sampler.propose_spin_flip, **kw)
+    mo = osamp.MCSampler(opsi, (L,), 5, **kw)
+    for _ in range(2):
+        assert np.array_equal(to_np(ms.sample()[0])[0], mo.sample()[0])
+    assert np.array_equal(to_np(ms.states), mo.states)
+
+
+def test_sym_streams():
+    """Symmetrised calls on two streams of one thread, each with its own
+    parameters and enough samples to overlap, keep their tables apart."""
+    L, H, n = 10, 12, 2000
+    rng = np.random.default_rng(15)
+    Hd, _ = tfim_pair((L,), -1.0, -0.7)
+    Hd.compile()
+    sd = torch.as_tensor(rng.integers(0, 2, size=(1, n, L)).astype(np.int32), device="cuda")
+    psis = [_sym_states(True, L, H, ALL, 0.1 * rng.normal(size=_num(True, L, H, True, False)))[0] for _ in range(2)]
+    kw = dict(numChains=64, numSamples=64, thermalizationSweeps=2, sweepSteps=20)
+
+    def calls(p):
+        ms = jv.sampler.MCSampler(p, (L,), 5, updateProposer=jv.sampler.propose_spin_flip, **kw)
+        lp = p(sd)
+        return lp, Hd.get_O_loc(sd, p, lp), ms.sample()[0]
+    ref = [[t.clone() for t in calls(p)] for p in psis]
+    streams = [torch.cuda.Stream() for _ in range(2)]
+    torch.cuda.synchronize()
+    out = [[], []]
+    for _ in range(4):
+        for k, st in enumerate(streams):
+            with torch.cuda.stream(st):
+                out[k].append(calls(psis[k]))
+    torch.cuda.synchronize()
+    for k in range(2):
+        assert all(torch.equal(a, b) for o in out[k] for a, b in zip(o, ref[k]))
+
+
 def test_sym_eloc_negative_sums():
     """A real network's negative sums have no logarithm: the local energy is NaN
     where any string with a matrix element leads to one, also where it cancels
