@@ -751,7 +751,7 @@ __device__ inline void rbmq_eloc_range(const RbmGeom& g, const double* __restric
                                        double* lds) {
   const int lane = threadIdx.x % WAVE, w = __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE);
   if constexpr (S > 0) {
-    if (rbmq_ok(g, tab, max(2, op.max_len), lane)) {
+    if (__builtin_expect(rbmq_ok(g, tab, max(2, op.max_len), lane), 1)) {
       for (int64_t k = 0; k < cnt; k += S) {
         const int64_t s = s0 + k;
         rbmq_eloc_tile<CPX, SMALL, S>(g, P, op, tab, cfg + s * g.L, (int)min((int64_t)S, cnt - k), nstr, lps + 2 * s,
@@ -1019,7 +1019,7 @@ template <bool CPX, int NH>
 __device__ inline int64_t rbmq_mc(const RbmGeom& g, const double* __restrict__ P, const jv_mc_args& a,
                                   const RbmTab& tab, int32_t* __restrict__ walkers, int32_t* __restrict__ configs,
                                   int chain, int lane, double* lds) {
-  if (rbmq_ok(g, tab, 2, lane))  // squared moduli: twice the exponent of one flip
+  if (__builtin_expect(rbmq_ok(g, tab, 2, lane), 1))  // squared moduli: twice the exponent of one flip
     return rbmq_mc_chain<CPX, NH>(g, P, a, tab, walkers, configs, chain, lane);
   return rbmq_mc_direct<CPX>(g, P, a, walkers, configs, chain, lane, lds);
 }
