@@ -104,7 +104,8 @@ typedef struct jv_optable {
 
 /* Symmetrisation of a network over an orbit of lattice symmetries (SymNet,
  * sym_wrapper.py:29-83).  The orbit matrices of symmetries.py:75-206 are signed
- * permutations; element g is stored as a site map: (g s)_i = s_j for
+ * permutations (rows that read a site twice are evaluated all the same, row by
+ * row); element g is stored as a site map: (g s)_i = s_j for
  * map[g][i] = j >= 0 and 1 - s_j for map[g][i] = -1 - j, which is
  * (o (2s - 1) + 1) // 2 of sym_wrapper.py:70-73 for a matrix row with a single
  * entry +1 (-1) in column j.  All pointers are device pointers. */
@@ -225,17 +226,21 @@ int jv_sym_gradients(const jv_net* net, const double* params, const jv_orbit* or
                      const int32_t* configs, int64_t n, int32_t layout, double* grad,
                      double* logpsi, void* stream);
 
-/* O_loc(s) = sum_j m_j exp(log psi(s'_j) - logpsi_s) for a symmetrised network:
- * s' materialised per sample chunk (jv_get_s_primes), log psi(s') from
- * jv_sym_forward.  Replaces Operator.get_O_loc (base.py:162-192) for a SymNet. */
+/* O_loc(s) = sum_j m_j exp(log psi(s'_j) - logpsi_s) for a symmetrised network.
+ * RBMs under EXP with strings of at most two sites: the orbit of s resident in
+ * one workgroup, a ratio per row and string; else s' materialised per sample
+ * chunk (jv_get_s_primes) and log psi(s') from jv_sym_forward.  A graph capture
+ * needs a call of the same size before it.  Replaces Operator.get_O_loc (base.py:162-192) for a SymNet. */
 int jv_sym_eloc(const jv_net* net, const double* params, const jv_orbit* orbit,
                 const jv_optable* op, const double* prefactor, const int32_t* configs,
                 const double* logpsi_s, int64_t n, double* out, void* stream);
 
 /* Metropolis sampling of a symmetrised network with single-spin-flip proposals:
- * the same arguments, Philox draws and emission order as jv_mc_sample; each
- * proposal is evaluated with jv_sym_forward on all chains at once and accepted
- * with u < exp(mu Re(log psi' - log psi)).
+ * the same arguments, Philox draws and emission order as jv_mc_sample; a
+ * proposal is accepted with u < exp(mu Re(log psi' - log psi)).  RBMs under EXP
+ * whose orbit fits one workgroup: a chain per workgroup and one launch; else
+ * each proposal is evaluated with jv_sym_forward on all chains at once.  A
+ * graph capture needs a call of the same size before it.
  * Replaces MCSampler._sweep / _get_samples_mcmc (sampler.py:264-367) for a SymNet. */
 int jv_sym_mc_sample(const jv_net* net, const double* params, const jv_orbit* orbit,
                      const jv_mc_args* args, int32_t* walkers, int32_t* configs, double* logpsi,

@@ -420,7 +420,10 @@ int gram_pp_f64(const double* D, int64_t n, int64_t p, int cpx, double* S, hipSt
   // slice leaves the second round of the L = 32 complex RBM's 561 tiles nearly
   // empty (16384 x 2112 complex: 8.7 ms, 5.05 with the slices this picks);
   // sixteen leave a 1240-column Gram's second round (880 workgroups) a quarter
-  // empty (0.310 ms; nine, one round of 495, 0.260).
+  // empty (0.310 ms; nine, one round of 495, 0.260).  The partial tiles of the
+  // slices take memory for it: 631 MB at 16384 x 2112 complex (70 with one
+  // slice; four slices, 280 MB, would cost a tenth more rounds), 1 GiB at most
+  // where there is more than one.
   const int64_t nkb = (n + G6K - 1) / G6K;
   int64_t splits = 1, best = INT64_MAX;
   for (int64_t s = 1; s <= 64 && s * 8 <= std::max<int64_t>(nkb, 8) && (s == 1 || ntiles * s <= 8192); ++s) {

@@ -1157,8 +1157,6 @@ __global__ void tdvp_project_S(const double* __restrict__ S0, int64_t pr, int im
   }
 }
 
-// Per-sample SNR data Q[n][k] = makeReal(-x conj(D[n][k]) e_n / w_n)
-// (stats.py:255-265 covar_data followed by transform, tdvp.py:175-178).
 // -x conj(D_t) e / w: the part of one sample's force the solve mode keeps.
 __device__ inline double tdvp_snr_q(const double* __restrict__ D, int64_t t, double er, double ei, double inv, double xr,
                                     double xi, int imag) {
@@ -1169,6 +1167,8 @@ __device__ inline double tdvp_snr_q(const double* __restrict__ D, int64_t t, dou
   return imag ? -(xr * pi_ + xi * pr_) : -(xr * pr_ - xi * pi_);
 }
 
+// Per-sample SNR data Q[n][k] = makeReal(-x conj(D[n][k]) e_n / w_n)
+// (stats.py:255-265 covar_data followed by transform, tdvp.py:175-178).
 __global__ void tdvp_snr_data(const double* __restrict__ D, const double* __restrict__ e,
                               const double* __restrict__ w, int64_t n, int64_t pr, double xr, double xi, int imag,
                               double* __restrict__ Q) {

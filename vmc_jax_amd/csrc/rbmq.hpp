@@ -298,8 +298,8 @@ __device__ inline void rbm_ab(double th, double& al, double& be, double& lin, do
 
 // ------------------------------------------------------------------ local energies
 // A workgroup of four waves evaluates a tile of samples together: eight where
-// that leaves four workgroups per CU (n >= 8192: 74 against 85 us with four at
-// 16384 samples of 32 sites x 64 units), else four (51 against 60 us at 3000
+// that leaves four workgroups per CU (n >= 8192: 67 against 81 us with four at
+// 16384 samples of 32 sites x 64 units), else four (49.5 against 57.7 us at 3000
 // samples of 45 x 90), and two for more than 256 hidden units, whose alpha,
 // beta would not fit otherwise.  A sample's result does not depend on it.
 constexpr int RBMQ_WAVES = 4;
@@ -360,10 +360,10 @@ __device__ inline cd string2(const OpDev& op, int o, const int32_t* c, bool& fa,
 // order of every sum and product depends on the sizes only, not on ns or on
 // which samples share a workgroup.
 // Measured (tables included): 16384 samples of 32 sites x 64 units, Ising
-// chain, 2042 -> 75 us; 3000 samples of 45 x 90, XXZ chain (90 two-site
-// strings, the X X and Y Y of a bond sharing one ratio), 1430 -> 53 us.  What
-// is left is latency: 43k cycles per tile, of which theta 10k, the reductions
-// and diagonal strings 8k, matrix elements 4k, the products 11k.
+// chain, 2042 -> 65 us; 3000 samples of 45 x 90, XXZ chain (90 two-site
+// strings, the X X and Y Y of a bond sharing one ratio), 1430 -> 49 us.  Vector
+// issue takes 65 % of the time (3200 instructions per wave and tile), bank
+// conflicts 4 %.
 // SMALL: strings of at most two factors without Jordan-Wigner signs.
 template <bool CPX, bool SMALL, int S>
 __device__ inline void rbmq_eloc_tile(const RbmGeom& g, const double* __restrict__ P, const OpDev& op,
@@ -793,7 +793,8 @@ __host__ __device__ inline bool rbmq_mc_fits(const RbmGeom& g) {
 // e = e^{-2 theta} is updated by products (relative error only) and recomputed
 // from the weights at emissions at least RBMQ_MC_REFRESH proposals apart.
 // 1024 chains x 1312 proposals, 32 sites x 64 units: 2080 us with a complex
-// log-cosh per unit and proposal, 440 us here (0.34 us per proposal).
+// log-cosh per unit and proposal, 428 us here (0.33 us and 64 vector
+// instructions per proposal, 38 % of the issue cycles).
 template <bool CPX, int NH>
 __device__ inline int64_t rbmq_mc_chain(const RbmGeom& g, const double* __restrict__ P, const jv_mc_args& a,
                                         const RbmTab& tab, int32_t* __restrict__ walkers,

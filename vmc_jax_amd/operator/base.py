@@ -66,7 +66,7 @@ class Operator(metaclass=abc.ABCMeta):
         lps = logPsiS.reshape(-1).to(torch.complex128).contiguous()
         out = torch.empty(n, dtype=torch.complex128, device=flat.device)
         if psi._sym is not None:
-            # symmetrised networks: s' materialised per chunk, log psi(s') over the orbit
+            # symmetrised networks: over the orbit (RBMs) or materialised s' (jv_sym_eloc)
             _lib.call("jv_sym_eloc", psi.desc, _lib.ptr(psi.params), psi._sym[0], self.table, _lib.ptr(pref),
                       _lib.ptr(flat), _lib.ptr(lps), n, _lib.ptr(out), _lib.stream_ptr())
         else:
