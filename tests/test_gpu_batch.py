@@ -116,3 +116,27 @@ def test_batch_steps_equal_alone(tmp_path, monkeypatch):
             assert np.linalg.norm(a - r) <= 1e-12 * np.linalg.norm(r), kind
     finally:
         b.close()
+
+
+def test_batch_of_a_single_string(tmp_path, monkeypatch):
+    """An operator of one string, which jv_eloc gives to the log-cosh kernel on
+    its own, equals it bit for bit in the batch, beside one that does not."""
+    from vmc_jax_amd import operator as dop
+    monkeypatch.setenv("VMC_JAX_AMD_TUNE_CACHE", str(tmp_path / "tune.json"))
+    inst, states = [], []
+    for kind, L, a, seed in KINDS[:2]:
+        psi, H = _spec(kind, L, a, seed)
+        if kind == "tdvp":
+            H = dop.BranchFreeOperator()
+            H.add(dop.scal_opstr(0.7, (dop.Sx(2),)))
+        inst.append(jb.Instance(psi, H, _make(kind, psi, H), 1e-2, key=seed, numChains=CHAINS, numSamples=SAMPLES))
+        states.append((psi, H))
+    b = jb.BatchedSweep(inst, workers=1, tune=False, graph=False)
+    try:
+        torch.cuda.current_stream().wait_event(b.sample_phase())
+        for ins, (psi, H) in zip(inst, states):
+            E = H.get_O_loc(ins.configs[None], psi, ins.logpsi[None])
+            torch.cuda.synchronize()
+            assert torch.equal(ins.eloc, E.reshape(-1).to(torch.complex128))
+    finally:
+        b.close()

@@ -133,6 +133,26 @@ def _late_pair(L, where):
     return out
 
 
+@pytest.mark.parametrize("cpx,H,strings,n", [(True, 64, 3, 2000), (True, 64, 3, 2001), (True, 65, 1, 3000), (True, 65, 2, 5),
+                                             (False, 640, 1, 1200), (False, 256, 2, 1501), (False, 300, 1, 3000), (False, 641, 2, 5), (True, 5, 1, 6001)])
+def test_eloc_few_strings(cpx, H, strings, n):
+    """Either side of the rule that gives few strings on few samples to the
+    log-cosh kernel."""
+    from vmc_jax_amd import operator as dop
+    L = 5
+    rng = np.random.default_rng(H)
+    P = 0.3 / np.sqrt(L) * rng.normal(size=_num(cpx, L, H, True, False))
+    psi, opsi = _states(cpx, L, H, True, False, P)
+    Hd, Ho = dop.BranchFreeOperator(), oop.BranchFreeOperator()
+    for k in range(strings):
+        Hd.add(dop.scal_opstr(0.5 + k, (dop.Sx(k), dop.Sz(4))))
+        Ho.add(oop.scal_opstr(0.5 + k, (oop.Sx(k), oop.Sz(4))))
+    s = rng.integers(0, 2, size=(n, L)).astype(np.int32)
+    sd = torch.as_tensor(s[None], device="cuda")
+    e = to_np(Hd.get_O_loc(sd, psi, psi(sd)))[0]
+    assert _rel(e, Ho.get_O_loc(s, opsi, opsi(s))) < TOL
+
+
 @pytest.mark.parametrize("L,H,n,where", [(2, 1, 9000, 0), (2, 1, 40, 3), (50, 5, 60, 0), (50, 5, 60, 63),
                                          (50, 5, 60, 64), (50, 5, 60, 99)])
 def test_eloc_string_that_flips_nothing(L, H, n, where):

@@ -165,7 +165,8 @@ static int batch_layout(jv_batch* b) {
   for (auto& I : b->host) {
     mc_lds = std::max(mc_lds, 8 * mc_rbm_lds_doubles(I.g));
     const size_t q = I.g.H <= RBMQ_MAX_H ? 8 * rbmq_block_lds_doubles(I.g, I.nstr, I.n) : 0;
-    I.tile = q > 0 && q <= 160 * 1024 ? rbmq_tile(I.g, I.n) : 0;
+    // the form jv_eloc takes on its own
+    I.tile = q > 0 && q <= 160 * 1024 && !rbmq_eloc_small(I.g, I.op.num_ops, I.n) ? rbmq_tile(I.g, I.n) : 0;
     el_lds = std::max(el_lds, I.tile ? q : RBMQ_WAVES * 2 * sizeof(cd) * (size_t)I.g.H);
   }
   int tot[4] = {0, 0, 0, 0};

@@ -630,10 +630,11 @@ int jv_eloc(const jv_net* net, const double* params, const jv_optable* op, const
   if (make_rbm_geom(net, rg)) {
     ScopedTimer tm("eloc", st);
     // ratio form, except where its tables cannot be built (a graph capture:
-    // the captured call keeps no pointer into scratch memory) or do not fit
+    // the captured call keeps no pointer into scratch memory), do not fit or do
+    // not pay
     const int nstr = rbmq_strings(d);
     const size_t lq = 8 * rbmq_block_lds_doubles(rg, nstr, n);
-    if (rg.H <= RBMQ_MAX_H && lq <= 160 * 1024 && !stream_capturing(st)) {
+    if (rg.H <= RBMQ_MAX_H && lq <= 160 * 1024 && !rbmq_eloc_small(rg, d.num_ops, n) && !stream_capturing(st)) {
       RbmTab tab;
       rc = build_rbm_tables(rg, params, &d, false, true, st, WS_RBMQ_ELOC, &tab);
       if (rc) return rc;

@@ -312,6 +312,18 @@ __host__ __device__ inline int rbmq_jp(int n) {
   while (jp > 1 && jp / 2 >= n) jp /= 2;
   return jp;
 }
+// Few strings on few samples: the log-cosh form's one launch is over before the
+// ratio form's table is (one Sx on 1000 samples of 16 x 32: 15.8 against 18.6
+// us a call, on 5000 24.9 against 27.2, on 20000 81.8 against 58.5; three on
+// 5000 40.1 against 26.2; real 21.6 against 25.4 for one on 5000).  Work is
+// counted in strings times units a lane, whose log-cosh costs a complex network
+// three times a real one's.  A real network's two-sample tiles do not pay for a
+// single string at any size (8 x 300, 100000 samples: 487 against 526 us).
+__host__ __device__ inline bool rbmq_eloc_small(const RbmGeom& g, int num_ops, int64_t n) {
+  const int64_t w = (int64_t)num_ops * ((g.H + WAVE - 1) / WAVE);
+  if (!g.cpx && g.H > 256 && num_ops == 1) return true;
+  return w <= (g.cpx ? 3 : 10) && n * w <= (g.cpx ? 6000 : 12000);
+}
 // LDS doubles of the workgroup, for at most `nstr` strings per sample: alpha,
 // beta; psi(s) / e^{lps}; matrix elements and per-wave products of a pass;
 // spins; one flag.
