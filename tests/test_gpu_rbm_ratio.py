@@ -483,6 +483,35 @@ def test_sym_out_of_range(cpx, L, H, names, op, mu):
     assert float(ms.acceptance_ratio()[0]) == float(np.ravel(mo.acceptance_ratio())[0])
 
 
+@pytest.mark.parametrize("cpx,L,H,names", [(True, 10, 20, ("reflection",)), (True, 12, 70, ALL), (False, 16, 32, ALL),
+                                           (True, 6, 200, ("reflection",))])
+def test_sym_eloc_forms(cpx, L, H, names):
+    """Local energies and log psi in each form the sizes choose between: one to
+    many strings (with and without diagonal ones) on one to some hundred
+    samples, whose strings share a workgroup or have several."""
+    from vmc_jax_amd import operator as dop
+    rng = np.random.default_rng(L * 1000 + H)
+    P = 0.3 / np.sqrt(L) * rng.normal(size=_num(cpx, L, H, True, False))
+    psi, opsi = _sym_states(cpx, L, H, names, P)
+    s = rng.integers(0, 2, size=(520, L)).astype(np.int32)
+    lpo = opsi(s)
+    for strings, diag in ((1, 0), (2, 0), (3, 1), (4, 3)):
+        Hd, Ho = dop.BranchFreeOperator(), oop.BranchFreeOperator()
+        for k in range(strings):
+            Hd.add(dop.scal_opstr(0.5 + k, (dop.Sx(k), dop.Sx(5 - k) if k == 1 else dop.Sz(5 - k))))
+            Ho.add(oop.scal_opstr(0.5 + k, (oop.Sx(k), oop.Sx(5 - k) if k == 1 else oop.Sz(5 - k))))
+        for k in range(diag):
+            Hd.add(dop.scal_opstr(0.3 * (k + 1), (dop.Sz(k), dop.Sz(k + 1))))
+            Ho.add(oop.scal_opstr(0.3 * (k + 1), (oop.Sz(k), oop.Sz(k + 1))))
+        ref = Ho.get_O_loc(s, opsi, lpo)
+        for n in (1, 5, 100, 257, 520):
+            sd = torch.as_tensor(s[None, :n].copy(), device="cuda")
+            lp = psi(sd)
+            assert np.max(np.abs(to_np(lp)[0] - lpo[:n])) < TOL * np.max(np.abs(lpo))
+            e = to_np(Hd.get_O_loc(sd, psi, lp))[0]
+            assert np.max(np.abs(e - ref[:n])) < TOL * np.max(np.abs(ref))
+
+
 @pytest.mark.parametrize("cpx,L,H,mu", [(True, 9, 12, 1.0), (False, 9, 33, 0.5), (True, 8, 5, 0.0)])
 def test_sym_chains_mu(cpx, L, H, mu):
     rng = np.random.default_rng(L * 100 + H)

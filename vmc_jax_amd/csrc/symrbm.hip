@@ -217,6 +217,24 @@ int sym_threads(const RbmGeom& g, int G, int SL) {
   return T;
 }
 
+// Estimated times in us, for the choice between the forms below and materialised
+// rows; they hold within a third over groups of 2 to 160, 8 to 64 sites and 3 to
+// 200 units (a real network's units cost half).
+//
+// log psi resident: loading theta, a step of SL threads times U units per site,
+// is a chain of loads; beyond 512 workgroups of 256 threads they queue.
+double sym_resident_us(const RbmGeom& g, int G, double n) {
+  bool four;
+  const int SL = sym_lanes(G, g.H, &four), T = sym_threads(g, G, SL), per = (four ? 4 : 1) * SL;
+  const double steps = (double)((G * SL + T - 1) / T) * ((g.H + per - 1) / per);
+  return (9.0 + (g.cpx ? 0.26 : 0.13) * g.L * steps) * std::max(1.0, 1.3 * n * T / (512.0 * SYM_T));
+}
+// ... over materialised rows, a wave each (without the launches).
+double sym_materialised_us(const RbmGeom& g, int G, double n) {
+  const double chain = (double)g.L * ((g.H + WAVE - 1) / WAVE);
+  return 0.16 * chain + (g.cpx ? 1.25e-4 : 0.63e-4) * n * G * chain;
+}
+
 // A workgroup per configuration.  FP64 issue (exp and sincos of every theta)
 // sets its time: 4096 samples, 16 sites x 32 units, 64 elements: 589 us with
 // materialised rows, 188 here (a call and its wait).
@@ -656,16 +674,17 @@ size_t sym_mc_lds(const RbmGeom& g, int G, bool tabl) {
 // 1024 chains x 128 proposals, one |Re W| = 90): 16 x 32, 64 elements E_loc
 // 17.8 -> 3.9 ms, chains 20.3 -> 5.3; 64 x 200, two elements 30.1 -> 11.2, 8.9
 // -> 4.2.
-// Few samples: the strings over gridDim.y workgroups each, whose sums [K][n]
-// sym_rbm_eloc, launched behind, adds up (16 samples of 64 x 200, two elements:
-// 1746 us with one workgroup a sample, 238 so; 659 with materialised rows).
+// Few samples: the strings over gridDim.y workgroups each, whose sums [K][n] the
+// launch behind adds up (16 samples of 64 x 200, two elements: 1746 us with one
+// workgroup a sample, 238 so; 659 with materialised rows).  Without tables
+// (tab.site null) it serves every parameter.
 template <bool CPX, int U>
 __global__ void __launch_bounds__(SYM_T, 2) sym_rows_eloc(RbmGeom g, SymGeom o, const double* __restrict__ P, OpDev op,
                                                           RbmTab tab, int SL, const int32_t* __restrict__ cfg,
                                                           const double* __restrict__ lps, int64_t n,
                                                           double* __restrict__ out) {
   extern __shared__ double lds[];
-  if (sym_ok(g, o, tab, threadIdx.x % WAVE)) return;
+  if (tab.site && sym_ok(g, o, tab, threadIdx.x % WAVE)) return;
   out += 2 * n * blockIdx.y;
   double* red = lds;
   cd* lin = (cd*)(red + 8);
@@ -739,6 +758,15 @@ __global__ void __launch_bounds__(SYM_T, 2) sym_rows_mc(RbmGeom g, SymGeom o, co
   }
 }
 
+__global__ void __launch_bounds__(SYM_T) sym_add_parts(const double* __restrict__ part, int K, int64_t n,
+                                                       double* __restrict__ out) {
+  for (int64_t q = blockIdx.x * (int64_t)SYM_T + threadIdx.x; q < 2 * n; q += (int64_t)gridDim.x * SYM_T) {
+    double v = 0.0;
+    for (int k = 0; k < K; ++k) v += part[2 * n * k + q];
+    out[q] = v;
+  }
+}
+
 __global__ void sym_zero_counters(int64_t* c) {
   if (threadIdx.x < 2) c[threadIdx.x] = 0;
 }
@@ -766,6 +794,10 @@ int sym_rbm_forward_launch(const jv_net* net, const double* params, const jv_orb
   const int SL = sym_lanes(o.G, g.H, &four), T = sym_threads(g, o.G, SL);
   const size_t lds = sym_rows_lds(g, o.G, T, SL);
   if (lds > 160 * 1024) return JV_OK;
+  // few configurations of large orbits: rows over the whole chip (three launches;
+  // 16 of 96 elements, 24 x 100: 27 us, resident 92; 256: 156 against 94)
+  if (std::max(22.0, 10.0 + sym_materialised_us(g, o.G, (double)n)) < 0.9 * (5.0 + sym_resident_us(g, o.G, (double)n)))
+    return JV_OK;
 #define JV_SYM_FWD(CPX)                                                                  \
   (four ? (SL == 4 ? sym_rbm_forward<CPX, 4, 4> : sym_rbm_forward<CPX, 4, 0>) : sym_rbm_forward<CPX, 1, 0>)
   const auto fn = g.cpx ? JV_SYM_FWD(true) : JV_SYM_FWD(false);
@@ -807,25 +839,49 @@ int sym_rbm_eloc_launch(const jv_net* net, const double* params, const jv_orbit*
   const int SL = sym_lanes(o.G, g.H, &four), T = sym_threads(g, o.G, SL);
   const size_t rlds = sym_rows_lds(g, o.G, T, SL);
   if (!RC || rlds > 160 * 1024) return JV_OK;
-  RbmTab tab;
-  int rc = build_rbm_tables(g, params, &d, false, true, st, slot0, &tab, o.map, o.G);
-  if (rc) return rc;
-#define JV_SYM_ELO(RCv)                                                                           \
-  (g.cpx ? (tabl ? sym_rbm_eloc<true, RCv, true> : sym_rbm_eloc<true, RCv, false>)                \
-         : (tabl ? sym_rbm_eloc<false, RCv, true> : sym_rbm_eloc<false, RCv, false>))
-  const auto fn = RC == 64 ? JV_SYM_ELO(64) : RC == 32 ? JV_SYM_ELO(32) : JV_SYM_ELO(16);
-#undef JV_SYM_ELO
-  rc = set_lds_limit((const void*)fn, lds);
+  // Times of the three forms: resident (alpha and beta of all rows once, then a
+  // product per string), a log psi per string, materialised s' and rows.
+  // 4000 samples, one string: 16 x 32, 64 elements 400 / 156 / 564 us, with 16
+  // more 453 / - / 17217; 64 x 200, two elements 2056 / 138 / 257, eight strings
+  // 2110 / - / 1797; one sample of 24 x 100, 96 elements 352 / 97 / 38.
+  const double steps = (double)((o.G + RC - 1) / RC) *
+                       ((tabl && !g.cpx ? 0.3 : 0.47) * g.H + 0.2 * g.L * ((g.H + 4 * (SYM_T / RC) - 1) / (4 * (SYM_T / RC))));
+  const double t_res = (18.0 + (g.cpx ? 1.0 : 0.5) * steps) * std::max(1.0, n / (lds > 80 * 1024 ? 340.0 : 512.0));
+  const int K = n <= 256 ? std::min(d.num_ops, 512 / (int)n) : 1;
+  const int kmax = std::min(d.num_ops, nstr + (d.num_diag > 1));  // strings of a sample with a matrix element
+  // (every workgroup sums the diagonal strings and looks at its share of all)
+  const double t_rows = 8.0 + (d.num_diag > 1 ? 2.2 * d.num_diag : 0.0) + 0.5 * ((d.num_ops + K - 1) / K) +
+                        (kmax + K - 1) / K * sym_resident_us(g, o.G, (double)n * K);
+  const double N = (double)n * d.num_ops;
+  const double t_mat = 28.0 + 2.5 * std::max(0, d.num_ops - 4) +
+                       std::min(sym_materialised_us(g, o.G, N), sym_resident_us(g, o.G, N));
+  const bool rows = t_rows < 0.9 * t_res;
+  if (t_mat < 0.9 * std::min(t_res, t_rows)) return JV_OK;
+  RbmTab tab = {};
+  int rc = rows ? JV_OK : build_rbm_tables(g, params, &d, false, true, st, slot0, &tab, o.map, o.G);
   if (rc) return rc;
   const auto rf = g.cpx ? (four ? sym_rows_eloc<true, 4> : sym_rows_eloc<true, 1>)
                         : (four ? sym_rows_eloc<false, 4> : sym_rows_eloc<false, 1>);
   if ((rc = set_lds_limit((const void*)rf, rlds))) return rc;
-  const int K = n <= 256 ? std::min(d.num_ops, 512 / (int)n) : 1;
   double* part = K > 1 ? (double*)capturable_workspace(16 * (size_t)K * n, slot1, st) : out;
   if (!part) return fail(JV_E_NOMEM, "jv_sym_eloc: workspace allocation failed");
   hipLaunchKernelGGL(rf, dim3((unsigned)std::min<int64_t>(n, 512 * SYM_T / T), (unsigned)K), dim3((unsigned)T), rlds, st, g, o,
                      params, d, tab, SL, configs, lps, n, part);
   JV_LAUNCH_CHECK("sym_rows_eloc");
+  if (rows) {
+    if (K > 1) {
+      hipLaunchKernelGGL(sym_add_parts, dim3((unsigned)((2 * n + SYM_T - 1) / SYM_T)), dim3(SYM_T), 0, st, part, K, n, out);
+      JV_LAUNCH_CHECK("sym_add_parts");
+    }
+    *done = true;
+    return JV_OK;
+  }
+#define JV_SYM_ELO(RCv)                                                                           \
+  (g.cpx ? (tabl ? sym_rbm_eloc<true, RCv, true> : sym_rbm_eloc<true, RCv, false>)                \
+         : (tabl ? sym_rbm_eloc<false, RCv, true> : sym_rbm_eloc<false, RCv, false>))
+  const auto fn = RC == 64 ? JV_SYM_ELO(64) : RC == 32 ? JV_SYM_ELO(32) : JV_SYM_ELO(16);
+#undef JV_SYM_ELO
+  if ((rc = set_lds_limit((const void*)fn, lds))) return rc;
   hipLaunchKernelGGL(fn, dim3((unsigned)std::min<int64_t>(n, 4096)), dim3(SYM_T), lds, st, g, o, params, d, tab, configs,
                      lps, n, nstr, part, K, out);
   JV_LAUNCH_CHECK("sym_rbm_eloc");
