@@ -231,7 +231,8 @@ int jv_sym_gradients(const jv_net* net, const double* params, const jv_orbit* or
  * one workgroup, a ratio per row and string (few strings: a log psi each);
  * else, and for few samples of large orbits, s' materialised per sample chunk
  * (jv_get_s_primes) and log psi(s') from jv_sym_forward.  A graph capture
- * needs a call of the same size before it.  Replaces Operator.get_O_loc (base.py:162-192) for a SymNet. */
+ * needs a call of the same size before it.
+ * Replaces Operator.get_O_loc (base.py:162-192) for a SymNet. */
 int jv_sym_eloc(const jv_net* net, const double* params, const jv_orbit* orbit,
                 const jv_optable* op, const double* prefactor, const int32_t* configs,
                 const double* logpsi_s, int64_t n, double* out, void* stream);

@@ -525,10 +525,11 @@ def test_sym_chains_mu(cpx, L, H, mu):
     assert np.array_equal(to_np(ms.states), mo.states)
 
 
-def test_sym_streams():
+@pytest.mark.parametrize("L,H,n", [(10, 12, 2000), (12, 70, 40)])
+def test_sym_streams(L, H, n):
     """Symmetrised calls on two streams of one thread, each with its own
-    parameters and enough samples to overlap, keep their tables apart."""
-    L, H, n = 10, 12, 2000
+    parameters, keep their scratch memory apart: enough samples to overlap, and
+    few enough for the materialised rows."""
     rng = np.random.default_rng(15)
     Hd, _ = tfim_pair((L,), -1.0, -0.7)
     Hd.compile()
@@ -544,7 +545,7 @@ def test_sym_streams():
     streams = [torch.cuda.Stream() for _ in range(2)]
     torch.cuda.synchronize()
     out = [[], []]
-    for _ in range(4):
+    for _ in range(8):
         for k, st in enumerate(streams):
             with torch.cuda.stream(st):
                 out[k].append(calls(psis[k]))

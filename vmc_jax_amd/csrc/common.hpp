@@ -33,6 +33,17 @@ void* stream_workspace(size_t bytes, int slot0, hipStream_t st);
 // The same for calls that may be captured (one more slot behind those).
 void* capturable_workspace(size_t bytes, int slot0, hipStream_t st);
 bool stream_capturing(hipStream_t st);
+// First slot of the k-th such buffer (behind the two of stream_workspace, 130 on).
+constexpr int ws_capturable(int k) { return 130 + 2 * WS_STREAMS + k * (WS_STREAMS + 1); }
+// Small scratch per stream, so that calls on several streams may overlap; large
+// scratch once per thread (a large call reserves the captured small ones' buffer
+// too: a capture may follow any call that was at least as large).
+inline void* scratch_workspace(size_t bytes, int slot, int k, hipStream_t st) {
+  constexpr size_t small = (size_t)16 << 20;
+  if (bytes <= small) return capturable_workspace(bytes, ws_capturable(k), st);
+  if (!stream_capturing(st) && !workspace(small, ws_capturable(k) + WS_STREAMS)) return nullptr;
+  return workspace(bytes, slot);
+}
 
 // Optional event timing of named kernels (jv_timer_enable / jv_timer_read).
 void* timer_begin(const char* name, hipStream_t st);

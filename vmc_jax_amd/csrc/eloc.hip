@@ -603,7 +603,7 @@ int jv_get_s_primes(const jv_optable* op, const double* prefactor, const int32_t
   if (n == 0) return JV_OK;
   hipStream_t st = (hipStream_t)stream;
   OpDev d = make_opdev(op, prefactor, num_sites);
-  int32_t* slot = (int32_t*)workspace(sizeof(int32_t) * (size_t)n * op->num_ops, 0);
+  int32_t* slot = (int32_t*)scratch_workspace(sizeof(int32_t) * (size_t)n * op->num_ops, 0, 11, st);
   if (!slot) return fail(JV_E_NOMEM, "jv_get_s_primes: workspace allocation failed");
   hipLaunchKernelGGL(sprime_compact, dim3((unsigned)((n + 127) / 128)), dim3(128), 0, st, d, configs, n,
                      num_sites, matel, slot, count);

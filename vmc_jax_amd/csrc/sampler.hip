@@ -46,7 +46,8 @@ __global__ void __launch_bounds__(256, 1) mc_rbmq(RbmGeom g, const double* __res
   const int w = __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE);
   const int chain = blockIdx.x * nw + w;
   if (chain >= a.num_chains) return;
-  const int64_t nacc = rbmq_mc<CPX, NH>(g, P, a, tab, walkers, configs, chain, lane, lds + (size_t)w * mc_rbm_lds_doubles(g));
+  const int64_t nacc =
+      rbmq_mc<CPX, NH>(g, P, a, tab, walkers, configs, chain, lane, lds + (size_t)w * mc_rbm_lds_doubles(g));
   if (lane == 0) {
     const int total = a.therm_steps + a.samples_per_chain * a.sweep_steps;
     atomicAdd((unsigned long long*)&counters[0], (unsigned long long)total);

@@ -29,9 +29,9 @@ int sym_rbm_mc_launch(const jv_net* net, const double* params, const jv_orbit* o
 
 namespace {
 // first slots of the resident forms' tables and partial sums in stream_workspace
-// (and one more slot each, capturable_workspace), behind WS_RBMQ_*
-constexpr int WS_SYM_ELOC_TAB = 130 + 2 * WS_STREAMS, WS_SYM_MC_TAB = WS_SYM_ELOC_TAB + WS_STREAMS + 1,
-              WS_SYM_ELOC_PART = WS_SYM_MC_TAB + WS_STREAMS + 1;
+// (ws_capturable; 3 .. 10: small calls' rows, s' and their log psi, 11:
+// jv_get_s_primes', 12 .. 16: chains)
+constexpr int WS_SYM_ELOC_TAB = ws_capturable(0), WS_SYM_MC_TAB = ws_capturable(1), WS_SYM_ELOC_PART = ws_capturable(2);
 // workspace slots of this file.  jv_sym_eloc may run on a side stream while
 // jv_sym_gradients runs on the main stream, so the forward pass inside
 // jv_sym_eloc has rows / log-psi slots of its own (WS_EROWS, WS_ELP).
@@ -318,8 +318,9 @@ int sym_forward(const jv_net* net, const double* params, const jv_orbit* orbit, 
   if (rc || done) return rc;
   const int L = net->num_sites, G = orbit->num_elements;
   const int64_t cs = std::min<int64_t>(n, rows_per_chunk(net, orbit, 0));
-  int32_t* rows = (int32_t*)workspace(sizeof(int32_t) * (size_t)cs * G * L, ws_rows);
-  double* lp = (double*)workspace(sizeof(double) * 2 * (size_t)cs * G, ws_lp);
+  const int k = ws_rows == WS_EROWS ? 5 : 3;
+  int32_t* rows = (int32_t*)scratch_workspace(sizeof(int32_t) * (size_t)cs * G * L, ws_rows, k, st);
+  double* lp = (double*)scratch_workspace(sizeof(double) * 2 * (size_t)cs * G, ws_lp, k + 1, st);
   if (!rows || !lp) return fail(JV_E_NOMEM, "jv_sym_forward: workspace allocation failed");
   const int cpx = sym_cpx(net, orbit);
   for (int64_t s0 = 0; s0 < n; s0 += cs) {
@@ -406,10 +407,10 @@ int jv_sym_eloc(const jv_net* net, const double* params, const jv_orbit* orbit, 
   const int L = net->num_sites, nops = op->num_ops;
   // s' of cs samples are cs * nops configurations, each expanded |orbit| times by jv_sym_forward
   const int64_t cs = std::max<int64_t>(1, std::min<int64_t>(n, rows_per_chunk(net, orbit, 0) * 4 / nops));
-  int32_t* sp = (int32_t*)workspace(sizeof(int32_t) * (size_t)cs * nops * L, WS_SP);
-  double* me = (double*)workspace(sizeof(double) * 2 * (size_t)cs * nops, WS_ME);
-  int32_t* cnt = (int32_t*)workspace(sizeof(int32_t) * (size_t)cs, WS_CNT);
-  double* lpsp = (double*)workspace(sizeof(double) * 2 * (size_t)cs * nops, WS_LPSP);
+  int32_t* sp = (int32_t*)scratch_workspace(sizeof(int32_t) * (size_t)cs * nops * L, WS_SP, 7, st);
+  double* me = (double*)scratch_workspace(sizeof(double) * 2 * (size_t)cs * nops, WS_ME, 8, st);
+  int32_t* cnt = (int32_t*)scratch_workspace(sizeof(int32_t) * (size_t)cs, WS_CNT, 9, st);
+  double* lpsp = (double*)scratch_workspace(sizeof(double) * 2 * (size_t)cs * nops, WS_LPSP, 10, st);
   if (!sp || !me || !cnt || !lpsp) return fail(JV_E_NOMEM, "jv_sym_eloc: workspace allocation failed");
   for (int64_t s0 = 0; s0 < n; s0 += cs) {
     const int64_t ns = std::min(cs, n - s0);
@@ -442,11 +443,11 @@ int jv_sym_mc_sample(const jv_net* net, const double* params, const jv_orbit* or
   rc = sym_rbm_mc_launch(net, params, orbit, a, walkers, configs, counters, st, WS_SYM_MC_TAB, &done);
   if (rc) return rc;
   if (done) return logpsi && ns > 0 ? jv_sym_forward(net, params, orbit, configs, ns, logpsi, stream) : JV_OK;
-  double* lacc = (double*)workspace(sizeof(double) * (size_t)C, WS_MC_LP);
-  int32_t* prop = (int32_t*)workspace(sizeof(int32_t) * (size_t)C * L, WS_MC_PROP);
-  double* u = (double*)workspace(sizeof(double) * (size_t)C, WS_MC_U);
-  int64_t* nacc = (int64_t*)workspace(sizeof(int64_t) * (size_t)C, WS_MC_NACC);
-  double* lpp = (double*)workspace(sizeof(double) * 2 * (size_t)C, WS_MC_LPP);
+  double* lacc = (double*)scratch_workspace(sizeof(double) * (size_t)C, WS_MC_LP, 12, st);
+  int32_t* prop = (int32_t*)scratch_workspace(sizeof(int32_t) * (size_t)C * L, WS_MC_PROP, 13, st);
+  double* u = (double*)scratch_workspace(sizeof(double) * (size_t)C, WS_MC_U, 14, st);
+  int64_t* nacc = (int64_t*)scratch_workspace(sizeof(int64_t) * (size_t)C, WS_MC_NACC, 15, st);
+  double* lpp = (double*)scratch_workspace(sizeof(double) * 2 * (size_t)C, WS_MC_LPP, 16, st);
   if (!lacc || !prop || !u || !nacc || !lpp) return fail(JV_E_NOMEM, "jv_sym_mc_sample: workspace allocation failed");
   if ((rc = jv_sym_forward(net, params, orbit, walkers, C, lpp, stream))) return rc;
   hipLaunchKernelGGL(sym_mc_init, dim3((unsigned)((C + 255) / 256)), dim3(256), 0, st, lpp, C, a.mu, lacc, nacc);

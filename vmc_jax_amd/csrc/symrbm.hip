@@ -496,9 +496,9 @@ __device__ inline void scale_row(cd& wt, int& ex) {
 // per CU, 6 % more); 386 vector instructions per wave and proposal, 38 % of the
 // issue cycles, bank conflicts of the table reads 37 % of the time.
 template <bool CPX, int HT, int MAXT, bool TAB>
-__global__ void __launch_bounds__(MAXT, MAXT == 256 ? 3 : MAXT == 512 ? 2 : 4) sym_rbm_mc(RbmGeom g, SymGeom o, const double* __restrict__ P, jv_mc_args a,
-                                                   RbmTab tab, int SL, int32_t* __restrict__ walkers,
-                                                   int32_t* __restrict__ configs, int64_t* __restrict__ counters) {
+__global__ void __launch_bounds__(MAXT, MAXT == 256 ? 3 : MAXT == 512 ? 2 : 4)
+    sym_rbm_mc(RbmGeom g, SymGeom o, const double* __restrict__ P, jv_mc_args a, RbmTab tab, int SL,
+               int32_t* __restrict__ walkers, int32_t* __restrict__ configs, int64_t* __restrict__ counters) {
   typedef typename num_of<CPX>::type T;
   extern __shared__ double lds[];
   const int L = g.L, H = g.H, G = o.G, tid = threadIdx.x, nt = blockDim.x, lane = tid % WAVE, nw = nt / WAVE;
@@ -865,8 +865,8 @@ int sym_rbm_eloc_launch(const jv_net* net, const double* params, const jv_orbit*
   if ((rc = set_lds_limit((const void*)rf, rlds))) return rc;
   double* part = K > 1 ? (double*)capturable_workspace(16 * (size_t)K * n, slot1, st) : out;
   if (!part) return fail(JV_E_NOMEM, "jv_sym_eloc: workspace allocation failed");
-  hipLaunchKernelGGL(rf, dim3((unsigned)std::min<int64_t>(n, 512 * SYM_T / T), (unsigned)K), dim3((unsigned)T), rlds, st, g, o,
-                     params, d, tab, SL, configs, lps, n, part);
+  hipLaunchKernelGGL(rf, dim3((unsigned)std::min<int64_t>(n, 512 * SYM_T / T), (unsigned)K), dim3((unsigned)T), rlds, st,
+                     g, o, params, d, tab, SL, configs, lps, n, part);
   JV_LAUNCH_CHECK("sym_rows_eloc");
   if (rows) {
     if (K > 1) {
